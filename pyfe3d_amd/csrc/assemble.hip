@@ -302,9 +302,9 @@ __device__ __forceinline__ void quad4_kc0(double K[6][6], const Geom &g, const S
     add_shear(K, s.Es, n.Ni, n.nxi, n.nyi, n.Nj, n.nxj, n.nyj, 4. * n.det, !thick, true, true);
 }
 
-// Quad4R KC0: quad4r.pyx:1300-1312 (E1eq, E2eq), 3081-3462
-__device__ __forceinline__ void quad4r_kc0(double K[6][6], const Geom &g, const Shell &s, int I,
-                                           int J, double k6rot, const double *hgf)
+// Quad4R hourglass moduli of DOFs 0..4: quad4r.pyx:1300-1312 (E1eq, E2eq)
+__device__ __forceinline__ void hourglass_moduli(const Geom &g, const Shell &s, const double *hgf,
+                                                 double Ehg[5])
 {
     const double A11 = s.C[0][0], A12 = s.C[0][1], A16 = s.C[0][2];
     const double A22 = s.C[1][1], A26 = s.C[1][2], A66 = s.C[2][2];
@@ -313,12 +313,32 @@ __device__ __forceinline__ void quad4r_kc0(double K[6][6], const Geom &g, const 
     const double a11 = (A22 * A66 - A26 * A26) / det3, a22 = (A11 * A66 - A16 * A16) / det3;
     const double E1eq = 1. / (s.h * a11), E2eq = 1. / (s.h * a22);
     const double damp = 1.0 + 1.0 / g.area, h3 = s.h * s.h * s.h;
-    double Ehg[5];
     Ehg[0] = hgf[0] * 0.1 * E1eq * s.h / damp;
     Ehg[1] = hgf[1] * 0.1 * E2eq * s.h / damp;
     Ehg[3] = hgf[3] * 0.1 * E2eq * h3 / damp;
     Ehg[4] = hgf[4] * 0.1 * E1eq * h3 / damp;
     Ehg[2] = hgf[2] * 0.5 * (Ehg[3] + Ehg[4]);
+}
+
+// hourglass mode amplitude d2N/dxdy at the centroid (+ on nodes 1 and 3, -
+// on 2 and 4)
+__device__ __forceinline__ double hourglass_gxy(const double *xe)
+{
+    const double J11 = 0.25 * (-xe[0] + xe[2] + xe[4] - xe[6]);
+    const double J12 = 0.25 * (-xe[1] + xe[3] + xe[5] - xe[7]);
+    const double J21 = 0.25 * (-xe[0] - xe[2] + xe[4] + xe[6]);
+    const double J22 = 0.25 * (-xe[1] - xe[3] + xe[5] + xe[7]);
+    const double dj = J11 * J22 - J12 * J21;
+    const double j11 = J22 / dj, j12 = -J12 / dj, j21 = -J21 / dj, j22 = J11 / dj;
+    return 0.25 * (j11 * j22 + j12 * j21);
+}
+
+// Quad4R KC0: quad4r.pyx:3081-3462
+__device__ __forceinline__ void quad4r_kc0(double K[6][6], const Geom &g, const Shell &s, int I,
+                                           int J, double k6rot, const double *hgf)
+{
+    double Ehg[5];
+    hourglass_moduli(g, s, hgf, Ehg);
 
     const double sxi = node_sx(I), syi = node_sy(I), sxj = node_sx(J), syj = node_sy(J);
     const Pair n = quad_pair(g.xe, 0., 0., sxi, syi, sxj, syj);
@@ -326,18 +346,11 @@ __device__ __forceinline__ void quad4r_kc0(double K[6][6], const Geom &g, const 
     add_abd(K, s.C, n.nxi, n.nyi, n.nxj, n.nyj, w);
     add_shear(K, s.Es, n.Ni, n.nxi, n.nyi, n.Nj, n.nxj, n.nyj, w, true, true, true);
     // hourglass modes gamma_I = d2N_I/dxdy at the centroid
-    const double *xe = g.xe;
-    const double J11 = 0.25 * (-xe[0] + xe[2] + xe[4] - xe[6]);
-    const double J12 = 0.25 * (-xe[1] + xe[3] + xe[5] - xe[7]);
-    const double J21 = 0.25 * (-xe[0] - xe[2] + xe[4] + xe[6]);
-    const double J22 = 0.25 * (-xe[1] - xe[3] + xe[5] + xe[7]);
-    const double dj = J11 * J22 - J12 * J21;
-    const double j11 = J22 / dj, j12 = -J12 / dj, j21 = -J21 / dj, j22 = J11 / dj;
-    const double gxy = 0.25 * (j11 * j22 + j12 * j21);
+    const double gxy = hourglass_gxy(g.xe);
     const double gI = (I & 1) ? -gxy : gxy, gJ = (J & 1) ? -gxy : gxy;
 #pragma unroll
     for (int d = 0; d < 5; d++) K[d][d] += w * Ehg[d] * gI * gJ;
-    const double kd = 1e-6 * k6rot * A66;
+    const double kd = 1e-6 * k6rot * s.C[2][2];
 #pragma unroll
     for (int p = 0; p < 4; p++) {
         const Pair m = quad_pair(g.xe, (p >> 1) ? GP2 : -GP2, (p & 1) ? GP2 : -GP2, sxi, syi,
@@ -355,15 +368,8 @@ __device__ __forceinline__ void tria_grad(const Geom &g, double Nx[3], double Ny
     Ny[0] = (p[4] - p[2]) / a2; Ny[1] = (p[0] - p[4]) / a2; Ny[2] = (p[2] - p[0]) / a2;
 }
 
-// Tria3R KC0: tria3r.pyx:1105-1122 (shear factor), 2116-2324 (terms).
-// Only the rz_I-rz_I drilling diagonal reaches the global matrix: the other
-// rz couplings computed at :2230-2324 are not used by the scatter at :2325-2974.
-// full_drill keeps every drilling coupling: the internal forces use them
-// (tria3r.pyx:549-948) although the KC0 scatter drops all rz couplings but
-// the rz_I-rz_I diagonal.
-__device__ __forceinline__ void tria3r_kc0(double K[6][6], const Geom &g, const Shell &s, int I,
-                                           int J, double k6rot, double alpha,
-                                           bool full_drill = false)
+// shear factor: tria3r.pyx:1105-1122
+__device__ __forceinline__ double tria_shear_factor(const Geom &g, const Shell &s, double alpha)
 {
     const double *p = g.xe;
     const double l12 = sqrt((p[0] - p[2]) * (p[0] - p[2]) + (p[1] - p[3]) * (p[1] - p[3]));
@@ -372,7 +378,17 @@ __device__ __forceinline__ void tria3r_kc0(double K[6][6], const Geom &g, const 
     double maxl = l12;
     if (l23 > maxl) maxl = l23;
     if (l31 > maxl) maxl = l31;
-    const double f = 1 / (1 + alpha * maxl * maxl / (s.h * s.h));
+    return 1 / (1 + alpha * maxl * maxl / (s.h * s.h));
+}
+
+// Tria3R KC0: tria3r.pyx:2116-2324.
+// Only the rz_I-rz_I drilling diagonal reaches the global matrix: the other
+// rz couplings computed at :2230-2324 are not used by the scatter at :2325-2974.
+// (The internal forces use every drilling coupling, see tria3r_fe.)
+__device__ __forceinline__ void tria3r_kc0(double K[6][6], const Geom &g, const Shell &s, int I,
+                                           int J, double k6rot, double alpha)
+{
+    const double f = tria_shear_factor(g, s, alpha);
     double E[2][2] = {{s.Es[0][0] * f, s.Es[0][1] * f}, {s.Es[1][0] * f, s.Es[1][1] * f}};
     double Nx[3], Ny[3];
     tria_grad(g, Nx, Ny);
@@ -385,7 +401,7 @@ __device__ __forceinline__ void tria3r_kc0(double K[6][6], const Geom &g, const 
 #pragma unroll
     for (int t = 0; t < 3; t++)
         add_drill(K, pick(P[t], I), nxi, nyi, pick(P[t], J), nxj, nyj, detJ * (0.5 / 3.) * kd,
-                  full_drill, I == J);
+                  false, I == J);
 }
 
 // membrane stress resultants from local displacements (quad4.pyx:1965-1967)
@@ -866,25 +882,191 @@ shell_kc0_sym(AsmArgs a)
 // Element internal forces in global axes, fe[e][6nn] = R6 K_e ue with
 // ue = blockdiag(R^T) u (update_probe_ue -> update_probe_finte -> rotation
 // in update_fint: quad4.pyx:627-680, 1174-1202, 1316-1363; quad4r.pyx:549,
-// 4620; tria3r.pyx:549, 2975).  Same lane mapping as shell_kc0_sym: the lane
-// owning block (I, J), I <= J, adds K_IJ ue_J to node I and K_IJ^T ue_I to
-// node J; the node sums are formed in a fixed lane order.
+// 4620; tria3r.pyx:549, 2975).
+//
+// One lane per element: K_e is never formed.  Each integration point takes
+// the strains B ue, the section forces C B ue and adds B^T of them to the
+// element's forces in registers, about 1,100 FMAs per quad.  (Forming the
+// ten node-pair blocks of K_e on ten lanes that each repeat the geometry
+// was bound by FP64 issue: 484 us for 1e6 quads against 109 us, now bound
+// by the gathers of x and u and the 192 MB of forces.)  230-250 VGPRs, two
+// waves per SIMD.  The forces leave through LDS so that the wave writes its
+// 64 elements' contiguous run with consecutive lanes.
 // ------------------------------------------------------------------------
+
+// forces of one integration point: membrane/bending strains -> C -> B^T
+// (rows as in add_abd), weight w
+template <int NN>
+__device__ __forceinline__ void fe_abd(double (&f)[6 * NN], const double (&ue)[6 * NN],
+                                       const double C[6][6], const double *Nx, const double *Ny,
+                                       double w)
+{
+    double e[6] = {0., 0., 0., 0., 0., 0.};
+#pragma unroll
+    for (int i = 0; i < NN; i++) {
+        const double *u = ue + 6 * i;
+        e[0] += Nx[i] * u[0];
+        e[1] += Ny[i] * u[1];
+        e[2] += Ny[i] * u[0] + Nx[i] * u[1];
+        e[3] += Nx[i] * u[4];
+        e[4] -= Ny[i] * u[3];
+        e[5] += Ny[i] * u[4] - Nx[i] * u[3];
+    }
+    double s[6];
+#pragma unroll
+    for (int a = 0; a < 6; a++) {
+        double t = 0.;
+#pragma unroll
+        for (int b = 0; b < 6; b++) t += C[a][b] * e[b];
+        s[a] = w * t;
+    }
+#pragma unroll
+    for (int i = 0; i < NN; i++) {
+        f[6 * i + 0] += Nx[i] * s[0] + Ny[i] * s[2];
+        f[6 * i + 1] += Ny[i] * s[1] + Nx[i] * s[2];
+        f[6 * i + 3] -= Ny[i] * s[4] + Nx[i] * s[5];
+        f[6 * i + 4] += Nx[i] * s[3] + Ny[i] * s[5];
+    }
+}
+
+// transverse shear at one point (N: one value per node); with thick the
+// gradient-gradient part (integrated at other points) is left out of row w
+template <int NN>
+__device__ __forceinline__ void fe_shear(double (&f)[6 * NN], const double (&ue)[6 * NN],
+                                         const double E[2][2], double N, const double *Nx,
+                                         const double *Ny, double w, bool thick)
+{
+    double gw[2] = {0., 0.}, gr[2] = {0., 0.};
+#pragma unroll
+    for (int i = 0; i < NN; i++) {
+        const double *u = ue + 6 * i;
+        gw[0] += Ny[i] * u[2];
+        gw[1] += Nx[i] * u[2];
+        gr[0] -= N * u[3];
+        gr[1] += N * u[4];
+    }
+    const double k0 = thick ? 0. : gw[0], k1 = thick ? 0. : gw[1];
+    const double q0 = w * (E[0][0] * (gw[0] + gr[0]) + E[0][1] * (gw[1] + gr[1]));
+    const double q1 = w * (E[1][0] * (gw[0] + gr[0]) + E[1][1] * (gw[1] + gr[1]));
+    const double p0 = w * (E[0][0] * (k0 + gr[0]) + E[0][1] * (k1 + gr[1]));
+    const double p1 = w * (E[1][0] * (k0 + gr[0]) + E[1][1] * (k1 + gr[1]));
+#pragma unroll
+    for (int i = 0; i < NN; i++) {
+        f[6 * i + 2] += Ny[i] * p0 + Nx[i] * p1;
+        f[6 * i + 3] -= N * q0;
+        f[6 * i + 4] += N * q1;
+    }
+}
+
+// drilling rz - (v,x - u,y)/2 at one point, weight w
+template <int NN>
+__device__ __forceinline__ void fe_drill(double (&f)[6 * NN], const double (&ue)[6 * NN],
+                                         const double *N, const double *Nx, const double *Ny,
+                                         double w)
+{
+    double d = 0.;
+#pragma unroll
+    for (int i = 0; i < NN; i++)
+        d += N[i] * ue[6 * i + 5] + 0.5 * (Ny[i] * ue[6 * i] - Nx[i] * ue[6 * i + 1]);
+    d *= w;
+#pragma unroll
+    for (int i = 0; i < NN; i++) {
+        f[6 * i + 0] += 0.5 * Ny[i] * d;
+        f[6 * i + 1] -= 0.5 * Nx[i] * d;
+        f[6 * i + 5] += N[i] * d;
+    }
+}
+
+// Quad4 (quad4.pyx:755-1172): ABD, drilling and the thick shells' shear
+// gradients at 2x2 points, shear at the centroid
+__device__ __forceinline__ void quad4_fe(double (&f)[24], const double (&ue)[24], const Geom &g,
+                                         const Shell &s)
+{
+    const bool thick = (s.h / sqrt(g.area)) >= 1.;
+#pragma unroll 1
+    for (int p = 0; p < 4; p++) {
+        QShape q;
+        quad_shape(g.xe, (p >> 1) ? GP2 : -GP2, (p & 1) ? GP2 : -GP2, q);
+        fe_abd<4>(f, ue, s.C, q.Nx, q.Ny, q.det);
+        fe_drill<4>(f, ue, q.N, q.Nx, q.Ny, q.det);
+        if (thick) {
+            double gw[2] = {0., 0.};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                gw[0] += q.Ny[i] * ue[6 * i + 2];
+                gw[1] += q.Nx[i] * ue[6 * i + 2];
+            }
+            const double p0 = q.det * (s.Es[0][0] * gw[0] + s.Es[0][1] * gw[1]);
+            const double p1 = q.det * (s.Es[1][0] * gw[0] + s.Es[1][1] * gw[1]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) f[6 * i + 2] += q.Ny[i] * p0 + q.Nx[i] * p1;
+        }
+    }
+    QShape q;
+    quad_shape(g.xe, 0., 0., q);
+    fe_shear<4>(f, ue, s.Es, 0.25, q.Nx, q.Ny, 4. * q.det, thick);
+}
+
+// Quad4R (quad4r.pyx:1300-1312, 3081-3462): ABD, shear and hourglass at the
+// centroid, drilling at 2x2 points
+__device__ __forceinline__ void quad4r_fe(double (&f)[24], const double (&ue)[24], const Geom &g,
+                                          const Shell &s, double k6rot, const double *hgf)
+{
+    double Ehg[5];
+    hourglass_moduli(g, s, hgf, Ehg);
+    QShape q;
+    quad_shape(g.xe, 0., 0., q);
+    const double w = 4. * q.det;
+    fe_abd<4>(f, ue, s.C, q.Nx, q.Ny, w);
+    fe_shear<4>(f, ue, s.Es, 0.25, q.Nx, q.Ny, w, false);
+    const double gxy = hourglass_gxy(g.xe);
+#pragma unroll
+    for (int d = 0; d < 5; d++) {
+        double t = 0.;
+#pragma unroll
+        for (int i = 0; i < 4; i++) t += ((i & 1) ? -gxy : gxy) * ue[6 * i + d];
+        t *= w * Ehg[d];
+#pragma unroll
+        for (int i = 0; i < 4; i++) f[6 * i + d] += ((i & 1) ? -gxy : gxy) * t;
+    }
+    const double kd = 1e-6 * k6rot * s.C[2][2];
+#pragma unroll 1
+    for (int p = 0; p < 4; p++) {
+        QShape m;
+        quad_shape(g.xe, (p >> 1) ? GP2 : -GP2, (p & 1) ? GP2 : -GP2, m);
+        fe_drill<4>(f, ue, m.N, m.Nx, m.Ny, m.det * kd);
+    }
+}
+
+// Tria3R (tria3r.pyx:549-948): every drilling coupling, unlike the KC0
+// scatter
+__device__ __forceinline__ void tria3r_fe(double (&f)[18], const double (&ue)[18], const Geom &g,
+                                          const Shell &s, double k6rot, double alpha)
+{
+    const double fs = tria_shear_factor(g, s, alpha);
+    const double E[2][2] = {{s.Es[0][0] * fs, s.Es[0][1] * fs}, {s.Es[1][0] * fs, s.Es[1][1] * fs}};
+    double Nx[3], Ny[3];
+    tria_grad(g, Nx, Ny);
+    const double detJ = 2 * g.area, w = 0.5 * detJ;
+    fe_abd<3>(f, ue, s.C, Nx, Ny, w);
+    fe_shear<3>(f, ue, E, 1. / 3., Nx, Ny, w, false);
+    const double kd = 1e-6 * k6rot * s.C[2][2];
+    const double P[3][3] = {{2. / 3, 1. / 6, 1. / 6}, {1. / 6, 1. / 6, 2. / 3}, {1. / 6, 2. / 3, 1. / 6}};
+#pragma unroll
+    for (int t = 0; t < 3; t++) fe_drill<3>(f, ue, P[t], Nx, Ny, detJ * (0.5 / 3.) * kd);
+}
+
 template <int ET>
 __global__ void __launch_bounds__(64) shell_fe(AsmArgs a, double *__restrict__ fe)
 {
     constexpr int NN = (ET == TRIA3R) ? 3 : 4;
-    constexpr int NUP = NN * (NN + 1) / 2;
-    constexpr int EPW = 64 / NUP;
-    __shared__ double part[EPW][NUP][2][6];
-    __shared__ double sr[EPW][9];
+    constexpr int ND = 6 * NN;
+    constexpr int LD = ND + 1;  // odd row length: consecutive lanes on different banks
+    __shared__ double out[64 * LD];
     const int lane = threadIdx.x;
-    const int slot = lane / NUP, sub = lane - slot * NUP;
-    int I, J;
-    upper_pair<NN>(sub, I, J);
-    const int64_t e = (int64_t)blockIdx.x * EPW + slot;
-    const bool active = slot < EPW && e < a.n_elem;
-    if (active) {
+    const int64_t e0 = (int64_t)blockIdx.x * 64;
+    const int64_t e = e0 + lane;
+    if (e < a.n_elem) {
         V3 X[NN];
         int64_t cn[NN];
 #pragma unroll
@@ -900,76 +1082,41 @@ __global__ void __launch_bounds__(64) shell_fe(AsmArgs a, double *__restrict__ f
         else quad_geometry(X, xm, g);
         Shell s;
         load_shell(a.props + (a.pid ? (int64_t)a.pid[e] : 0) * SHELL_STRIDE, g.m, s);
-        double K[6][6];
+        double ue[ND], f[ND];
 #pragma unroll
-        for (int i = 0; i < 6; i++)
+        for (int i = 0; i < NN; i++)
 #pragma unroll
-            for (int j = 0; j < 6; j++) K[i][j] = 0.;
+            for (int b = 0; b < 2; b++) {
+                const double *pu = a.u + cn[i] + 3 * b;
+                const double u0 = pu[0], u1 = pu[1], u2 = pu[2];
+#pragma unroll
+                for (int t = 0; t < 3; t++) {
+                    ue[6 * i + 3 * b + t] = g.r[t] * u0 + g.r[3 + t] * u1 + g.r[6 + t] * u2;
+                    f[6 * i + 3 * b + t] = 0.;
+                }
+            }
         const double k6 = a.k6rot ? a.k6rot[e] : 100.;
-        if (ET == QUAD4) quad4_kc0(K, g, s, I, J);
-        else if (ET == QUAD4R) {
+        if constexpr (ET == QUAD4) quad4_fe(f, ue, g, s);
+        else if constexpr (ET == QUAD4R) {
             double hgf[5] = {1., 1., 1., 1., 1.};
             if (a.hg)
 #pragma unroll
                 for (int d = 0; d < 5; d++) hgf[d] = a.hg[5 * e + d];
-            quad4r_kc0(K, g, s, I, J, k6, hgf);
+            quad4r_fe(f, ue, g, s, k6, hgf);
         } else {
-            tria3r_kc0(K, g, s, I, J, k6, a.alpha ? a.alpha[e] : 0.7, true);
+            tria3r_fe(f, ue, g, s, k6, a.alpha ? a.alpha[e] : 0.7);
         }
-        // local displacements of nodes I and J
-        int64_t ci = cn[0], cj = cn[0];
 #pragma unroll
-        for (int i = 1; i < NN; i++) {
-            ci = (I == i) ? cn[i] : ci;
-            cj = (J == i) ? cn[i] : cj;
-        }
-        double ui[6], uj[6];
+        for (int i = 0; i < 2 * NN; i++)
 #pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int t = 0; t < 3; t++) {
-                double si = 0., sj = 0.;
-#pragma unroll
-                for (int q = 0; q < 3; q++) {
-                    si += g.r[3 * q + t] * a.u[ci + 3 * b + q];
-                    sj += g.r[3 * q + t] * a.u[cj + 3 * b + q];
-                }
-                ui[3 * b + t] = si;
-                uj[3 * b + t] = sj;
-            }
-#pragma unroll
-        for (int i = 0; i < 6; i++) {
-            double fi = 0., fj = 0.;
-#pragma unroll
-            for (int j = 0; j < 6; j++) {
-                fi += K[i][j] * uj[j];
-                fj += K[j][i] * ui[j];
-            }
-            part[slot][sub][0][i] = fi;
-            part[slot][sub][1][i] = (I != J) ? fj : 0.;
-        }
-        if (sub == 0)
-#pragma unroll
-            for (int i = 0; i < 9; i++) sr[slot][i] = g.r[i];
+            for (int q = 0; q < 3; q++)
+                out[lane * LD + 3 * i + q] = g.r[3 * q] * f[3 * i] + g.r[3 * q + 1] * f[3 * i + 1] +
+                                             g.r[3 * q + 2] * f[3 * i + 2];
     }
     __syncthreads();
-    if (active && sub < NN) {
-        const int P = sub;
-        double f[6] = {0., 0., 0., 0., 0., 0.};
-        for (int t = 0; t < NUP; t++) {
-            int It, Jt;
-            upper_pair<NN>(t, It, Jt);
-            if (It == P)
-                for (int i = 0; i < 6; i++) f[i] += part[slot][t][0][i];
-            else if (Jt == P)
-                for (int i = 0; i < 6; i++) f[i] += part[slot][t][1][i];
-        }
-        double *o = fe + (e * NN + P) * 6;
-        for (int b = 0; b < 2; b++)
-            for (int q = 0; q < 3; q++)
-                o[3 * b + q] = sr[slot][3 * q] * f[3 * b] + sr[slot][3 * q + 1] * f[3 * b + 1] +
-                               sr[slot][3 * q + 2] * f[3 * b + 2];
-    }
+    const int total = (int)((a.n_elem - e0) < 64 ? (a.n_elem - e0) : 64) * ND;
+    double *o = fe + e0 * ND;
+    for (int t = lane; t < total; t += 64) o[t] = out[t + t / ND];
 }
 
 // Geometry of each element: r (9), m (4), area/length, local x/y (2*nn).
@@ -1841,8 +1988,7 @@ hipError_t pf3d_launch_rod_fe(int etype, const AsmArgs &a, double *fe, hipStream
 
 hipError_t pf3d_launch_shell_fe(int etype, const AsmArgs &a, double *fe, hipStream_t s)
 {
-    const int nup = etype == TRIA3R ? 6 : 10;
-    const int64_t blocks = (a.n_elem + 64 / nup - 1) / (64 / nup);
+    const int64_t blocks = (a.n_elem + 63) / 64;
     if (blocks == 0) return hipSuccess;
     switch (etype) {
     case QUAD4:

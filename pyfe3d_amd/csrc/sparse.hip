@@ -177,7 +177,19 @@ __global__ void gather_nodes(int64_t n_nodes, const int64_t *__restrict__ offset
     if (t >= 6 * n_nodes) return;
     const int64_t p = t / 6, d = t - 6 * p;
     double s = fint[t];
-    for (int64_t k = offsets[p]; k < offsets[p + 1]; k++) s += fe[ids[k] * 6 + d];
+    // four entries' id and force loads in flight at a time (an entry past
+    // the end re-reads the last one and is not added)
+    const int64_t k1 = offsets[p + 1];
+    for (int64_t k = offsets[p]; k < k1; k += 4) {
+        int64_t id[4];
+        double f[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) id[j] = ids[k + j < k1 ? k + j : k1 - 1];
+#pragma unroll
+        for (int j = 0; j < 4; j++) f[j] = fe[id[j] * 6 + d];
+#pragma unroll
+        for (int j = 0; j < 4; j++) s = k + j < k1 ? s + f[j] : s;
+    }
     fint[t] = s;
 }
 
