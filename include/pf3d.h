@@ -487,6 +487,12 @@ int pf3d_bsr_dirichlet(int64_t nb, const int32_t *row_ptr, const int32_t *col_id
 int pf3d_bsr_dirichlet_diag(int64_t nb, const int32_t *row_ptr, const int32_t *col_idx,
                             double *val, const uint8_t *fixed, double diag, void *stream);
 
+/* val = src with the conditions of pf3d_bsr_dirichlet and val32 its FP32
+ * copy, in one pass (src, val and val32 distinct). */
+int pf3d_bsr_system(int64_t nb, const int32_t *row_ptr, const int32_t *col_idx,
+                    const double *src, const uint8_t *fixed, double *val, float *val32,
+                    void *stream);
+
 /* b[i] = (float)a[i] */
 int pf3d_to_f32(int64_t n, const double *a, float *b, void *stream);
 

@@ -75,6 +75,7 @@ SIGNATURES = {
     'pf3d_amg_smooth_prolongator': [I64, P, P, P, P, P, P, F64, P, P, P],
     'pf3d_bsr_symmetrize': [I64, I64, P, P, P, P, P, P, P],
     'pf3d_bsr_dirichlet': [I64, P, P, P, P, P],
+    'pf3d_bsr_system': [I64, P, P, P, P, P, P, P],
     'pf3d_to_f32': [I64, P, P, P],
     'pf3d_bsr_dirichlet_diag': [I64, P, P, P, P, F64, P],
     'pf3d_gemv_t': [I64, I32, P, I64, P, P, F64, F64, P],

@@ -487,26 +487,36 @@ __global__ void blk_emit(int64_t n, int nn, int64_t n_nodes, const int64_t *__re
     if (t == n - 1) src_ptr[nnzb] = n;
 }
 
-// one thread per (BSR block, row m): 6 contiguous values per source
-__global__ void blk_apply(int64_t nnzb, const int64_t *__restrict__ src_ptr,
-                          const int64_t *__restrict__ src, int stride,
-                          const double *__restrict__ v, double *__restrict__ out, int accumulate)
+// one thread per pair of neighbouring entries of a BSR block (18 per
+// block): lanes write consecutive 16-byte pairs, and the loads of four
+// sources are in flight at a time (a source past the end re-reads the last
+// one and is not added).  Sums run over the sources in order.  864 MB (the
+// element blocks of 119,899 quads read, 1.08e6 blocks written): 164 us, 5.3
+// TB/s; one thread per block row, its sources one after another, took 188.
+using dbl2 = double __attribute__((ext_vector_type(2), aligned(8)));
+
+__global__ void __launch_bounds__(256)
+    blk_apply(int64_t nnzb, const int64_t *__restrict__ src_ptr, const int64_t *__restrict__ src,
+              int stride, const double *__restrict__ v, double *__restrict__ out, int accumulate)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nnzb * 6) return;
-    const int64_t b = t / 6;
-    const int m = (int)(t - b * 6);
-    double s[6];
-    double *o = out + b * 36 + m * 6;
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= nnzb * 18) return;
+    const int64_t b = t / 18;
+    const int pr = (int)(t - b * 18), m = pr / 3, n = 2 * (pr - 3 * m);
+    const double *p = v + (int64_t)stride * m + n;
+    dbl2 *o = reinterpret_cast<dbl2 *>(out + 2 * t);
+    dbl2 s = accumulate ? *o : dbl2{0., 0.};
+    const int64_t k1 = src_ptr[b + 1];
+    for (int64_t k = src_ptr[b]; k < k1; k += 4) {
+        dbl2 x[4];
 #pragma unroll
-    for (int n = 0; n < 6; n++) s[n] = accumulate ? o[n] : 0.;
-    for (int64_t k = src_ptr[b]; k < src_ptr[b + 1]; k++) {
-        const double *p = v + src[k] + (int64_t)stride * m;
+        for (int j = 0; j < 4; j++)
+            x[j] = *reinterpret_cast<const dbl2 *>(p + src[k + j < k1 ? k + j : k1 - 1]);
 #pragma unroll
-        for (int n = 0; n < 6; n++) s[n] += p[n];
+        for (int j = 0; j < 4; j++)
+            if (k + j < k1) s += x[j];
     }
-#pragma unroll
-    for (int n = 0; n < 6; n++) o[n] = s[n];
+    *o = s;
 }
 
 }  // namespace
@@ -603,7 +613,7 @@ int pf3d_block_apply(int64_t nnzb, const int64_t *src_ptr, const int64_t *src, i
 {
     if (nnzb <= 0 || !src_ptr || !src || nn < 2 || nn > 4 || !v || !bsr_val)
         return pf3d_fail(PF3D_E_ARG, "pf3d_block_apply: bad arguments");
-    hipLaunchKernelGGL(blk_apply, dim3(nblk(nnzb * 6, 256)), dim3(256), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(blk_apply, dim3(nblk(nnzb * 18, 256)), dim3(256), 0, (hipStream_t)stream,
                        nnzb, src_ptr, src, 6 * nn, v, bsr_val, accumulate);
     return pf3d_hip_check(hipGetLastError(), "pf3d_block_apply");
 }

@@ -32,18 +32,23 @@ class StaticSystem:
         if fixed.numel() != 6 * nb:
             raise ValueError('fixed must have one entry per DOF')
         self.fixed = fixed
-        self.val = val.clone()
         s = _s(stream)
-        _lib.call('pf3d_bsr_dirichlet', nb, plan.row_ptr.data_ptr(), plan.col_idx.data_ptr(),
-                  self.val.data_ptr(), fixed.data_ptr(), s)
+        src = val.contiguous()
+        if stream is not None:
+            src.record_stream(stream)
+        # (values past the plan's blocks are kept as they are)
+        whole = src.numel() == 36 * plan.col_idx.numel()
+        self.val = torch.empty_like(src) if whole else src.clone()
+        self.val32 = (torch.empty_like(src, dtype=torch.float32) if whole
+                      else src.to(torch.float32))
+        _lib.call('pf3d_bsr_system', nb, plan.row_ptr.data_ptr(), plan.col_idx.data_ptr(),
+                  src.data_ptr(), fixed.data_ptr(), self.val.data_ptr(), self.val32.data_ptr(), s)
         self.dinv = torch.empty(nb * 36, dtype=torch.float64, device=dev)
         self.dinv32 = torch.empty(nb * 36, dtype=torch.float32, device=dev)
         bad = torch.zeros(1, dtype=torch.int32, device=dev)
         _lib.call('pf3d_bjacobi', nb, plan.row_ptr.data_ptr(), plan.col_idx.data_ptr(),
                   self.val.data_ptr(), self.dinv.data_ptr(), self.dinv32.data_ptr(),
                   bad.data_ptr(), s)
-        self.val32 = torch.empty(self.val.numel(), dtype=torch.float32, device=dev)
-        _lib.call('pf3d_to_f32', self.val.numel(), self.val.data_ptr(), self.val32.data_ptr(), s)
         if int(bad.item()):
             raise _lib.Pf3dError('%d singular 6x6 diagonal blocks' % int(bad.item()))
         nbytes = ctypes.c_int64()
