@@ -584,6 +584,36 @@ int pf3d_batch_solve(int64_t n_var, int64_t nb, const int64_t *row0, const int32
 /* callers' scipy spsolve, tests/test_quad4_static_point_load.py:84-102) */
 /* ------------------------------------------------------------------ */
 
+/* Nested dissection: multifrontal Cholesky of the independent systems of a
+ * block-diagonal BSR matrix (after pf3d_bsr_dirichlet).
+ * pf3d_nd_create analyses the pattern on the host (no device call): host
+ * arrays row_ptr, col_idx; system s owns block rows [node0[s],
+ * node0[s + 1]), which must cover all n_nodes and reference only each
+ * other; coord NULL or the grid position (2 int32 per node) of structured
+ * plates; parts of at most `leaf` nodes are not divided further.  *plan is
+ * an opaque handle for the calls below, read-only after creation, released
+ * by pf3d_nd_free.
+ * pf3d_nd_sizes: sizes[0] bytes of the plan's device image, [1] doubles of
+ * the factor, [2] of the factorisation's scratch, [3] of the solve's
+ * scratch, [4] fronts, [5] rows of the largest front; *flops of one
+ * factorisation.  pf3d_nd_image writes the image to host memory; the caller
+ * keeps a copy of it on the device. */
+int pf3d_nd_create(int64_t n_nodes, const int32_t *row_ptr, const int32_t *col_idx,
+                   const int32_t *coord, int64_t n_sys, const int64_t *node0, int leaf,
+                   void **plan);
+int pf3d_nd_sizes(const void *plan, int64_t *sizes, double *flops);
+int pf3d_nd_image(const void *plan, void *image);
+int pf3d_nd_free(void *plan);
+
+/* Factorise (val: the BSR values; *bad, a device int, counts panels that met
+ * a non-positive pivot), then solve any number of right-hand sides (f, x: 6
+ * doubles per node in the original numbering).  Kernel launches only: no
+ * allocation, no synchronisation. */
+int pf3d_nd_factor(const void *plan, const void *image, const double *val, double *factor,
+                   double *update, int *bad, void *stream);
+int pf3d_nd_solve(const void *plan, const void *image, const double *factor, const double *f,
+                  double *x, double *work, void *stream);
+
 /* Largest bandwidth (scalars below the diagonal) the kernels accept. */
 int pf3d_band_max_width(void);
 

@@ -100,6 +100,12 @@ SIGNATURES = {
     'pf3d_band_chol': [I64, P, P, P, P, P, P, I32, I32, P, P, P, P],
     'pf3d_band_backsolve': [I64, P, P, P, P, P, P, P, P, I32, P],
     'pf3d_band_solve': [I64, P, P, P, P, P, P, P, P, P, I32, P],
+    'pf3d_nd_create': [I64, P, P, P, I64, P, I32, P],
+    'pf3d_nd_sizes': [P, P, P],
+    'pf3d_nd_image': [P, P],
+    'pf3d_nd_free': [P],
+    'pf3d_nd_factor': [P, P, P, P, P, P, P],
+    'pf3d_nd_solve': [P, P, P, P, P, P, P],
     'pf3d_nn_gemm': [I32, I32, I32, P, I64, I64, P, I64, I64, P, I64, I32, P, I32, I32, P, P],
     'pf3d_nn_im2col': [I32, I32, I32, I32, I32, P, P, P],
     'pf3d_nn_col2im': [I32, I32, I32, I32, I32, P, P, I32, P],

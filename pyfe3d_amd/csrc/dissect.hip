@@ -1,0 +1,616 @@
+// Direct solves by nested dissection: multifrontal Cholesky of many
+// independent SPD systems (the diagonal blocks of a block-diagonal 6x6 BSR
+// matrix), the counterpart of the reference callers' scipy spsolve
+// (tests/test_quad4_static_point_load.py:84-102).
+//
+// Against the banded factorisation (banded.hip: one workgroup walks a plate
+// 32 columns at a time, n b^2 operations in a chain of n / 32 panels) the
+// separators of a plate need 5-7 times fewer operations and leave a chain of
+// about 35 panels, and every front of a tree level, of every system, is
+// worked on at once by as many workgroups as it has row blocks and tiles.
+//
+// Per tree level (deepest first), all launches over all fronts of the level:
+//   * panel p: 32 own columns of each front.  A workgroup takes 128 rows
+//     below the panel's diagonal block: it forms that block (redundantly, so
+//     the launch needs no exchange between workgroups) and its rows, the
+//     original entries plus the children's update matrices minus the
+//     products with the panels before (FP64 MFMA, operands straight from the
+//     cached front), factorises the block in one wave while the others form
+//     rows, and solves its rows against it;
+//   * update: the front's boundary block, the children's contributions minus
+//     L21 L21^T, in 64 x 64 tiles; it is read by the parent only.
+// The triangular solves take one workgroup per front and level.
+//
+// Every sum has a fixed order: the same bits on every run.
+#include <hip/hip_runtime.h>
+#include <math.h>
+#include <string.h>
+
+#include "../../include/pf3d.h"
+#include "diag_block.hpp"
+#include "dissect.hpp"
+
+int pf3d_fail(int code, const char *fmt, ...);
+int pf3d_hip_check(hipError_t e, const char *where);
+
+namespace {
+
+using namespace nd;
+using band::diag_block;
+using band::readlane_d;
+using band::v4d;
+
+// largest front (DOFs): its right-hand side fits LDS in the solves, and
+// offsets inside it fit 32 bits
+constexpr int MAX_FRONT = 6144;
+
+// device image of a plan
+struct Image {
+    const Front *fronts;
+    const Task *tasks;
+    const int32_t *nodes, *cmap, *pnode, *ld;
+    const int64_t *dest;
+};
+
+size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
+
+struct Layout {
+    size_t fronts, tasks, nodes, cmap, pnode, ld, dest, total;
+    explicit Layout(const Plan &p)
+    {
+        size_t o = 0;
+        auto take = [&](size_t bytes) {
+            const size_t at = o;
+            o += align256(bytes);
+            return at;
+        };
+        fronts = take(p.fronts.size() * sizeof(Front));
+        tasks = take(p.tasks.size() * sizeof(Task));
+        nodes = take(p.nodes.size() * 4);
+        cmap = take(p.cmap.size() * 4);
+        pnode = take(p.pnode.size() * 4);
+        ld = take(p.ld.size() * 4);
+        dest = take(p.dest.size() * 8);
+        total = o;
+    }
+};
+
+Image image_at(const Plan &p, const void *base)
+{
+    const Layout l(p);
+    const char *b = (const char *)base;
+    return Image{(const Front *)(b + l.fronts), (const Task *)(b + l.tasks),
+                 (const int32_t *)(b + l.nodes), (const int32_t *)(b + l.cmap),
+                 (const int32_t *)(b + l.pnode), (const int32_t *)(b + l.ld),
+                 (const int64_t *)(b + l.dest)};
+}
+
+__global__ void nd_zero(int64_t n, double *__restrict__ p)
+{
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n;
+         t += (int64_t)gridDim.x * blockDim.x)
+        p[t] = 0.;
+}
+
+// original entries into the panels: one thread per entry of each BSR block
+// on or below the diagonal of the elimination order
+__global__ void nd_scatter(int64_t nnzb, const int64_t *__restrict__ dest,
+                           const int32_t *__restrict__ ld, const double *__restrict__ val,
+                           double *__restrict__ L)
+{
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t b = t / 36;
+    if (b >= nnzb) return;
+    const int64_t d = dest[b];
+    if (d < 0) return;
+    // consecutive lanes: consecutive rows of a column
+    const int e = (int)(t - b * 36), c = e / 6, r = e - 6 * c;
+    L[d + (int64_t)c * ld[b] + r] = val[b * 36 + 6 * r + c];
+}
+
+// the children's update matrices as seen by one front
+struct Kids {
+    const double *u[2];
+    int ld[2];
+    const int32_t *map;  // the front's list: 2 per node
+};
+
+__device__ __forceinline__ Kids kids_of(const Front *F, const Front &f, const int32_t *cmap,
+                                        const double *Uc)
+{
+    Kids k;
+    k.map = cmap + 2 * f.noff;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const int id = c ? f.c1 : f.c0;
+        k.u[c] = id < 0 ? nullptr : Uc + F[id].uoff;
+        k.ld[c] = id < 0 ? 0 : F[id].m;
+    }
+    return k;
+}
+
+// Tiles are computed transposed, as in the banded factorisation: lane l holds
+// row r[t] (its row l % 16 of tile t) of the columns c[s][v] (column l / 16 +
+// 4 v of block s), so that a load or store of a column covers 16 consecutive
+// rows.  Offsets inside a front fit 32 bits (MAX_FRONT).
+
+// acc += what the children add at (r, c).  Positions first, then every value
+// of a child in one round of loads (an entry it does not have reads its
+// first one and is not added).  Above the diagonal the values are arbitrary
+// and must not be used.
+template <int NT, int NS>
+__device__ __forceinline__ void add_kids(v4d (&acc)[NT][NS], const Kids &k, const int (&r)[NT],
+                                         const int (&c)[NS][4])
+{
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        if (!k.u[i]) continue;
+        int pr[NT], pc[NS][4];
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const int q = r[t] / 6, p = k.map[2 * q + i];
+            pr[t] = p < 0 ? -1 : 6 * p + r[t] - 6 * q;
+        }
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int q = c[s][v] / 6, p = k.map[2 * q + i];
+                pc[s][v] = p < 0 ? -1 : (6 * p + c[s][v] - 6 * q) * k.ld[i];
+            }
+        double x[NT][NS][4];
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    x[t][s][v] = k.u[i][(pr[t] | pc[s][v]) < 0 ? 0 : pr[t] + pc[s][v]];
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if ((pr[t] | pc[s][v]) >= 0) acc[t][s][v] += x[t][s][v];
+    }
+}
+
+// acc -= (rows r[t]) x (rows rc[s])^T over the first kk1 columns of the
+// front's panel; UN steps of four columns are loaded together, so that a
+// wave waits once for UN (NT + NS) loads.
+template <int NT, int NS, int UN>
+__device__ __forceinline__ void tile_products(v4d (&acc)[NT][NS], const double *Lf, int ld,
+                                              const int (&r)[NT], const int (&rc)[NS], int kk1,
+                                              int lk)
+{
+    auto step = [&](const double (&a)[NS], const double (&b)[NT]) {
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+                acc[t][s] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[t], acc[t][s], 0, 0, 0);
+    };
+    int kk = 0;
+    for (; kk + 4 * UN <= kk1; kk += 4 * UN) {
+        double a[UN][NS], b[UN][NT];
+#pragma unroll
+        for (int u = 0; u < UN; u++) {
+            const int o = (kk + 4 * u + lk) * ld;
+#pragma unroll
+            for (int s = 0; s < NS; s++) a[u][s] = -Lf[o + rc[s]];
+#pragma unroll
+            for (int t = 0; t < NT; t++) b[u][t] = Lf[o + r[t]];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < UN; u++) step(a[u], b[u]);
+    }
+    for (; kk < kk1; kk += 4) {  // (own blocks of 6 x odd nodes end inside a step)
+        const bool in = kk + lk < kk1;
+        const int o = (in ? kk + lk : 0) * ld;
+        double a[NS], b[NT];
+#pragma unroll
+        for (int s = 0; s < NS; s++) a[s] = in ? -Lf[o + rc[s]] : 0.;
+#pragma unroll
+        for (int t = 0; t < NT; t++) b[t] = in ? Lf[o + r[t]] : 0.;
+        step(a, b);
+    }
+}
+
+__global__ void __launch_bounds__(256, 3)
+    nd_panel(Image g, int64_t task0, int p, double *__restrict__ L, double *__restrict__ D,
+             const double *__restrict__ Uc, int *__restrict__ bad)
+{
+    __shared__ double P[RB][NF + 1];  // the workgroup's rows
+    __shared__ double Q[NF][NF + 1];  // the diagonal block
+    __shared__ double dinv[NF];
+    __shared__ double Lk[2][NF];
+    const Task task = g.tasks[task0 + blockIdx.x];
+    const Front f = g.fronts[task.front];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int li = lane & 15, lk = lane >> 4;
+    const int n = f.k + f.m, c0 = p * NF, jn = min(NF, f.k - c0);
+    const int r0 = c0 + jn + task.part * RB, nr = min(RB, n - r0);
+    double *Lf = L + f.loff;
+    const int ld = n, last = n - 1;
+    const Kids kids = kids_of(g.fronts, f, g.cmap, Uc);
+    // (columns past the own ones repeat the last of them: not used)
+    int c[2][4];
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) c[s][v] = min(c0 + 16 * s + lk + 4 * v, f.k - 1);
+    const int rc[2] = {min(c0 + li, last), min(c0 + 16 + li, last)};
+    bool failed = false;
+    if (wave == 0) {
+        // the diagonal block, formed and factorised while the other waves
+        // form rows (its upper 16 x 16 tile is computed with the rest)
+        v4d acc[2][2];
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int s = 0; s < 2; s++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[t][s][v] = Lf[c[s][v] * ld + rc[t]];
+        add_kids(acc, kids, rc, c);
+        tile_products<2, 2, 4>(acc, Lf, ld, rc, rc, c0, lk);
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int s = 0; s < 2; s++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    Q[16 * t + li][16 * s + lk + 4 * v] = acc[t][s][v];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        diag_block(Q, dinv, Lk, jn, lane, failed);
+        if (lane >= jn && lane < NF) dinv[lane] = 0.;
+    } else if (nr > 0) {
+        // waves 1 .. 3 form the rows, 16 at a time (3, 3 and 2 tiles)
+        v4d acc[3][2];
+        int row[3];
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            row[t] = min(r0 + 16 * (wave - 1 + 3 * t) + li, last);
+#pragma unroll
+            for (int s = 0; s < 2; s++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[t][s][v] = Lf[c[s][v] * ld + row[t]];
+        }
+        add_kids(acc, kids, row, c);
+        tile_products<3, 2, 4>(acc, Lf, ld, row, rc, c0, lk);
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            const int q = 16 * (wave - 1 + 3 * t) + li;
+            if (q < RB)
+#pragma unroll
+                for (int s = 0; s < 2; s++)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) P[q][16 * s + lk + 4 * v] = acc[t][s][v];
+        }
+    }
+    __syncthreads();
+    // the rows against L11: x L11^T = a, column by column
+    if (tid < nr) {
+        // (L11 is read from LDS where it is used, not hoisted into registers)
+        asm volatile("" ::: "memory");
+        double x[NF];
+#pragma unroll
+        for (int c = 0; c < NF; c++) x[c] = P[tid][c];
+#pragma unroll
+        for (int c = 0; c < NF; c++) {
+            x[c] *= dinv[c];
+#pragma unroll
+            for (int c2 = c + 1; c2 < NF; c2++) x[c2] -= x[c] * Q[c2][c];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        double *o = Lf + (int64_t)c0 * ld + r0 + tid;
+#pragma unroll
+        for (int c = 0; c < NF; c++) P[tid][c] = x[c];
+        for (int c = 0; c < jn; c++) o[c * ld] = P[tid][c];
+    } else if (wave == 3 && task.part == 0) {
+        // the factorised diagonal block, its reciprocal pivots on the
+        // diagonal (the entries in L stay: other workgroups still read them)
+        double *d = D + f.doff + (int64_t)p * NF * NF;
+        for (int t = lane; t < NF * NF; t += 64) {
+            const int r = t >> 5, c = t & 31;
+            d[t] = r == c ? dinv[r] : (r > c && r < jn) ? Q[r][c] : 0.;
+        }
+    }
+    if (failed && lane == 0 && task.part == 0) atomicAdd(bad, 1);
+}
+
+__global__ void __launch_bounds__(256)
+    nd_update(Image g, int64_t task0, const double *__restrict__ L, const double *__restrict__ Uc,
+              double *__restrict__ Uo)
+{
+    const Task task = g.tasks[task0 + blockIdx.x];
+    const Front f = g.fronts[task.front];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = lane & 15, lk = lane >> 4;
+    const int I = task.part >> 16, K = task.part & 0xffff;
+    const int wi = wave >> 1, wk = wave & 1;
+    if (I == K && wk > wi) return;  // above the diagonal
+    const int last = f.k + f.m - 1;
+    const int rb = TS * I + 32 * wi, cb = TS * K + 32 * wk;  // in the boundary
+    if (rb >= f.m || cb >= f.m) return;
+    v4d acc[2][2];
+    int row[2], rc[2], c[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        row[t] = min(f.k + rb + 16 * t + li, last);
+        rc[t] = min(f.k + cb + 16 * t + li, last);
+#pragma unroll
+        for (int v = 0; v < 4; v++) c[t][v] = min(f.k + cb + 16 * t + lk + 4 * v, last);
+#pragma unroll
+        for (int s = 0; s < 2; s++) acc[t][s] = v4d{0., 0., 0., 0.};
+    }
+    add_kids(acc, kids_of(g.fronts, f, g.cmap, Uc), row, c);
+    tile_products<2, 2, 4>(acc, L + f.loff, f.k + f.m, row, rc, f.k, lk);
+    double *U = Uo + f.uoff;
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const int r = rb + 16 * t + li;
+        if (r >= f.m) continue;
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int q = cb + 16 * s + lk + 4 * v;
+                if (q < f.m && r >= q) U[q * f.m + r] = acc[t][s][v];
+            }
+    }
+}
+
+// L y = f, front by front: own part of y (permuted numbering) from f and the
+// children's boundary parts, then the front's own boundary part into w
+__global__ void __launch_bounds__(256)
+    nd_forward(Image g, int64_t front0, const double *__restrict__ L, const double *__restrict__ D,
+               const double *__restrict__ f0, double *__restrict__ y, double *__restrict__ w)
+{
+    extern __shared__ double v[];  // k + m entries
+    __shared__ double T[NF][NF + 1];
+    const Front f = g.fronts[front0 + blockIdx.x];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = f.k + f.m;
+    const int32_t *map = g.cmap + 2 * f.noff;
+    const double *w0 = f.c0 < 0 ? nullptr : w + g.fronts[f.c0].woff;
+    const double *w1 = f.c1 < 0 ? nullptr : w + g.fronts[f.c1].woff;
+    for (int r = tid; r < n; r += 256) {
+        const int q = r / 6, d = r - 6 * q;
+        double s = r < f.k ? f0[6 * (int64_t)g.pnode[f.own0 + q] + d] : 0.;
+        if (w0 && map[2 * q] >= 0) s += w0[6 * map[2 * q] + d];
+        if (w1 && map[2 * q + 1] >= 0) s += w1[6 * map[2 * q + 1] + d];
+        v[r] = s;
+    }
+    const double *Lf = L + f.loff;
+    const int64_t ld = n;
+    for (int c0 = 0, p = 0; c0 < f.k; c0 += NF, p++) {
+        const int jn = min(NF, f.k - c0);
+        const double *d = D + f.doff + (int64_t)p * NF * NF;
+        for (int t = tid; t < NF * NF; t += 256) T[t >> 5][t & 31] = d[t];
+        __syncthreads();
+        if (wave == 0) {
+            double yc = lane < jn ? v[c0 + lane] : 0.;
+            const int rr = lane & 31;
+            for (int c = 0; c < jn; c++) {
+                if (lane == c) yc *= T[c][c];
+                const double yv = readlane_d(yc, c);
+                if (lane > c && lane < jn) yc -= T[rr][c] * yv;
+            }
+            if (lane < jn) v[c0 + lane] = yc;
+        }
+        __syncthreads();
+        for (int r = c0 + jn + tid; r < n; r += 256) {
+            const double *a = Lf + (int64_t)c0 * ld + r;
+            double acc = 0.;
+            if (jn == NF) {
+#pragma unroll 16
+                for (int c = 0; c < NF; c++) acc = fma(a[(int64_t)c * ld], v[c0 + c], acc);
+            } else {
+#pragma unroll 6
+                for (int c = 0; c < jn; c++) acc = fma(a[(int64_t)c * ld], v[c0 + c], acc);
+            }
+            v[r] -= acc;
+        }
+        __syncthreads();
+    }
+    if (f.k == 0) __syncthreads();
+    for (int r = tid; r < n; r += 256) {
+        if (r < f.k) y[6 * (int64_t)f.own0 + r] = v[r];
+        else w[f.woff + r - f.k] = v[r];
+    }
+}
+
+// L^T x = y, parents before children; x also goes back to the original
+// numbering
+__global__ void __launch_bounds__(256)
+    nd_backward(Image g, int64_t front0, const double *__restrict__ L,
+                const double *__restrict__ D, double *__restrict__ y, double *__restrict__ x)
+{
+    extern __shared__ double v[];
+    __shared__ double T[NF][NF + 1];
+    __shared__ double part[NF];
+    const Front f = g.fronts[front0 + blockIdx.x];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = f.k + f.m;
+    const int32_t *nodes = g.nodes + f.noff;
+    for (int r = tid; r < n; r += 256) {
+        const int q = r / 6;
+        v[r] = y[6 * (int64_t)nodes[q] + r - 6 * q];
+    }
+    __syncthreads();
+    const double *Lf = L + f.loff;
+    const int64_t ld = n;
+    for (int p = (f.k + NF - 1) / NF - 1; p >= 0; p--) {
+        const int c0 = p * NF, jn = min(NF, f.k - c0);
+        const double *d = D + f.doff + (int64_t)p * NF * NF;
+        for (int t = tid; t < NF * NF; t += 256) T[t >> 5][t & 31] = d[t];
+        // wave w: columns 8 w .. 8 w + 7 of the panel against the rows below
+        double s[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) s[j] = 0.;
+        for (int r = c0 + jn + lane; r < n; r += 64) {
+            const double vr = v[r];
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                s[j] = fma(Lf[(int64_t)min(c0 + 8 * wave + j, f.k - 1) * ld + r], vr, s[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) s[j] += __shfl_xor(s[j], o, 64);
+            if (lane == 0) part[8 * wave + j] = s[j];
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const int rr = lane & 31;
+            double rhs = lane < jn ? v[c0 + lane] - part[rr] : 0.;
+            for (int c = jn - 1; c >= 0; c--) {
+                if (lane == c) rhs *= T[c][c];
+                const double xv = readlane_d(rhs, c);
+                if (lane < c) rhs -= T[c][rr] * xv;
+            }
+            if (lane < jn) v[c0 + lane] = rhs;
+        }
+        __syncthreads();
+    }
+    for (int r = tid; r < f.k; r += 256) {
+        const int q = r / 6, d = r - 6 * q;
+        y[6 * (int64_t)f.own0 + r] = v[r];
+        x[6 * (int64_t)g.pnode[f.own0 + q] + d] = v[r];
+    }
+}
+
+inline unsigned nb256(int64_t n) { return (unsigned)((n + 255) / 256); }
+
+}  // namespace
+
+extern "C" {
+
+int pf3d_nd_create(int64_t n_nodes, const int32_t *row_ptr, const int32_t *col_idx,
+                   const int32_t *coord, int64_t n_sys, const int64_t *node0, int leaf,
+                   void **plan)
+{
+    if (n_nodes <= 0 || n_nodes > 357913941 || !row_ptr || !col_idx || n_sys <= 0 || !node0 ||
+        leaf < 1 || !plan)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nd_create: bad arguments");
+    *plan = nullptr;
+    if (node0[0] != 0 || node0[n_sys] != n_nodes || row_ptr[0] != 0)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nd_create: the systems must cover the nodes");
+    for (int64_t s = 0; s < n_sys; s++) {
+        if (node0[s + 1] < node0[s])
+            return pf3d_fail(PF3D_E_ARG, "pf3d_nd_create: node0 must not decrease");
+        for (int64_t r = node0[s]; r < node0[s + 1]; r++) {
+            if (row_ptr[r + 1] < row_ptr[r])
+                return pf3d_fail(PF3D_E_ARG, "pf3d_nd_create: row_ptr must not decrease");
+            for (int b = row_ptr[r]; b < row_ptr[r + 1]; b++)
+                if (col_idx[b] < node0[s] || col_idx[b] >= node0[s + 1])
+                    return pf3d_fail(PF3D_E_ARG, "pf3d_nd_create: a block couples two systems");
+        }
+    }
+    Plan *p = nullptr;
+    try {
+        p = new Plan;
+        build(*p, n_nodes, row_ptr, col_idx, coord, n_sys, node0, leaf);
+    } catch (const std::exception &) {
+        delete p;
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nd_create: out of memory");
+    }
+    if (p->widest > MAX_FRONT || p->fronts.size() > 2000000000 || p->tasks.size() > 2000000000) {
+        const int w = p->widest;
+        delete p;
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nd_create: a front of %d DOFs exceeds %d", w, MAX_FRONT);
+    }
+    *plan = p;
+    return PF3D_OK;
+}
+
+int pf3d_nd_sizes(const void *plan, int64_t *sizes, double *flops)
+{
+    if (!plan || !sizes || !flops) return pf3d_fail(PF3D_E_ARG, "pf3d_nd_sizes: bad arguments");
+    const Plan &p = *(const Plan *)plan;
+    sizes[0] = (int64_t)Layout(p).total;
+    sizes[1] = p.l_size + p.d_size;
+    sizes[2] = p.u_size[0] + p.u_size[1];
+    sizes[3] = 6 * p.n_nodes + p.w_size;
+    sizes[4] = (int64_t)p.fronts.size();
+    sizes[5] = p.widest;
+    *flops = p.flops;
+    return PF3D_OK;
+}
+
+int pf3d_nd_image(const void *plan, void *image)
+{
+    if (!plan || !image) return pf3d_fail(PF3D_E_ARG, "pf3d_nd_image: bad arguments");
+    const Plan &p = *(const Plan *)plan;
+    const Layout l(p);
+    char *b = (char *)image;
+    memcpy(b + l.fronts, p.fronts.data(), p.fronts.size() * sizeof(Front));
+    memcpy(b + l.tasks, p.tasks.data(), p.tasks.size() * sizeof(Task));
+    memcpy(b + l.nodes, p.nodes.data(), p.nodes.size() * 4);
+    memcpy(b + l.cmap, p.cmap.data(), p.cmap.size() * 4);
+    memcpy(b + l.pnode, p.pnode.data(), p.pnode.size() * 4);
+    memcpy(b + l.ld, p.ld.data(), p.ld.size() * 4);
+    memcpy(b + l.dest, p.dest.data(), p.dest.size() * 8);
+    return PF3D_OK;
+}
+
+int pf3d_nd_free(void *plan)
+{
+    delete (Plan *)plan;
+    return PF3D_OK;
+}
+
+int pf3d_nd_factor(const void *plan, const void *image, const double *val, double *factor,
+                   double *update, int *bad, void *stream)
+{
+    if (!plan || !image || !val || !factor || !update || !bad)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nd_factor: null argument");
+    const Plan &p = *(const Plan *)plan;
+    const Image g = image_at(p, image);
+    hipStream_t s = (hipStream_t)stream;
+    double *L = factor, *D = factor + p.l_size;
+    double *U[2] = {update, update + p.u_size[0]};
+    const unsigned zb = std::min(nb256(p.l_size), 16384u);
+    hipLaunchKernelGGL(nd_zero, dim3(zb), dim3(256), 0, s, p.l_size, L);
+    hipLaunchKernelGGL(nd_scatter, dim3(nb256(p.nnzb * 36)), dim3(256), 0, s, p.nnzb, g.dest, g.ld,
+                       val, L);
+    int depth = (int)p.levels.size() - 1;
+    for (const Level &lv : p.levels) {
+        const double *Uc = U[(depth + 1) & 1];
+        for (size_t q = 0; q < lv.panels.size(); q++) {
+            const auto t = lv.panels[q];
+            hipLaunchKernelGGL(nd_panel, dim3((unsigned)(t.second - t.first)), dim3(256), 0, s, g,
+                               t.first, (int)q, L, D, Uc, bad);
+        }
+        if (lv.upd1 > lv.upd0)
+            hipLaunchKernelGGL(nd_update, dim3((unsigned)(lv.upd1 - lv.upd0)), dim3(256), 0, s, g,
+                               lv.upd0, L, Uc, U[depth & 1]);
+        depth--;
+    }
+    return pf3d_hip_check(hipGetLastError(), "pf3d_nd_factor");
+}
+
+int pf3d_nd_solve(const void *plan, const void *image, const double *factor, const double *f,
+                  double *x, double *work, void *stream)
+{
+    if (!plan || !image || !factor || !f || !x || !work)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nd_solve: null argument");
+    const Plan &p = *(const Plan *)plan;
+    const Image g = image_at(p, image);
+    hipStream_t s = (hipStream_t)stream;
+    const double *L = factor, *D = factor + p.l_size;
+    double *y = work, *w = work + 6 * p.n_nodes;
+    const size_t lds = (size_t)p.widest * sizeof(double);
+    for (const Level &lv : p.levels)
+        hipLaunchKernelGGL(nd_forward, dim3((unsigned)(lv.front1 - lv.front0)), dim3(256), lds, s,
+                           g, lv.front0, L, D, f, y, w);
+    for (size_t i = p.levels.size(); i-- > 0;)
+        hipLaunchKernelGGL(nd_backward, dim3((unsigned)(p.levels[i].front1 - p.levels[i].front0)),
+                           dim3(256), lds, s, g, p.levels[i].front0, L, D, y, x);
+    return pf3d_hip_check(hipGetLastError(), "pf3d_nd_solve");
+}
+
+}  // extern "C"

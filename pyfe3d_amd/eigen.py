@@ -10,7 +10,7 @@ Shift-invert Lanczos: with C = A - sigma B (symmetric positive definite for
 the shifts used here) the operator T = C^-1 B is self-adjoint in the
 C-inner product and its largest eigenvalues theta = 1 / (lambda - sigma)
 belong to the eigenvalues lambda closest above sigma.  Each step is one
-block-sparse product with B, one banded Cholesky solve with C (factorised
+block-sparse product with B, one sparse Cholesky solve with C (factorised
 once, on the GPU) and a full re-orthogonalisation against the basis in the
 C-inner product (the basis V and U = C V are both kept, so no product with
 C is needed).  Fixed DOFs are removed as in the static solve: identity rows
@@ -57,10 +57,7 @@ class GeneralizedEigen:
                   self.plan.col_idx.data_ptr(), val.data_ptr(), x.data_ptr(), y.data_ptr(), _s())
 
     def _csolve(self, f, x):
-        c = self.C
-        _lib.call('pf3d_band_solve', 1, None, c._band_dof0.data_ptr(), c._band_bw.data_ptr(),
-                  c._band_off.data_ptr(), c._band.data_ptr(), c._band_pnode.data_ptr(),
-                  f.data_ptr(), x.data_ptr(), c._band_work.data_ptr(), 0, _s())
+        self.C.direct_solve(f, x)
 
     def _dots(self, V, j, x, out):
         """out[0:j] = V[:, 0:j]^T x"""

@@ -90,49 +90,69 @@ class StaticSystem:
         f[self.fixed.bool()] = 0.
         return f
 
-    def factor_direct(self, stream=None):
-        """Banded Cholesky of the system on the GPU (one workgroup), in the
-        node numbering (given, or reverse Cuthill-McKee; host, once) with the
-        narrower band.  Raises if the band is wider than the kernels accept."""
+    def _band_numbering(self):
+        """(half-bandwidth in DOF, permuted order of the nodes and its inverse)
+        of the given numbering or reverse Cuthill-McKee, whichever band is
+        narrower (host)."""
         import scipy.sparse as ss
         from scipy.sparse.csgraph import reverse_cuthill_mckee
         nb = self.nb
-        if not hasattr(self, '_band'):
+        rp = self.plan.row_ptr.cpu().numpy()
+        ci = self.plan.col_idx.cpu().numpy()
+        g = ss.csr_matrix((np.ones(ci.size), ci, rp), shape=(nb, nb))
+        rows = np.repeat(np.arange(nb), np.diff(rp))
+        best = None
+        for pnode in (np.arange(nb, dtype=np.int64),
+                      np.asarray(reverse_cuthill_mckee(g, symmetric_mode=True), np.int64)):
+            pinv = np.empty_like(pnode)
+            pinv[pnode] = np.arange(nb)
+            w = 6 * int(np.abs(pinv[rows] - pinv[ci]).max()) + 5
+            if best is None or w < best[0]:
+                best = (w, pnode, pinv)
+        return best
+
+    @property
+    def bandwidth(self):
+        """Half-bandwidth (DOF) of the narrower of the two numberings."""
+        return self._band_numbering()[0]
+
+    def _direct_plan(self):
+        """The pattern's nested-dissection plan, kept with the pattern."""
+        d = getattr(self.plan, '_dissection', None)
+        if d is None:
+            from .direct import DirectPlan
             rp = self.plan.row_ptr.cpu().numpy()
             ci = self.plan.col_idx.cpu().numpy()
-            g = ss.csr_matrix((np.ones(ci.size), ci, rp), shape=(nb, nb))
-            rows = np.repeat(np.arange(nb), np.diff(rp))
-            best = None
-            # the given numbering or reverse Cuthill-McKee, whichever band is narrower
-            for pnode in (np.arange(nb, dtype=np.int64),
-                          np.asarray(reverse_cuthill_mckee(g, symmetric_mode=True), np.int64)):
-                pinv = np.empty_like(pnode)
-                pinv[pnode] = np.arange(nb)
-                w = 6 * int(np.abs(pinv[rows] - pinv[ci]).max()) + 5
-                if best is None or w < best[0]:
-                    best = (w, pnode, pinv)
-            bw, pnode, pinv = best
             maxb = _lib.call('pf3d_band_max_width')
-            if bw > maxb:
-                raise ValueError('bandwidth %d after renumbering exceeds %d: use PCG' % (bw, maxb))
-            dev = self.val.device
-            self._band_bw = torch.tensor([bw], dtype=torch.int32, device=dev)
-            self._band_off = torch.zeros(1, dtype=torch.int64, device=dev)
-            self._band_dof0 = torch.tensor([0, 6 * nb], dtype=torch.int64, device=dev)
-            self._band_var = torch.zeros(nb, dtype=torch.int32, device=dev)
-            self._band_pinv = torch.as_tensor(pinv, device=dev)
-            self._band_pnode = torch.as_tensor(pnode, device=dev)
-            self._band_size = 6 * nb * (bw + 1)
-            self._band = torch.empty(self._band_size, dtype=torch.float64, device=dev)
-            self._band_work = torch.empty(6 * nb, dtype=torch.float64, device=dev)
+            rows = np.repeat(np.arange(self.nb), np.diff(rp))
+            if 6 * int(np.abs(rows - ci[:rows.size]).max(initial=0)) + 5 > maxb:
+                bw = self._band_numbering()[0]
+                if bw > maxb:
+                    raise ValueError('bandwidth %d after renumbering exceeds %d: use PCG'
+                                     % (bw, maxb))
+            d = self.plan._dissection = DirectPlan(rp, ci, self.val.device)
+        return d
+
+    def factor_direct(self, stream=None):
+        """Cholesky factor of the system on the GPU by nested dissection
+        (pyfe3d_amd.direct).  Raises if no numbering of the nodes (given, or
+        reverse Cuthill-McKee) has a band within pf3d_band_max_width."""
+        d = self._direct_plan()
+        dev = self.val.device
+        if not hasattr(self, '_factor'):
+            self._factor = torch.empty(d.factor_size, dtype=torch.float64, device=dev)
+            self._direct_work = torch.empty(d.work_size, dtype=torch.float64, device=dev)
             self._band_bad = torch.zeros(1, dtype=torch.int32, device=dev)
-            self.bandwidth = bw
-        _lib.call('pf3d_band_factor', 1, nb, None, self._band_dof0.data_ptr(),
-                  self._band_bw.data_ptr(), self._band_off.data_ptr(), self._band_size,
-                  self._band.data_ptr(), self.plan.row_ptr.data_ptr(),
-                  self.plan.col_idx.data_ptr(), self.val.data_ptr(), self._band_var.data_ptr(),
-                  self._band_pinv.data_ptr(), self._band_bad.data_ptr(), 0, 0, _s(stream))
+        with torch.cuda.stream(stream):  # (the scratch belongs to the launch stream)
+            update = torch.empty(max(1, d.update_size), dtype=torch.float64, device=dev)
+            d.factor(self.val.data_ptr(), self._factor, update, self._band_bad, _s(stream))
         self._factored = True
+
+    def direct_solve(self, b, x, stream=None):
+        """x = K^-1 b with the factor of :meth:`factor_direct`."""
+        self._direct_plan().solve(self._factor, b.data_ptr(), x.data_ptr(), self._direct_work,
+                                  _s(stream))
+        return x
 
     def setup_amg(self, xyz, log=None, precisions=('fp64',), graph=True, **kw):
         """Smoothed-aggregation multigrid for method='amg' (FP64 V-cycle)
@@ -175,7 +195,7 @@ class StaticSystem:
         matrix with FP64 vectors and a true FP64 residual replacing the
         recursive one every `replace` iterations; info['outer'] counts the
         replacements), 'ir' (FP64 iterative refinement around restarted
-        FP32-matrix PCG solves to inner_rtol) or 'direct' (banded Cholesky,
+        FP32-matrix PCG solves to inner_rtol) or 'direct' (sparse Cholesky,
         factor kept for later right-hand sides unless refactor), 'amg' (CG
         preconditioned by one smoothed-aggregation V-cycle per iteration,
         after setup_amg) or 'amg32' (the same with the V-cycle in FP32, after
@@ -241,12 +261,9 @@ class StaticSystem:
         elif method == 'direct':
             if refactor or not getattr(self, '_factored', False):
                 self.factor_direct(stream=stream)
-            _lib.call('pf3d_band_solve', 1, None, self._band_dof0.data_ptr(),
-                      self._band_bw.data_ptr(), self._band_off.data_ptr(),
-                      self._band.data_ptr(), self._band_pnode.data_ptr(), b.data_ptr(),
-                      x.data_ptr(), self._band_work.data_ptr(), 0, _s(stream))
+            self.direct_solve(b, x, stream=stream)
             if int(self._band_bad.item()):
-                raise _lib.Pf3dError('band factorisation met a non-positive pivot')
+                raise _lib.Pf3dError('the factorisation met a non-positive pivot')
             info = dict(iters=0, outer=0)
         else:
             raise ValueError(method)

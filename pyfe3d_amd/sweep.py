@@ -32,6 +32,9 @@ from .sparse import BlockPlan
 # LDS panel width of the narrow factorisation shape: 74 KB of LDS, so two
 # workgroups share a CU (the 448-wide panel takes one CU each)
 NARROW_PANEL = 256
+# the sweep is solved by nested dissection when its widest band (DOFs)
+# exceeds this, else by the banded kernels
+BANDED_MAX = 96
 
 
 def split_order(bandwidths, sizes, narrow=NARROW_PANEL):
@@ -321,17 +324,50 @@ class PlateSweep:
             chol(self.n_var - nw, order[nw:].data_ptr(), sft, NARROW_PANEL, side.cuda_stream)
         main.wait_stream(side)
 
+    def _dissection(self):
+        """The sweep's nested-dissection plan and buffers, or None where the
+        banded kernels are used."""
+        if not hasattr(self, '_batch'):
+            dims = np.array(self.dims)
+            bw = 6 * (dims.min(axis=1) + 2) + 5
+            maxb = _lib.call('pf3d_band_max_width')
+            if bw.max() > maxb:
+                raise ValueError('plate too wide for the direct solver (bandwidth %d > %d)'
+                                 % (bw.max(), maxb))
+            self._batch = None
+            if bw.max() > BANDED_MAX:
+                from .direct import DirectBatch
+                ny = np.repeat(dims[:, 1] + 1, np.diff(self.node0))
+                local = np.arange(self.n_nodes) - np.repeat(self.node0[:-1], np.diff(self.node0))
+                coord = np.stack([local // ny, local % ny], axis=1)  # PlateMesh: i * ny + j
+                self._batch = DirectBatch(self.plan.row_ptr.cpu().numpy(),
+                                          self.plan.col_idx.cpu().numpy(), self.device,
+                                          self.node0, coord)
+        return self._batch
+
     def solve_direct(self, rtol=1e-8, polish_iter=0, config=None, stream=None):
-        """Banded Cholesky of every variant (one workgroup each) with the
-        forward substitution fused into it, the backward substitution, then
-        the FP64 true residual of each variant into self.relres (and, with
+        """Cholesky factorisation and solve of every variant, then the FP64
+        true residual of each variant into self.relres (and, with
         polish_iter > 0, block-Jacobi PCG from the direct solution for any
-        variant that misses rtol).  config: (factor threads, panel
-        bandwidth, solve threads[, narrow-band factor threads]), default the
-        one chosen by :meth:`autotune_direct`, else (1024, 576, 1024)."""
+        variant that misses rtol).
+
+        Without config: nested dissection (pyfe3d_amd.direct) for sweeps with
+        a band wider than BANDED_MAX, else the banded kernels with the launch
+        shape chosen by :meth:`autotune_direct`, else (1024, 576, 1024).
+        config: the banded kernels with (factor threads, panel bandwidth,
+        solve threads[, narrow-band factor threads]): banded Cholesky of every
+        variant (one workgroup each) with the forward substitution fused into
+        it, then the backward substitution."""
+        s = _s(stream)
+        batch = None if config is not None else self._dissection()
+        if batch is not None:
+            if polish_iter > 0:
+                self.precondition(stream=stream)
+            batch.solve(self.val, self.f, self.u, s)
+            self.solve(mode='fp64', rtol=rtol, max_iter=polish_iter, x0=True, stream=stream)
+            return
         if not hasattr(self, 'band'):
             self._band_setup()
-        s = _s(stream)
         cfg = self._direct_config(config)
         st = cfg[2]
         self.factor_direct(config=cfg, stream=stream, forward=True)
@@ -481,6 +517,9 @@ class PlateSweep:
             raise _lib.Pf3dError('%d singular diagonal blocks' % int(self.singular.item()))
         if hasattr(self, 'band_bad') and int(self.band_bad.item()):
             raise _lib.Pf3dError('%d band factorisations failed' % int(self.band_bad.item()))
+        if getattr(self, '_batch', None) is not None and int(self._batch.bad.item()):
+            raise _lib.Pf3dError('%d panels of the factorisation met a non-positive pivot'
+                                 % int(self._batch.bad.item()))
 
     def variant(self, v):
         """(node range, element range) of variant v."""

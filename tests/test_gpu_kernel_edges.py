@@ -83,3 +83,176 @@ def test_static_system_setup(etype, nx, ny):
         # residual of an inverse by elimination with pivoting: a few n eps cond
         assert np.abs(inv @ blk - np.eye(6)).max() <= 64 * 2.3e-16 * np.linalg.cond(blk)
     assert torch.equal(s.dinv32, s.dinv.to(torch.float32))
+
+
+def _graph(name):
+    """Block pattern as a list of neighbour sets."""
+    rng = np.random.default_rng(len(name))
+
+    def grid(nx, ny, hole=False):
+        at, nb = {}, []
+        for i in range(nx):
+            for j in range(ny):
+                if hole and nx // 3 < i < 2 * nx // 3 and ny // 3 < j < 2 * ny // 3:
+                    continue
+                at[i, j] = len(at)
+        nb = [set() for _ in at]
+        for (i, j), v in at.items():
+            for di in (-1, 0, 1):
+                for dj in (-1, 0, 1):
+                    if (i + di, j + dj) in at:
+                        nb[v].add(at[i + di, j + dj])
+        return nb
+
+    if name == 'one':
+        return [{0}]
+    if name == 'chain':
+        return [{j for j in (i - 1, i, i + 1) if 0 <= j < 90} for i in range(90)]
+    if name == 'isolated':
+        return grid(6, 5) + [{30 + i} for i in range(7)]
+    if name == 'two parts':
+        a = grid(9, 7)
+        return a + [{v + len(a) for v in s} for s in a]
+    if name == 'complete':
+        return [set(range(40)) for _ in range(40)]
+    if name == 'random':
+        nb = [{i} for i in range(160)]
+        for _ in range(260):
+            a, b = rng.integers(0, 160, 2)
+            nb[a].add(b)
+            nb[b].add(a)
+        return nb
+    nx, ny = (int(t) for t in name.split(' ')[0].split('x'))
+    return grid(nx, ny, 'hole' in name)
+
+
+def _block_system(nb, seed):
+    """(row_ptr, col_idx, values (nnzb, 6, 6), dense) of a random symmetric,
+    diagonally dominant matrix on the pattern."""
+    rng = np.random.default_rng(seed)
+    n = len(nb)
+    rp = np.concatenate([[0], np.cumsum([len(s) for s in nb])]).astype(np.int32)
+    ci = np.concatenate([sorted(s) for s in nb]).astype(np.int32)
+    A = np.zeros((n, 6, n, 6))
+    for r in range(n):
+        for c in sorted(nb[r]):
+            if c <= r:
+                A[r, :, c, :] = rng.uniform(-1, 1, (6, 6))
+    A = A.reshape(6 * n, 6 * n)
+    A = np.tril(A, -1)
+    A = A + A.T
+    A[np.diag_indices(6 * n)] = np.abs(A).sum(axis=1) + 1.
+    rows = np.repeat(np.arange(n), np.diff(rp))
+    val = A.reshape(n, 6, n, 6)[rows, :, ci, :]
+    return rp, ci, val, A
+
+
+@pytest.mark.parametrize('leaf', [1, 5, 16])
+@pytest.mark.parametrize('name', ['one', 'chain', '2x2', '7x5', '16x16', '40x9', '23x23 hole',
+                                  'isolated', 'two parts', 'complete', 'random'])
+def test_dissection_against_dense(name, leaf):
+    """Nested dissection on patterns with fronts of 6 to 240 own DOFs, panels
+    of 6 to 32 columns, more and less than 128 rows, empty separators and
+    isolated nodes, two right-hand sides from one factor.  Diagonally
+    dominant matrices (condition below 1e3): 1e-12 of numpy's solution."""
+    from pyfe3d_amd.direct import DirectPlan
+    rp, ci, val, A = _block_system(_graph(name), leaf)
+    plan = DirectPlan(rp, ci, DEV, leaf=leaf)
+    n = A.shape[0]
+    new = lambda m: torch.full((max(1, m),), float('nan'), dtype=torch.float64, device=DEV)
+    factor, update, work = new(plan.factor_size), new(plan.update_size), new(plan.work_size)
+    bad = torch.zeros(1, dtype=torch.int32, device=DEV)
+    tv = T(val.reshape(-1), torch.float64)
+    s = torch.cuda.current_stream().cuda_stream
+    plan.factor(tv.data_ptr(), factor, update, bad, s)
+    rng = np.random.default_rng(7)
+    for _ in range(2):
+        b = rng.normal(size=n)
+        tb, x = T(b, torch.float64), new(n)
+        plan.solve(factor, tb.data_ptr(), x.data_ptr(), work, s)
+        ref = np.linalg.solve(A, b)
+        err = np.linalg.norm(x.cpu().numpy() - ref) / np.linalg.norm(ref)
+        print(name, leaf, 'err %.2e, %d fronts, widest %d' % (err, plan.n_fronts, plan.widest))
+        assert err <= 1e-12
+    assert int(bad.item()) == 0
+    # not positive definite: reported
+    val[rp[:-1] + [sorted(s_).index(i) for i, s_ in enumerate(_graph(name))]] *= -1.
+    tv = T(val.reshape(-1), torch.float64)
+    plan.factor(tv.data_ptr(), factor, update, bad, s)
+    assert int(bad.item()) > 0
+
+
+def test_dissection_sweep_matches_banded(monkeypatch):
+    """The sweep's route by nested dissection against the banded kernels
+    (an explicit launch shape) on uneven plates: every variant within 1e-9
+    and at the same residual level; one group or several, graph replays and
+    eager steps: the same bits."""
+    import pyfe3d_amd.direct as D
+    from pyfe3d_amd.sweep import PlateSweep
+    dims = [(41, 50), (10, 12), (2, 40), (20, 30), (8, 64), (3, 3)]
+    sw = PlateSweep(dims)
+    h, f = sw.random_designs(5)
+    sw.set_thickness(h)
+    sw.set_loads(f)
+    sw.assemble()
+    sw.solve_direct(config=(512, 448, 512))
+    ref, res = sw.u.clone(), sw.relres.clone()
+    sw.u.zero_()
+    sw.solve_direct()
+    sw.check()
+    got = sw.u.clone()
+    assert len(sw._batch.groups) == 1
+    assert float(sw.relres.max()) <= max(1e-8, 2 * float(res.max()))
+    for v in range(sw.n_var):
+        nodes, _ = sw.variant(v)
+        a, b = ref[6 * nodes.start:6 * nodes.stop], got[6 * nodes.start:6 * nodes.stop]
+        assert float((a - b).norm()) <= 1e-9 * float(a.norm()), v
+    monkeypatch.setattr(D.DirectBatch, 'GROUP_NODES', 1000)
+    sw2 = PlateSweep(dims)
+    sw2.set_thickness(h)
+    sw2.set_loads(f)
+    g = sw2.capture(mode='direct')
+    assert len(sw2._batch.groups) > 1
+    for seed in (5, 9, 5):
+        h, f = sw2.random_designs(seed)
+        sw2.set_thickness(h)
+        sw2.set_loads(f)
+        g.replay()
+        torch.cuda.synchronize()
+        u = sw2.u.clone()
+        sw2.step(mode='direct')
+        assert torch.equal(u, sw2.u), seed
+    assert torch.equal(u, got)
+
+
+def test_direct_refuses_wide_bands_and_takes_streams():
+    """A star of 240 nodes has no numbering within the widest band: refused
+    as before; a plate factorised and solved on a side stream gives the
+    current stream's bits; a singular system is reported."""
+    from types import SimpleNamespace
+    from pyfe3d_amd import _lib
+    from pyfe3d_amd.solver import StaticSystem
+    nb = [set(range(240))] + [{0, i} for i in range(1, 240)]
+
+    def system(nb, seed, **kw):
+        rp, ci, val, A = _block_system(nb, seed)
+        plan = SimpleNamespace(row_ptr=T(rp, torch.int32), col_idx=T(ci, torch.int32),
+                               n_nodes=len(nb))
+        return StaticSystem(plan, T(val.reshape(-1), torch.float64), np.zeros(6 * len(nb)), **kw)
+
+    with pytest.raises(ValueError, match='exceeds'):
+        system(nb, 1).factor_direct()
+    grid = _graph('12x9')
+    f = np.random.default_rng(3).normal(size=6 * len(grid))
+    a = system(grid, 2)
+    u, info = a.solve(f, method='direct')
+    assert info['converged'] and a.bandwidth == 6 * 10 + 5
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        v, _ = system(grid, 2, stream=s).solve(f, method='direct', stream=s)
+    s.synchronize()
+    assert torch.equal(u, v)
+    a.val.neg_()
+    with pytest.raises(_lib.Pf3dError):
+        a.solve(f, method='direct', refactor=True)
