@@ -607,10 +607,12 @@ int pf3d_nd_free(void *plan);
 
 /* Factorise (val: the BSR values; *bad, a device int, counts panels that met
  * a non-positive pivot), then solve any number of right-hand sides (f, x: 6
- * doubles per node in the original numbering).  Kernel launches only: no
- * allocation, no synchronisation. */
-int pf3d_nd_factor(const void *plan, const void *image, const double *val, double *factor,
-                   double *update, int *bad, void *stream);
+ * doubles per node in the original numbering).  A right-hand side given to
+ * pf3d_nd_factor (else NULL) is carried through the factorisation, and
+ * pf3d_nd_solve with f = NULL then runs the backward substitution only.
+ * Kernel launches only: no allocation, no synchronisation. */
+int pf3d_nd_factor(const void *plan, const void *image, const double *val, const double *f,
+                   double *factor, double *update, int *bad, void *stream);
 int pf3d_nd_solve(const void *plan, const void *image, const double *factor, const double *f,
                   double *x, double *work, void *stream);
 

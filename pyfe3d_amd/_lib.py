@@ -104,7 +104,7 @@ SIGNATURES = {
     'pf3d_nd_sizes': [P, P, P],
     'pf3d_nd_image': [P, P],
     'pf3d_nd_free': [P],
-    'pf3d_nd_factor': [P, P, P, P, P, P, P],
+    'pf3d_nd_factor': [P, P, P, P, P, P, P, P],
     'pf3d_nd_solve': [P, P, P, P, P, P, P],
     'pf3d_nn_gemm': [I32, I32, I32, P, I64, I64, P, I64, I64, P, I64, I32, P, I32, I32, P, P],
     'pf3d_nn_im2col': [I32, I32, I32, I32, I32, P, P, P],

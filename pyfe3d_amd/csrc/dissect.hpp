@@ -18,10 +18,16 @@ constexpr int NF = 32;    // panel width (DOFs)
 constexpr int RB = 128;   // rows below the diagonal block per workgroup
 constexpr int TS = 64;    // update tile
 
+// column length of a panel (n rows and the right-hand side's) and of an
+// update matrix: whole 128-byte lines
+constexpr int32_t LINE = 16;
+constexpr int32_t column(int32_t rows) { return (rows + LINE - 1) / LINE * LINE; }
+
 // One front: k own DOFs (eliminated here) and m boundary DOFs.  Its panel
-// is k columns of k + m rows (column-major) at loff; its update matrix m x m
-// at uoff of the buffer of its depth's parity; its diagonal blocks at doff,
-// NF x NF per panel.  noff: its own-then-boundary node list in `nodes` and
+// is k columns of k + m + 1 rows (column-major) at loff, the last row the
+// right-hand side; its update matrix, m columns of m + 1 rows, at uoff of
+// the buffer of its depth's parity; its diagonal blocks at doff, NF x NF per
+// panel.  noff: its own-then-boundary node list in `nodes` and
 // `cmap`.  woff: its boundary part of a right-hand side.  c0, c1: its
 // children (-1: none).
 struct Front {
@@ -47,6 +53,8 @@ struct Plan {
     std::vector<int32_t> pnode;   // original node of each permuted one
     std::vector<int64_t> dest;    // panel offset of each BSR block, -1: the upper one of its pair
     std::vector<int32_t> ld;      // its panel's column length
+    std::vector<int64_t> rdest;   // right-hand side entry of each permuted node's first column
+    std::vector<int32_t> rld;
     std::vector<Task> tasks;
     std::vector<Level> levels;    // deepest first
     int64_t l_size = 0, d_size = 0, u_size[2] = {0, 0}, w_size = 0;
@@ -394,13 +402,13 @@ inline void build(Plan &P, int64_t n_nodes, const int32_t *rp, const int32_t *ci
             F.depth = d;
             F.c0 = f.c0 < 0 ? -1 : id[si.first][f.c0];
             F.c1 = f.c1 < 0 ? -1 : id[si.first][f.c1];
-            const int64_t n = F.k + F.m, np = (F.k + NF - 1) / NF;
+            const int32_t n = F.k + F.m, np = (F.k + NF - 1) / NF;
             F.loff = P.l_size;
-            P.l_size += n * F.k;
+            P.l_size += (int64_t)column(n + 1) * F.k;
             F.doff = P.d_size;
-            P.d_size += np * NF * NF;
+            P.d_size += (int64_t)np * NF * NF;
             F.uoff = uoff;
-            uoff += (int64_t)F.m * F.m;
+            uoff += (int64_t)F.m * column(F.m + 1);
             F.woff = P.w_size;
             P.w_size += F.m;
             F.noff = (int64_t)P.nodes.size();
@@ -424,17 +432,17 @@ inline void build(Plan &P, int64_t n_nodes, const int32_t *rp, const int32_t *ci
             for (int64_t f = lv.front0; f < lv.front1; f++) {
                 const Front &F = P.fronts[f];
                 if (F.k <= p * NF) continue;
-                const int below = F.k + F.m - std::min(F.k, (p + 1) * NF);
-                const int parts = std::max(1, (below + RB - 1) / RB);
+                const int below = F.k + F.m + 1 - std::min(F.k, (p + 1) * NF);
+                const int parts = (below + RB - 1) / RB;
                 for (int q = 0; q < parts; q++) P.tasks.push_back({(int32_t)f, q});
             }
             lv.panels.push_back({t0, (int64_t)P.tasks.size()});
         }
         lv.upd0 = (int64_t)P.tasks.size();
         for (int64_t f = lv.front0; f < lv.front1; f++) {
-            const int nt = (P.fronts[f].m + TS - 1) / TS;
-            for (int j = 0; j < nt; j++)
-                for (int i = j; i < nt; i++) P.tasks.push_back({(int32_t)f, (i << 16) | j});
+            const int m = P.fronts[f].m;
+            for (int j = 0; j < (m + TS - 1) / TS; j++)
+                for (int i = j; i < (m + TS) / TS; i++) P.tasks.push_back({(int32_t)f, (i << 16) | j});
         }
         lv.upd1 = (int64_t)P.tasks.size();
         P.levels.push_back(std::move(lv));
@@ -459,8 +467,17 @@ inline void build(Plan &P, int64_t n_nodes, const int32_t *rp, const int32_t *ci
     // where each BSR block goes: the panel of the earlier of its two nodes
     std::vector<int32_t> perm(n_nodes), owner(n_nodes);
     for (int64_t i = 0; i < n_nodes; i++) perm[P.pnode[i]] = (int32_t)i;
-    for (size_t f = 0; f < P.fronts.size(); f++)
-        for (int i = 0; i < P.fronts[f].k / 6; i++) owner[P.fronts[f].own0 + i] = (int32_t)f;
+    P.rdest.resize(n_nodes);
+    P.rld.resize(n_nodes);
+    for (size_t f = 0; f < P.fronts.size(); f++) {
+        const Front &F = P.fronts[f];
+        const int32_t n = F.k + F.m;
+        for (int i = 0; i < F.k / 6; i++) {
+            owner[F.own0 + i] = (int32_t)f;
+            P.rld[F.own0 + i] = column(n + 1);
+            P.rdest[F.own0 + i] = F.loff + (int64_t)6 * i * column(n + 1) + n;
+        }
+    }
     P.dest.assign(P.nnzb, -1);
     P.ld.assign(P.nnzb, 0);
     each(n_sys, 1, [&](int64_t s) {
@@ -472,7 +489,7 @@ inline void build(Plan &P, int64_t n_nodes, const int32_t *rp, const int32_t *ci
                 const int32_t *mine = P.nodes.data() + F.noff;
                 const int cnt = (F.k + F.m) / 6;
                 const int64_t row = std::lower_bound(mine, mine + cnt, p) - mine;
-                P.ld[b] = F.k + F.m;
+                P.ld[b] = column(F.k + F.m + 1);
                 P.dest[b] = F.loff + (int64_t)6 * (q - F.own0) * P.ld[b] + 6 * row;
             }
     });

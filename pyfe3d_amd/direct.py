@@ -59,15 +59,18 @@ class DirectPlan:
         if plan:
             self._free(plan)
 
-    def factor(self, val, factor, update, bad, stream):
+    def factor(self, val, factor, update, bad, stream, f=None):
         """Cholesky factor of the systems with BSR values val (device
         address) into factor (factor_size doubles); update (update_size) is
-        scratch; bad counts systems' panels with a non-positive pivot."""
-        _lib.call('pf3d_nd_factor', self._plan, self.image.data_ptr(), val, factor.data_ptr(),
+        scratch; bad counts systems' panels with a non-positive pivot.  f: a
+        right-hand side (device address) whose forward substitution is
+        carried along; :meth:`solve` with f None then finishes it."""
+        _lib.call('pf3d_nd_factor', self._plan, self.image.data_ptr(), val, f, factor.data_ptr(),
                   update.data_ptr(), bad.data_ptr(), stream)
 
     def solve(self, factor, f, x, work, stream):
-        """x = A^-1 f (device addresses; 6 doubles per node)."""
+        """x = A^-1 f (device addresses; 6 doubles per node); f None: the
+        right-hand side given to :meth:`factor`."""
         _lib.call('pf3d_nd_solve', self._plan, self.image.data_ptr(), factor.data_ptr(), f, x,
                   work.data_ptr(), stream)
 
@@ -108,5 +111,6 @@ class DirectBatch:
     def solve(self, val, f, x, stream):
         """x = A^-1 f for BSR values val (contiguous FP64 tensors)."""
         for plan, vo, fo in self.groups:
-            plan.factor(val.data_ptr() + vo, self.factor, self.update, self.bad, stream)
-            plan.solve(self.factor, f.data_ptr() + fo, x.data_ptr() + fo, self.work, stream)
+            plan.factor(val.data_ptr() + vo, self.factor, self.update, self.bad, stream,
+                        f=f.data_ptr() + fo)
+            plan.solve(self.factor, None, x.data_ptr() + fo, self.work, stream)

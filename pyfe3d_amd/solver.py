@@ -133,9 +133,10 @@ class StaticSystem:
             d = self.plan._dissection = DirectPlan(rp, ci, self.val.device)
         return d
 
-    def factor_direct(self, stream=None):
+    def factor_direct(self, stream=None, b=None):
         """Cholesky factor of the system on the GPU by nested dissection
-        (pyfe3d_amd.direct).  Raises if no numbering of the nodes (given, or
+        (pyfe3d_amd.direct); b: a right-hand side whose forward substitution
+        is carried along (then direct_solve(None, x) finishes it).  Raises if no numbering of the nodes (given, or
         reverse Cuthill-McKee) has a band within pf3d_band_max_width."""
         d = self._direct_plan()
         dev = self.val.device
@@ -145,13 +146,15 @@ class StaticSystem:
             self._band_bad = torch.zeros(1, dtype=torch.int32, device=dev)
         with torch.cuda.stream(stream):  # (the scratch belongs to the launch stream)
             update = torch.empty(max(1, d.update_size), dtype=torch.float64, device=dev)
-            d.factor(self.val.data_ptr(), self._factor, update, self._band_bad, _s(stream))
+            d.factor(self.val.data_ptr(), self._factor, update, self._band_bad, _s(stream),
+                     f=None if b is None else b.data_ptr())
         self._factored = True
 
     def direct_solve(self, b, x, stream=None):
-        """x = K^-1 b with the factor of :meth:`factor_direct`."""
-        self._direct_plan().solve(self._factor, b.data_ptr(), x.data_ptr(), self._direct_work,
-                                  _s(stream))
+        """x = K^-1 b with the factor of :meth:`factor_direct` (b None: the
+        right-hand side given there)."""
+        self._direct_plan().solve(self._factor, None if b is None else b.data_ptr(),
+                                  x.data_ptr(), self._direct_work, _s(stream))
         return x
 
     def setup_amg(self, xyz, log=None, precisions=('fp64',), graph=True, **kw):
@@ -260,8 +263,10 @@ class StaticSystem:
             return u, info
         elif method == 'direct':
             if refactor or not getattr(self, '_factored', False):
-                self.factor_direct(stream=stream)
-            self.direct_solve(b, x, stream=stream)
+                self.factor_direct(stream=stream, b=b)
+                self.direct_solve(None, x, stream=stream)
+            else:
+                self.direct_solve(b, x, stream=stream)
             if int(self._band_bad.item()):
                 raise _lib.Pf3dError('the factorisation met a non-positive pivot')
             info = dict(iters=0, outer=0)

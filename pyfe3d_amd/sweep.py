@@ -32,9 +32,13 @@ from .sparse import BlockPlan
 # LDS panel width of the narrow factorisation shape: 74 KB of LDS, so two
 # workgroups share a CU (the 448-wide panel takes one CU each)
 NARROW_PANEL = 256
-# the sweep is solved by nested dissection when its widest band (DOFs)
-# exceeds this, else by the banded kernels
-BANDED_MAX = 96
+# widest band (DOFs) of the sweeps for which the banded kernels with a tuned
+# launch shape are kept; wider ones, and all without a tuned shape, are solved
+# by nested dissection.  4,096 plates of 12 x 12 elements (band 89): 11.4 ms
+# banded and tuned, 13.6 ms by dissection, 22.8 ms banded with the default
+# shape; 512 of 24 x 24 (band 161): 8.0, 8.1 and 12.2 ms; 512 of 8 to 64
+# elements a side: 72.3, 19.9 and 72.6 ms
+BANDED_MAX = 160
 
 
 def split_order(bandwidths, sizes, narrow=NARROW_PANEL):
@@ -327,22 +331,22 @@ class PlateSweep:
     def _dissection(self):
         """The sweep's nested-dissection plan and buffers, or None where the
         banded kernels are used."""
+        dims = np.array(self.dims)
+        bw = 6 * (dims.min(axis=1) + 2) + 5
+        if bw.max() <= BANDED_MAX and getattr(self, 'direct_config', None):
+            return None
         if not hasattr(self, '_batch'):
-            dims = np.array(self.dims)
-            bw = 6 * (dims.min(axis=1) + 2) + 5
             maxb = _lib.call('pf3d_band_max_width')
             if bw.max() > maxb:
                 raise ValueError('plate too wide for the direct solver (bandwidth %d > %d)'
                                  % (bw.max(), maxb))
-            self._batch = None
-            if bw.max() > BANDED_MAX:
-                from .direct import DirectBatch
-                ny = np.repeat(dims[:, 1] + 1, np.diff(self.node0))
-                local = np.arange(self.n_nodes) - np.repeat(self.node0[:-1], np.diff(self.node0))
-                coord = np.stack([local // ny, local % ny], axis=1)  # PlateMesh: i * ny + j
-                self._batch = DirectBatch(self.plan.row_ptr.cpu().numpy(),
-                                          self.plan.col_idx.cpu().numpy(), self.device,
-                                          self.node0, coord)
+            from .direct import DirectBatch
+            ny = np.repeat(dims[:, 1] + 1, np.diff(self.node0))
+            local = np.arange(self.n_nodes) - np.repeat(self.node0[:-1], np.diff(self.node0))
+            coord = np.stack([local // ny, local % ny], axis=1)  # PlateMesh: i * ny + j
+            self._batch = DirectBatch(self.plan.row_ptr.cpu().numpy(),
+                                      self.plan.col_idx.cpu().numpy(), self.device, self.node0,
+                                      coord)
         return self._batch
 
     def solve_direct(self, rtol=1e-8, polish_iter=0, config=None, stream=None):
@@ -351,10 +355,9 @@ class PlateSweep:
         polish_iter > 0, block-Jacobi PCG from the direct solution for any
         variant that misses rtol).
 
-        Without config: nested dissection (pyfe3d_amd.direct) for sweeps with
-        a band wider than BANDED_MAX, else the banded kernels with the launch
-        shape chosen by :meth:`autotune_direct`, else (1024, 576, 1024).
-        config: the banded kernels with (factor threads, panel bandwidth,
+        Without config: nested dissection (pyfe3d_amd.direct), or, for sweeps
+        of bands up to BANDED_MAX whose launch shape :meth:`autotune_direct`
+        has chosen, the banded kernels with that shape.  config: the banded kernels with (factor threads, panel bandwidth,
         solve threads[, narrow-band factor threads]): banded Cholesky of every
         variant (one workgroup each) with the forward substitution fused into
         it, then the backward substitution."""

@@ -172,6 +172,11 @@ def test_dissection_against_dense(name, leaf):
         plan.solve(factor, tb.data_ptr(), x.data_ptr(), work, s)
         ref = np.linalg.solve(A, b)
         err = np.linalg.norm(x.cpu().numpy() - ref) / np.linalg.norm(ref)
+        # the same right-hand side carried through the factorisation
+        y, factor2 = new(n), new(plan.factor_size)
+        plan.factor(tv.data_ptr(), factor2, update, bad, s, f=tb.data_ptr())
+        plan.solve(factor2, None, y.data_ptr(), work, s)
+        err = max(err, np.linalg.norm(y.cpu().numpy() - ref) / np.linalg.norm(ref))
         print(name, leaf, 'err %.2e, %d fronts, widest %d' % (err, plan.n_fronts, plan.widest))
         assert err <= 1e-12
     assert int(bad.item()) == 0
