@@ -582,7 +582,12 @@ __device__ __forceinline__ double block_sum(double v, double *sh)
 // state of one solve, in device memory
 struct PcgState {
     double rz, rz_old, pq, alpha, beta, rr, bb, pad;
+    double rzs[2];  // r.z by parity of the iteration (pcg_direction)
 };
+
+// a / b, 0 where b is 0: an iteration on a residual that has become exactly
+// zero inside a batch (a single block row, an exact start) changes nothing
+__device__ __forceinline__ double ratio(double a, double b) { return b != 0. ? a / b : 0.; }
 
 // partial[k][blk] for up to 2 dot products, grid-strided over n
 template <typename T>
@@ -605,7 +610,8 @@ __global__ void __launch_bounds__(VB) dot2(int64_t n, const T *__restrict__ a,
 }
 
 // single-workgroup finisher: mode 0: pq -> alpha; mode 1: rz, rr -> beta;
-// mode 2: init (rz, rr) ; mode 3: bb ; mode 4: rr from the first sum
+// mode 2: init (rz, rr) ; mode 3: bb ; mode 4: rr from the first sum ;
+// mode 5: rr
 __global__ void __launch_bounds__(VB) finish(int nparts, const double *__restrict__ partial,
                                              PcgState *st, int mode)
 {
@@ -620,17 +626,19 @@ __global__ void __launch_bounds__(VB) finish(int nparts, const double *__restric
     if (threadIdx.x) return;
     if (mode == 0) {
         st->pq = s0;
-        st->alpha = st->rz / s0;
+        st->alpha = ratio(st->rz, s0);
     } else if (mode == 1) {
         st->rz_old = st->rz;
         st->rz = s0;
         st->rr = s1;
-        st->beta = s0 / st->rz_old;
+        st->beta = ratio(s0, st->rz_old);
     } else if (mode == 2) {
         st->rz = s0;
         st->rr = s1;
     } else if (mode == 3) {
         st->bb = s0;
+    } else if (mode == 5) {
+        st->rr = s1;
     } else {
         st->rr = s0;
     }
@@ -723,6 +731,227 @@ inline unsigned red_blocks(int64_t n)
     return (unsigned)(b < RED_BLOCKS ? (b < 1 ? 1 : b) : RED_BLOCKS);
 }
 
+// ------------------------------------------- PCG iteration in two launches
+// An iteration was six dependent launches of 2-6 us (product, p.q, its
+// finish, update, its finish, direction), and on small systems nothing but
+// their latency.  Two kernels remain, each starting with the scalar that the
+// other left as partial sums: every workgroup adds those few partials
+// itself, in the order of `finish`, while its first loads are in flight.
+//   pcg_direction: beta, p = z + beta p, q = A p.  Neighbours' entries of the
+//     new p are formed where they are read; each row stores its own into the
+//     other of two p buffers.
+//   pcg_update: p.q, alpha, x, r, z = Dinv r, partials of (r.z, r.r).
+// 20 x 20 plate: 24.2 -> 13.7 us per iteration (4.3 and 6.3 us in the
+// kernels); recording the iterations in a graph gave 13.4.  Above PQ_MAX
+// entries p.q comes from dot2 in between; up to it every workgroup forms it
+// (40 x 40 plate, 10,086 entries: 18.1 us against 16.8).  Above FUSED_MAX the
+// separate kernels stay: reading z and p of every neighbour costs a
+// bandwidth-bound product more than the launches (100 x 100 plate 31.2 ->
+// 23.3 us, but 200 x 200 46 -> 50 and 500 x 500 208 -> 295).  All sums in the
+// order of the separate kernels: the same bits.
+constexpr int64_t PQ_MAX = 8192, FUSED_MAX = 131072;
+constexpr int UT = 768;  // pcg_update: 6 threads per row, 2 x 128 rows
+
+// sum of a 256-entry block in block_sum's order, entry l, l + 64, l + 128 and
+// l + 192 given by lane l; the result in lane 0
+__device__ __forceinline__ double tree256(double e0, double e1, double e2, double e3)
+{
+    double v = (e0 + e2) + (e1 + e3);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+    return v;
+}
+
+// block_sum over threads 0 .. 255 of a larger workgroup, to all threads; sh
+// has 257 doubles
+__device__ __forceinline__ double sum256(double v, double *sh)
+{
+    const int t = threadIdx.x;
+    if (t < 256) sh[t] = v;
+    __syncthreads();
+    if (t < 64) {
+        const double s = tree256(sh[t], sh[t + 64], sh[t + 128], sh[t + 192]);
+        if (t == 0) sh[256] = s;
+    }
+    __syncthreads();
+    return sh[256];
+}
+
+// two sums at once, wave 0 the first and wave 1 the second; to thread 0
+__device__ __forceinline__ void sum256_pair(double &a, double &b, double *sha, double *shb)
+{
+    const int t = threadIdx.x;
+    if (t < 256) {
+        sha[t] = a;
+        shb[t] = b;
+    }
+    __syncthreads();
+    if (t < 128) {
+        double *sh = t < 64 ? sha : shb;
+        const int l = t & 63;
+        const double s = tree256(sh[l], sh[l + 64], sh[l + 128], sh[l + 192]);
+        if (l == 0) sh[256] = s;
+    }
+    __syncthreads();
+    a = sha[256];
+    b = shb[256];
+}
+
+template <typename MT>
+__global__ void __launch_bounds__(256)
+    pcg_direction(int64_t nb, const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
+                  const MT *__restrict__ val, const double *__restrict__ z,
+                  const double *__restrict__ pold, double *__restrict__ pnew,
+                  double *__restrict__ y, const double *__restrict__ partial, int nparts,
+                  PcgState *st, int par, int first)
+{
+    __shared__ double part[4][64];
+    __shared__ double sh[257];
+    // one block row per wave, lanes as in bsr_spmv
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * 4 + wave;
+    const int j = lane / 6, i = lane - 6 * (lane / 6);
+    const bool ok = row < nb && j < 10;
+    int b = ok ? rp[row] + j : 0;
+    const int b1 = ok ? rp[row + 1] : 0;
+    double acc = 0., m[6], zv[6], pv[6];
+    auto load = [&]() {
+        const MT *v = val + (int64_t)b * 36 + i * 6;
+        const int64_t c = (int64_t)ci[b] * 6;
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            m[k] = (double)v[k];
+            zv[k] = z[c + k];
+            pv[k] = first ? 0. : pold[c + k];
+        }
+    };
+    if (b < b1) load();
+    const bool own = row < nb && lane < 6;
+    const double zo = own ? z[row * 6 + lane] : 0.;
+    const double po = own && !first ? pold[row * 6 + lane] : 0.;
+    double beta = 0.;
+    if (first) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->rzs[par] = st->rz;
+    } else {
+        const double old = st->rzs[par ^ 1];
+        double s = 0.;
+        for (int k = threadIdx.x; k < nparts; k += 256) s += partial[k];
+        s = sum256(s, sh);
+        beta = ratio(s, old);
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->rzs[par] = s;
+    }
+    if (own) pnew[row * 6 + lane] = first ? zo : zo + beta * po;
+    while (b < b1) {
+#pragma unroll
+        for (int k = 0; k < 6; k++) acc += m[k] * (first ? zv[k] : zv[k] + beta * pv[k]);
+        b += 10;
+        if (b < b1) load();
+    }
+    part[wave][lane] = acc;
+    __syncthreads();
+    if (own) {
+        double s = 0.;
+#pragma unroll
+        for (int jj = 0; jj < 10; jj++) s += part[wave][lane + 6 * jj];
+        y[row * 6 + lane] = s;
+    }
+}
+
+// x += alpha p ; r -= alpha q ; z = Dinv r ; partial (r.z, r.r) of 256-row
+// blocks in update_xrz's order.  Thread (row, component): a row's threads
+// share its r through LDS, threads 0 .. 255 keep the sums of one row slot.
+template <typename MT, bool OWN_PQ>
+__global__ void __launch_bounds__(UT)
+    pcg_update(int64_t nb, PcgState *st, int par, const double *__restrict__ pqpart, int npq,
+               double *__restrict__ x, double *__restrict__ r, const double *__restrict__ p,
+               const double *__restrict__ q, const MT *__restrict__ dinv, double *__restrict__ z,
+               double *__restrict__ partial)
+{
+    __shared__ double sh[257], rs[UT], ss[2][UT], rr[2][UT];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int slot = tid / 6, comp = tid - 6 * slot;
+    const int64_t n = nb * 6;
+    double xv[2], pv[2], rv[2], qv[2], d[2][6];
+    auto load = [&](int64_t base) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int64_t row = base + 128 * h + slot;
+            if (row >= nb) continue;
+            const int64_t t = row * 6 + comp;
+            xv[h] = x[t];
+            pv[h] = p[t];
+            rv[h] = r[t];
+            qv[h] = q[t];
+#pragma unroll
+            for (int k = 0; k < 6; k++) d[h][k] = (double)dinv[row * 36 + comp * 6 + k];
+        }
+    };
+    load((int64_t)blockIdx.x * 256);
+    double s = 0.;
+    if (OWN_PQ) {
+        // p.q: wave w takes 256-entry blocks w, w + 12, ... (dot2's blocks)
+        const int nd = (int)((n + 255) / 256);
+        for (int k = wave; k < nd; k += UT / 64) {
+            double e[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int64_t t = (int64_t)k * 256 + 64 * c + lane;
+                e[c] = t < n ? p[t] * q[t] : 0.;
+            }
+            const double v = tree256(e[0], e[1], e[2], e[3]);
+            if (lane == 0) rs[k] = v;
+        }
+        __syncthreads();
+        s = tid < nd ? rs[tid] : 0.;
+    } else if (tid < 256) {
+        for (int k = tid; k < npq; k += 256) s += pqpart[k];
+    }
+    s = sum256(s, sh);
+    const double alpha = ratio(st->rzs[par], s);
+    double s0 = 0., s1 = 0.;  // (threads 0 .. 255: row slot tid)
+    for (int64_t base = (int64_t)blockIdx.x * 256; base < nb; base += (int64_t)gridDim.x * 256) {
+        if (base != (int64_t)blockIdx.x * 256) load(base);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int64_t row = base + 128 * h + slot;
+            __syncthreads();
+            double rn = 0.;
+            if (row < nb) {
+                const int64_t t = row * 6 + comp;
+                x[t] = xv[h] + alpha * pv[h];
+                rn = rv[h] - alpha * qv[h];
+                r[t] = rn;
+                rs[tid] = rn;
+            }
+            __syncthreads();
+            if (row < nb) {
+                double a = 0.;
+#pragma unroll
+                for (int k = 0; k < 6; k++) a += d[h][k] * rs[6 * slot + k];
+                z[row * 6 + comp] = a;
+                ss[h][tid] = a;
+                rr[h][tid] = rn;
+            }
+        }
+        __syncthreads();
+        if (tid < 256 && base + tid < nb) {
+            const int h = tid >> 7, at = 6 * (tid & 127);
+#pragma unroll
+            for (int k = 0; k < 6; k++) {
+                const double a = ss[h][at + k], b = rr[h][at + k];
+                s0 += a * b;
+                s1 += b * b;
+            }
+        }
+        __syncthreads();
+    }
+    sum256_pair(s0, s1, sh, &ss[0][0]);
+    if (tid == 0) {
+        partial[blockIdx.x] = s0;
+        partial[RED_BLOCKS + blockIdx.x] = s1;
+    }
+}
+
 // ------------------------------------------------------------- PCG driver
 struct Mat {
     int64_t nb;
@@ -738,39 +967,40 @@ hipError_t spmv(const Mat &A, const VT *x, VT *y, hipStream_t s)
     return hipGetLastError();
 }
 
-// workspace: 4 vectors of T (r, z, p, q), partials, state
+// workspace: 5 vectors of T (r, z, p, q, second p), partials of p.q and of
+// (r.z, r.r), state
 size_t pcg_bytes(int64_t n, size_t tsize)
 {
-    return ((4 * n * tsize + 255) / 256) * 256 + 2 * RED_BLOCKS * sizeof(double) + 256;
+    return ((5 * n * tsize + 255) / 256) * 256 + 4 * RED_BLOCKS * sizeof(double) + 256;
 }
 
 // Solve A x = b to ||r|| <= rtol ||b|| (recursive residual), starting from
 // the true residual of x (x0 != 0) or from x = 0.  Matrix and block-Jacobi
-// inverse are stored as MT, vectors as VT.
-template <typename MT, typename VT>
-int pcg_run(const Mat &A, const VT *b, VT *x, double rtol, int maxiter, int x0, void *work,
+// inverse are stored as MT, vectors as FP64.
+template <typename MT>
+int pcg_run(const Mat &A, const double *b, double *x, double rtol, int maxiter, int x0, void *work,
             hipStream_t s, int64_t *iters, double *relres, int check_every)
 {
     const int64_t n = A.nb * 6;
     char *w = (char *)work;
-    VT *r = (VT *)w, *z = r + n, *p = z + n, *q = p + n;
-    double *partial = (double *)(w + ((4 * n * sizeof(VT) + 255) / 256) * 256);
-    PcgState *st = (PcgState *)(partial + 2 * RED_BLOCKS);
+    double *r = (double *)w, *z = r + n, *p = z + n, *q = p + n, *p2 = q + n;
+    double *partial = (double *)(w + ((5 * n * sizeof(double) + 255) / 256) * 256);
+    double *pqpart = partial + 2 * RED_BLOCKS;
+    PcgState *st = (PcgState *)(partial + 4 * RED_BLOCKS);
     const unsigned nv = nblk(n, VB), nr = red_blocks(A.nb), nd = red_blocks(n);
+    const double *null = nullptr;
     hipError_t e;
-    hipLaunchKernelGGL(dot2<VT>, dim3(nd), dim3(VB), 0, s, n, b, b, (const VT *)nullptr,
-                       (const VT *)nullptr, partial);
+    hipLaunchKernelGGL(dot2<double>, dim3(nd), dim3(VB), 0, s, n, b, b, null, null, partial);
     hipLaunchKernelGGL(finish, dim3(1), dim3(VB), 0, s, (int)nd, partial, st, 3);
-    if (!x0) hipLaunchKernelGGL(fill0<VT>, dim3(nv), dim3(VB), 0, s, n, x);
-    if ((e = spmv<MT, VT>(A, x, q, s)) != hipSuccess) return pf3d_hip_check(e, "pcg spmv");
+    if (!x0) hipLaunchKernelGGL(fill0<double>, dim3(nv), dim3(VB), 0, s, n, x);
+    if ((e = spmv<MT, double>(A, x, q, s)) != hipSuccess) return pf3d_hip_check(e, "pcg spmv");
     // r = b - A x ; z = M r ; (r.z, r.r) through the update kernel with p = 0
-    hipLaunchKernelGGL(fill0<VT>, dim3(nv), dim3(VB), 0, s, n, p);
-    hipMemcpyAsync(r, b, sizeof(VT) * n, hipMemcpyDeviceToDevice, s);
+    hipLaunchKernelGGL(fill0<double>, dim3(nv), dim3(VB), 0, s, n, p);
+    hipMemcpyAsync(r, b, sizeof(double) * n, hipMemcpyDeviceToDevice, s);
     hipLaunchKernelGGL(set_alpha, dim3(1), dim3(1), 0, s, st, 1.);
-    hipLaunchKernelGGL((update_xrz<MT, VT>), dim3(nr), dim3(VB), 0, s, A.nb, st, x, r, p, q,
+    hipLaunchKernelGGL((update_xrz<MT, double>), dim3(nr), dim3(VB), 0, s, A.nb, st, x, r, p, q,
                        (const MT *)A.dinv, z, partial);
     hipLaunchKernelGGL(finish, dim3(1), dim3(VB), 0, s, (int)nr, partial, st, 2);
-    hipMemcpyAsync(p, z, sizeof(VT) * n, hipMemcpyDeviceToDevice, s);
     PcgState h;
     e = hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -778,17 +1008,38 @@ int pcg_run(const Mat &A, const VT *b, VT *x, double rtol, int maxiter, int x0, 
     const double bb = h.bb > 0 ? h.bb : 1.;
     double rel = sqrt(h.rr / bb);
     int it = 0;
+    const MT *val = (const MT *)A.val, *dinv = (const MT *)A.dinv;
+    const unsigned gd = nblk(A.nb, 4);
+    if (n > FUSED_MAX) hipMemcpyAsync(p, z, sizeof(double) * n, hipMemcpyDeviceToDevice, s);
     while (rel > rtol && it < maxiter) {
         for (int k = 0; k < check_every && it < maxiter; k++, it++) {
-            spmv<MT, VT>(A, p, q, s);
-            hipLaunchKernelGGL(dot2<VT>, dim3(nd), dim3(VB), 0, s, n, p, q, (const VT *)nullptr,
-                               (const VT *)nullptr, partial);
-            hipLaunchKernelGGL(finish, dim3(1), dim3(VB), 0, s, (int)nd, partial, st, 0);
-            hipLaunchKernelGGL((update_xrz<MT, VT>), dim3(nr), dim3(VB), 0, s, A.nb, st, x, r,
-                               p, q, (const MT *)A.dinv, z, partial);
-            hipLaunchKernelGGL(finish, dim3(1), dim3(VB), 0, s, (int)nr, partial, st, 1);
-            hipLaunchKernelGGL(update_p<VT>, dim3(nv), dim3(VB), 0, s, n, st, z, p);
+            const int par = it & 1;
+            const double *pold = par ? p : p2;
+            double *pnew = par ? p2 : p;
+            if (n > FUSED_MAX) {
+                spmv<MT, double>(A, p, q, s);
+                hipLaunchKernelGGL(dot2<double>, dim3(nd), dim3(VB), 0, s, n, p, q, null, null,
+                                   partial);
+                hipLaunchKernelGGL(finish, dim3(1), dim3(VB), 0, s, (int)nd, partial, st, 0);
+                hipLaunchKernelGGL((update_xrz<MT, double>), dim3(nr), dim3(VB), 0, s, A.nb, st, x,
+                                   r, p, q, dinv, z, partial);
+                hipLaunchKernelGGL(finish, dim3(1), dim3(VB), 0, s, (int)nr, partial, st, 1);
+                hipLaunchKernelGGL(update_p<double>, dim3(nv), dim3(VB), 0, s, n, st, z, p);
+                continue;
+            }
+            hipLaunchKernelGGL(pcg_direction<MT>, dim3(gd), dim3(256), 0, s, A.nb, A.rp, A.ci, val,
+                               z, pold, pnew, q, partial, (int)nr, st, par, it == 0);
+            if (n <= PQ_MAX) {
+                hipLaunchKernelGGL((pcg_update<MT, true>), dim3(nr), dim3(UT), 0, s, A.nb, st, par,
+                                   pqpart, 0, x, r, pnew, q, dinv, z, partial);
+            } else {
+                hipLaunchKernelGGL(dot2<double>, dim3(nd), dim3(VB), 0, s, n, pnew, q, null, null,
+                                   pqpart);
+                hipLaunchKernelGGL((pcg_update<MT, false>), dim3(nr), dim3(UT), 0, s, A.nb, st,
+                                   par, pqpart, (int)nd, x, r, pnew, q, dinv, z, partial);
+            }
         }
+        hipLaunchKernelGGL(finish, dim3(1), dim3(VB), 0, s, (int)nr, partial, st, 5);
         e = hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) return pf3d_hip_check(e, "pcg iterate");
@@ -809,7 +1060,7 @@ int pcg64_restarted(const Mat &A, const double *b, double *x, double rtol, int64
     double rel = 0.;
     for (int restart = 0; restart < 8; restart++) {
         int64_t it = 0;
-        int st = pcg_run<double, double>(A, b, x, rtol, (int)(maxiter - total), x0 || restart,
+        int st = pcg_run<double>(A, b, x, rtol, (int)(maxiter - total), x0 || restart,
                                          work, s, &it, &rel, 25);
         if (st) return st;
         total += it;
@@ -835,8 +1086,8 @@ int pcg_mixed_run(const Mat &A64, const Mat &A32, const double *b, double *x, do
     const int64_t n = A64.nb * 6;
     char *w = (char *)work;
     double *r = (double *)w, *z = r + n, *p = z + n, *q = p + n;
-    double *partial = (double *)(w + ((4 * n * 8 + 255) / 256) * 256);
-    PcgState *st = (PcgState *)(partial + 2 * RED_BLOCKS);
+    double *partial = (double *)(w + ((5 * n * 8 + 255) / 256) * 256);
+    PcgState *st = (PcgState *)(partial + 4 * RED_BLOCKS);
     double *y = (double *)(w + pcg_bytes(n, sizeof(double)));
     const unsigned nv = nblk(n, VB), nr = red_blocks(A64.nb), nd = red_blocks(n);
     hipError_t e;
@@ -1067,7 +1318,7 @@ int pf3d_pcg(int64_t nb, const int32_t *row_ptr, const int32_t *col_idx, const d
 }
 
 /* Allocation-free FP64 PCG (pf3d_pcg without the caller's workspace):
- * the four PCG vectors, the reduction partials and the solver state live
+ * the PCG vectors, the reduction partials and the solver state live
  * in `scratch`, a file-scope device array of fixed size (one copy per GPU,
  * held until the process ends).  Its address on each device comes from
  * hipGetSymbolAddress once, with that device current; host code uses that
@@ -1077,8 +1328,8 @@ int pf3d_pcg(int64_t nb, const int32_t *row_ptr, const int32_t *col_idx, const d
 
 namespace {
 constexpr size_t PCG_STATIC_BYTES =
-    ((4 * 6 * (size_t)PF3D_PCG_STATIC_MAX_ROWS * sizeof(double) + 255) / 256) * 256 +
-    2 * RED_BLOCKS * sizeof(double) + 256;
+    ((5 * 6 * (size_t)PF3D_PCG_STATIC_MAX_ROWS * sizeof(double) + 255) / 256) * 256 +
+    4 * RED_BLOCKS * sizeof(double) + 256;
 }  // namespace
 
 static __device__ __align__(256) char scratch[PCG_STATIC_BYTES];
@@ -1191,7 +1442,7 @@ int pf3d_ir_solve(int64_t nb, const int32_t *row_ptr, const int32_t *col_idx,
         int64_t it = 0;
         double inner_rel = 0.;
         // inner solve on the FP32-stored matrix with FP64 vectors
-        int st2 = pcg_run<float, double>(A32, r64, d64, inner_rtol, max_inner, 0, inner, s, &it,
+        int st2 = pcg_run<float>(A32, r64, d64, inner_rtol, max_inner, 0, inner, s, &it,
                                          &inner_rel, 25);
         if (st2) return st2;
         inner_total += it;

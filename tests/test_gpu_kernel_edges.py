@@ -261,3 +261,42 @@ def test_direct_refuses_wide_bands_and_takes_streams():
     a.val.neg_()
     with pytest.raises(_lib.Pf3dError):
         a.solve(f, method='direct', refactor=True)
+
+
+@pytest.mark.parametrize('rows', [1, 2, 43, 127, 128, 129, 256, 257, 1365, 1366, 2731, 21846])
+@pytest.mark.parametrize('method', ['fp64', 'ir'])
+def test_pcg_routes(rows, method):
+    """Chains of 1 to 21,846 block rows: one and two row slots per thread,
+    one and several 256-row blocks, p.q formed in the update (up to 8,192
+    entries), by the separate kernel, and the separate kernels throughout
+    (above 131,072).  Diagonally dominant (condition below 100), solved to
+    1e-12: within 1e-10 of the solution the loads were made from,
+    a start at the solution needs no iteration, maxiter is kept."""
+    from types import SimpleNamespace
+    from pyfe3d_amd.solver import StaticSystem
+    rng = np.random.default_rng(rows)
+    off = rng.uniform(-1, 1, (rows, 6, 6))        # block (i, i + 1)
+    diag = rng.uniform(-1, 1, (rows, 6, 6))
+    diag = diag + diag.transpose(0, 2, 1) + 30. * np.eye(6)
+    idx = np.arange(rows)
+    r = np.concatenate([idx, idx[:-1], idx[1:]])
+    c = np.concatenate([idx, idx[1:], idx[:-1]])
+    v = np.concatenate([diag, off[:-1], off[:-1].transpose(0, 2, 1)])
+    order = np.lexsort((c, r))
+    rp = np.concatenate([[0], np.cumsum(np.bincount(r, minlength=rows))])
+    plan = SimpleNamespace(row_ptr=T(rp, torch.int32), col_idx=T(c[order], torch.int32),
+                           n_nodes=rows)
+    s = StaticSystem(plan, T(v[order].reshape(-1), torch.float64), np.zeros(6 * rows))
+    u = rng.normal(size=(rows, 6))
+    f = np.einsum('nij,nj->ni', diag, u)
+    f[:-1] += np.einsum('nij,nj->ni', off[:-1], u[1:])
+    f[1:] += np.einsum('nji,nj->ni', off[:-1], u[:-1])
+    rtol = 1e-12 if method == 'fp64' else 1e-11
+    x, info = s.solve(f.reshape(-1), method=method, rtol=rtol)
+    assert info['relres'] <= 2 * rtol and info['iters'] > 0
+    assert np.linalg.norm(x.cpu().numpy() - u.ravel()) <= 1e-10 * np.linalg.norm(u)
+    if method == 'fp64':
+        _, again = s.solve(f.reshape(-1), method=method, rtol=1e-9, x0=x)
+        assert again['iters'] == 0
+        _, few = s.solve(f.reshape(-1), method=method, rtol=1e-30, maxiter=3)
+        assert few['iters'] == 3
