@@ -724,6 +724,26 @@ int pf3d_axpby(int64_t n, double a, const double *x, double b, double *y, void *
 int pf3d_nn_gemm(int M, int N, int K, const float *A, int64_t sam, int64_t sak, const float *B,
                  int64_t sbn, int64_t sbk, float *C, int64_t ldc, int accumulate,
                  const float *bias, int relu, int splits, float *partial, void *stream);
+/* 3x3 convolution (zero padding 1, stride 1 or 2) of x (B, H, W, C) to y
+ * (B, Ho, Wo, N), its input gradient (dx (+)= ...) and its weight gradient
+ * dw (N, 9, C), without a column matrix.  Operands are rounded to bfloat16,
+ * sums are FP32.  wf and wb are the weights' bfloat16 copies [N][9][C] and
+ * [C][9][N], written by pf3d_nn_pack for up to 16 layers (host arrays of
+ * channel counts and device pointers).  Tensors 16-byte aligned;
+ * pf3d_nn_conv: C a multiple of 32, N of 4; _dx: N of 32, C of 4; _dw: both
+ * of 32, work at least N*9*C floats (more of them, more workgroups). */
+int pf3d_nn_pack(int count, const int *co, const int *ci, const float *const *w, void *const *wf,
+                 void *const *wb, void *stream);
+int pf3d_nn_conv(int B, int H, int W, int C, int stride, const float *x, const void *wf,
+                 const float *bias, int relu, int N, float *y, void *stream);
+int pf3d_nn_conv_dx(int B, int H, int W, int C, int stride, const float *dy, const void *wb,
+                    int N, float *dx, int accumulate, void *stream);
+int pf3d_nn_conv_dw(int B, int H, int W, int C, int stride, const float *x, const float *dy, int N,
+                    float *dw, float *work, int64_t work_floats, void *stream);
+/* pf3d_nn_adam on up to 32 tensors in one launch (host arrays) */
+int pf3d_nn_adam_many(int count, const int64_t *n, float *const *p, const float *const *g,
+                      float *const *m, float *const *v, float lr, float b1, float b2, float eps,
+                      int step, void *stream);
 /* 3x3 patches with zero padding 1 and stride 1 or 2, and the adjoint */
 int pf3d_nn_im2col(int B, int H, int W, int C, int stride, const float *x, float *col,
                    void *stream);

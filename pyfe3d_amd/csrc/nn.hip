@@ -201,6 +201,267 @@ __global__ void col2im3(int B, int H, int W, int C, int s, const float *__restri
     dx[t] = accumulate ? dx[t] + acc : acc;
 }
 
+// ------------------------------------------------ 3x3 convolutions, direct
+// Forward, input gradient and weight gradient without a column matrix (it
+// was 9 times the activations, written once and read two or three times).
+// Matrix-core operands come straight from memory in their register layout:
+// NHWC rows are contiguous in the channel, so that 8 consecutive channels of
+// a pixel (K) are two 16-byte loads, rounded to bfloat16 in registers; the
+// taps' reuse of a pixel is left to the caches.  Weights are rounded once per
+// pass (nn_pack).  Channels of the contracted side must be a multiple of 32.
+
+// 8 floats -> bfloat16 (round to nearest even)
+__device__ __forceinline__ bf16x8 pack8(const f32x4 &a, const f32x4 &b)
+{
+    bf16x8 r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        r[i] = (__bf16)a[i];
+        r[i + 4] = (__bf16)b[i];
+    }
+    return r;
+}
+
+struct Conv {
+    int B, H, W, C, s;   // input grid, input channels, stride
+    int Ho, Wo, N;       // output grid and channels
+    const float *x;      // source of the gathered operand
+    const __bf16 *w;     // [columns][9][K channels]
+    const float *bias;
+    float *y;
+    int relu, accumulate;
+};
+
+// OUT columns (output channels of the forward pass, input channels of the
+// gradient) of 16 R pixels per wave, 32 columns per workgroup in y.  The
+// pixels' operand is the second one, so a lane ends with 4 consecutive
+// columns of a pixel: one 16-byte store.
+//   forward:  row = output pixel, source x at (oy s - 1 + ky, ...)
+//   gradient: row = input pixel,  source dy; with stride 2 the launch's z is
+//   the pixel's parity class, whose pixels share the taps that reach them
+template <int R, bool GRAD>
+__global__ void __launch_bounds__(256) conv3(Conv c, int64_t M)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = lane & 15, k8 = 8 * (lane >> 4);
+    const int K = GRAD ? c.N : c.C, cols = GRAD ? c.C : c.N;
+    const int Hs = GRAD ? c.Ho : c.H, Ws = GRAD ? c.Wo : c.W;  // source grid
+    const int py = blockIdx.z >> 1, px = blockIdx.z & 1;
+    // rows of this part: output pixels, input pixels, or one parity class
+    const bool cls = GRAD && c.s == 2;
+    const int Hr = !GRAD ? c.Ho : cls ? (c.H - py + 1) / 2 : c.H;
+    const int Wr = !GRAD ? c.Wo : cls ? (c.W - px + 1) / 2 : c.W;
+    const int64_t rows = (int64_t)c.B * Hr * Wr;
+    const int64_t m0 = ((int64_t)blockIdx.x * 4 + wave) * 16 * R;
+    if (m0 >= rows) return;
+    const int n0 = blockIdx.y * 32;
+    int iy[R], ix[R];
+    const float *src[R];
+    int64_t out[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int64_t m = min(m0 + 16 * r + li, rows - 1);
+        const int64_t q = m / Wr;
+        const int x = (int)(m - q * Wr), b = (int)(q / Hr), y = (int)(q - (int64_t)b * Hr);
+        iy[r] = GRAD ? y : y * c.s - 1;
+        ix[r] = GRAD ? x : x * c.s - 1;
+        src[r] = c.x + (int64_t)b * Hs * Ws * K + k8;
+        out[r] = cls ? ((int64_t)b * c.H + 2 * y + py) * c.W + 2 * x + px : m;
+    }
+    f32x4 acc[R][2];
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int t = 0; t < 2; t++) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const __bf16 *wp[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) wp[t] = c.w + (int64_t)min(n0 + 16 * t + li, cols - 1) * 9 * K + k8;
+    for (int ky = 0; ky < 3; ky++) {
+        if (cls && ((ky & 1) == py)) continue;  // tap parity: row 2 i + py reads ky = 1 - py (mod 2)
+        const int oy = GRAD ? (cls ? (py + 1 - ky) / 2 : 1 - ky) : ky;
+        for (int kx = 0; kx < 3; kx++) {
+            if (cls && ((kx & 1) == px)) continue;
+            const int ox = GRAD ? (cls ? (px + 1 - kx) / 2 : 1 - kx) : kx;
+            const int tap = 3 * ky + kx;
+            const float *p[R];
+            bool in[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const int y = iy[r] + oy, x = ix[r] + ox;
+                in[r] = y >= 0 && y < Hs && x >= 0 && x < Ws;
+                p[r] = src[r] + ((int64_t)(in[r] ? y : 0) * Ws + (in[r] ? x : 0)) * K;
+            }
+#pragma unroll 2
+            for (int k = 0; k < K; k += 32) {
+                bf16x8 a[2], b[R];
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+                    a[t] = *reinterpret_cast<const bf16x8 *>(wp[t] + tap * K + k);
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    f32x4 u = *reinterpret_cast<const f32x4 *>(p[r] + k);
+                    f32x4 v = *reinterpret_cast<const f32x4 *>(p[r] + k + 4);
+                    if (!in[r]) u = v = f32x4{0.f, 0.f, 0.f, 0.f};
+                    b[r] = pack8(u, v);
+                }
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+                        acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b[r], acc[r][t],
+                                                                             0, 0, 0);
+            }
+        }
+    }
+    // lane: columns n0 + 16 t + 4 (lane / 16) + 0..3 of pixel li
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (m0 + 16 * r + li >= rows) continue;
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int n = n0 + 16 * t + 4 * (lane >> 4);
+            if (n >= cols) continue;
+            f32x4 *o = reinterpret_cast<f32x4 *>(c.y + out[r] * cols + n);
+            f32x4 v = acc[r][t];
+            if (c.bias) v += *reinterpret_cast<const f32x4 *>(c.bias + n);
+            if (c.accumulate) v += *o;
+            if (c.relu)
+#pragma unroll
+                for (int q = 0; q < 4; q++) v[q] = v[q] < 0.f ? 0.f : v[q];
+            *o = v;
+        }
+    }
+}
+
+// dW[co][tap][ci] = sum over output pixels of dy[pixel][co] x[source][ci].
+// A workgroup takes 32 co x 32 ci x the three taps of one kernel row, its
+// four waves a quarter of the pixels of its split each (added in wave order
+// through LDS); a lane's operand is one channel of 8 consecutive pixels.
+// The splits' sums go to part[split][co][9 ci] and are added in order.
+__global__ void __launch_bounds__(256)
+    conv3_dw(Conv c, const float *__restrict__ dy, int64_t M, int64_t chunk,
+             float *__restrict__ part)
+{
+    __shared__ float red[3][12][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = lane & 15, k8 = 8 * (lane >> 4);
+    const int nci = c.C / 32;
+    const int ky = blockIdx.x % 3, tile = blockIdx.x / 3;
+    const int co0 = 32 * (tile / nci), ci0 = 32 * (tile % nci);
+    f32x4 acc[3][2][2];
+#pragma unroll
+    for (int t = 0; t < 3; t++)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) acc[t][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int64_t beg = ((int64_t)blockIdx.y * 4 + wave) * chunk;
+    const int64_t end = min(M, beg + chunk);
+    for (int64_t m0 = beg; m0 < end; m0 += 32) {
+        // this lane's 8 pixels, outside ones contribute zero
+        const int64_t m = m0 + k8;
+        const int64_t q = m / c.Wo;
+        int ox = (int)(m - q * c.Wo), b = (int)(q / c.Ho), oy = (int)(q - (int64_t)b * c.Ho);
+        bf16x8 a[2], xv[3][2];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const bool on = m + e < end;
+            const float *d = dy + (on ? m + e : 0) * c.N + co0 + li;
+            const int y = oy * c.s + ky - 1;
+            const bool yin = on && y >= 0 && y < c.H;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const float v = d[16 * i];
+                a[i][e] = (__bf16)(on ? v : 0.f);
+            }
+#pragma unroll
+            for (int t = 0; t < 3; t++) {
+                const int x = ox * c.s + t - 1;
+                const bool in = yin && x >= 0 && x < c.W;
+                const float *p = c.x + (in ? (((int64_t)b * c.H + y) * c.W + x) * c.C : 0) + ci0 + li;
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const float v = p[16 * j];
+                    xv[t][j][e] = (__bf16)(in ? v : 0.f);
+                }
+            }
+            if (++ox == c.Wo) {
+                ox = 0;
+                if (++oy == c.Ho) {
+                    oy = 0;
+                    b++;
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 3; t++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    acc[t][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], xv[t][j],
+                                                                             acc[t][i][j], 0, 0, 0);
+    }
+    if (wave)
+#pragma unroll
+        for (int t = 0; t < 12; t++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                red[wave - 1][t][e][lane] = acc[t / 4][(t >> 1) & 1][t & 1][e];
+    __syncthreads();
+    if (wave) return;
+    float *o = part + (int64_t)blockIdx.y * c.N * 9 * c.C;
+#pragma unroll
+    for (int t = 0; t < 12; t++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            float v = acc[t / 4][(t >> 1) & 1][t & 1][e];
+            for (int w = 0; w < 3; w++) v += red[w][t][e][lane];
+            // D: row (co) 4 (lane / 16) + e, column (ci) lane % 16
+            const int co = co0 + 16 * ((t >> 1) & 1) + 4 * (lane >> 4) + e;
+            const int ci = ci0 + 16 * (t & 1) + li;
+            o[((int64_t)co * 9 + 3 * ky + t / 4) * c.C + ci] = v;
+        }
+}
+
+// out[t] = sum of part[z][t] over the splits, 4 threads per entry (splits
+// z = 0, 4, .. and so on, added in order)
+__global__ void __launch_bounds__(256)
+    dw_sum(int64_t n, int splits, const float *__restrict__ part, float *__restrict__ out)
+{
+    __shared__ float sh[4][64];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t t = (int64_t)blockIdx.x * 64 + l;
+    float v = 0.f;
+    if (t < n)
+        for (int z = w; z < splits; z += 4) v += part[z * n + t];
+    sh[w][l] = v;
+    __syncthreads();
+    if (w == 0 && t < n) out[t] = ((sh[0][l] + sh[1][l]) + sh[2][l]) + sh[3][l];
+}
+
+// bfloat16 copies of the weights w[co][9][ci], as they are and with input
+// and output channels exchanged ([ci][9][co]), several layers per launch
+constexpr int MAX_PACK = 16;
+struct Pack {
+    int count;
+    int co[MAX_PACK], ci[MAX_PACK];
+    const float *w[MAX_PACK];
+    __bf16 *a[MAX_PACK], *b[MAX_PACK];
+};
+
+__global__ void __launch_bounds__(256) nn_pack(Pack p)
+{
+    const int l = blockIdx.y, co = p.co[l], ci = p.ci[l];
+    const int64_t n = (int64_t)co * 9 * ci;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
+        const int c = (int)(t % ci), q = (int)(t / ci), tap = q % 9, o = q / 9;
+        const __bf16 v = (__bf16)p.w[l][t];
+        p.a[l][t] = v;
+        p.b[l][((int64_t)c * 9 + tap) * co + o] = v;
+    }
+}
+
 // dy <- dy * (y > 0)
 __global__ void relu_bwd(int64_t n, const float *__restrict__ y, float *__restrict__ dy)
 {
@@ -433,7 +694,59 @@ __global__ void adam_step(int64_t n, float *__restrict__ p, const float *__restr
     p[t] -= lr * (mt / c1) / (sqrtf(vt / c2) + eps);
 }
 
+// the same update on several tensors in one launch
+constexpr int MAX_TENSORS = 32;
+struct Tensors {
+    int64_t n[MAX_TENSORS];
+    float *p[MAX_TENSORS], *m[MAX_TENSORS], *v[MAX_TENSORS];
+    const float *g[MAX_TENSORS];
+};
+
+__global__ void __launch_bounds__(256)
+    adam_many(Tensors a, float lr, float b1, float b2, float eps, float c1, float c2)
+{
+    const int k = blockIdx.y;
+    float *p = a.p[k], *m = a.m[k], *v = a.v[k];
+    const float *g = a.g[k];
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < a.n[k];
+         t += (int64_t)gridDim.x * 256) {
+        const float gt = g[t];
+        const float mt = b1 * m[t] + (1.f - b1) * gt;
+        const float vt = b2 * v[t] + (1.f - b2) * gt * gt;
+        m[t] = mt;
+        v[t] = vt;
+        p[t] -= lr * (mt / c1) / (sqrtf(vt / c2) + eps);
+    }
+}
+
 inline unsigned nb256(int64_t n) { return (unsigned)((n + 255) / 256); }
+
+bool conv_ok(int B, int H, int W, int C, int stride, int N)
+{
+    return B > 0 && H > 0 && W > 0 && (stride == 1 || stride == 2) && C > 0 && N > 0;
+}
+
+Conv conv_of(int B, int H, int W, int C, int stride, int N)
+{
+    Conv c{};
+    c.B = B; c.H = H; c.W = W; c.C = C; c.s = stride; c.N = N;
+    c.Ho = (H - 1) / stride + 1;
+    c.Wo = (W - 1) / stride + 1;
+    return c;
+}
+
+// 32 pixels per wave where that still gives some 16 waves per CU, else 16
+template <bool GRAD>
+void launch_conv(const Conv &c, int64_t rows, int cols, int parts, hipStream_t s)
+{
+    const unsigned gy = (cols + 31) / 32;
+    if (rows * gy * parts >= 131072)
+        hipLaunchKernelGGL((conv3<2, GRAD>), dim3((unsigned)((rows + 127) / 128), gy, parts),
+                           dim3(256), 0, s, c, rows);
+    else
+        hipLaunchKernelGGL((conv3<1, GRAD>), dim3((unsigned)((rows + 63) / 64), gy, parts),
+                           dim3(256), 0, s, c, rows);
+}
 
 }  // namespace
 
@@ -484,6 +797,99 @@ int pf3d_nn_col2im(int B, int H, int W, int C, int stride, const float *dcol, fl
     hipLaunchKernelGGL(col2im3, dim3(nb256(n)), dim3(256), 0, (hipStream_t)stream, B, H, W, C,
                        stride, dcol, dx, accumulate);
     return pf3d_hip_check(hipGetLastError(), "pf3d_nn_col2im");
+}
+
+int pf3d_nn_pack(int count, const int *co, const int *ci, const float *const *w, void *const *wf,
+                 void *const *wb, void *stream)
+{
+    if (count < 1 || count > MAX_PACK || !co || !ci || !w || !wf || !wb)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nn_pack: bad arguments");
+    Pack p{};
+    p.count = count;
+    int64_t most = 0;
+    for (int l = 0; l < count; l++) {
+        if (co[l] <= 0 || ci[l] <= 0 || !w[l] || !wf[l] || !wb[l])
+            return pf3d_fail(PF3D_E_ARG, "pf3d_nn_pack: bad layer %d", l);
+        p.co[l] = co[l];
+        p.ci[l] = ci[l];
+        p.w[l] = w[l];
+        p.a[l] = (__bf16 *)wf[l];
+        p.b[l] = (__bf16 *)wb[l];
+        const int64_t n = (int64_t)co[l] * 9 * ci[l];
+        most = n > most ? n : most;
+    }
+    const unsigned gx = nb256(most) < 256 ? nb256(most) : 256;
+    hipLaunchKernelGGL(nn_pack, dim3(gx, count), dim3(256), 0, (hipStream_t)stream, p);
+    return pf3d_hip_check(hipGetLastError(), "pf3d_nn_pack");
+}
+
+int pf3d_nn_conv(int B, int H, int W, int C, int stride, const float *x, const void *wf,
+                 const float *bias, int relu, int N, float *y, void *stream)
+{
+    if (!conv_ok(B, H, W, C, stride, N) || C % 32 || N % 4 || !x || !wf || !y)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nn_conv: bad arguments");
+    Conv c = conv_of(B, H, W, C, stride, N);
+    c.x = x; c.w = (const __bf16 *)wf; c.bias = bias; c.relu = relu; c.y = y;
+    launch_conv<false>(c, (int64_t)B * c.Ho * c.Wo, N, 1, (hipStream_t)stream);
+    return pf3d_hip_check(hipGetLastError(), "pf3d_nn_conv");
+}
+
+int pf3d_nn_conv_dx(int B, int H, int W, int C, int stride, const float *dy, const void *wb,
+                    int N, float *dx, int accumulate, void *stream)
+{
+    if (!conv_ok(B, H, W, C, stride, N) || N % 32 || C % 4 || !dy || !wb || !dx)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nn_conv_dx: bad arguments");
+    Conv c = conv_of(B, H, W, C, stride, N);
+    c.x = dy; c.w = (const __bf16 *)wb; c.y = dx; c.accumulate = accumulate;
+    // (stride 2: one part per parity class, the largest sizes the grid)
+    const int64_t rows = stride == 2 ? (int64_t)B * ((H + 1) / 2) * ((W + 1) / 2) : (int64_t)B * H * W;
+    launch_conv<true>(c, rows, C, stride == 2 ? 4 : 1, (hipStream_t)stream);
+    return pf3d_hip_check(hipGetLastError(), "pf3d_nn_conv_dx");
+}
+
+int pf3d_nn_conv_dw(int B, int H, int W, int C, int stride, const float *x, const float *dy, int N,
+                    float *dw, float *work, int64_t work_floats, void *stream)
+{
+    if (!conv_ok(B, H, W, C, stride, N) || C % 32 || N % 32 || !x || !dy || !dw || !work)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nn_conv_dw: bad arguments");
+    Conv c = conv_of(B, H, W, C, stride, N);
+    c.x = x;
+    const int64_t M = (int64_t)B * c.Ho * c.Wo, n = (int64_t)N * 9 * C;
+    const int tiles = 3 * (N / 32) * (C / 32);
+    // some 12 waves per CU, at least one 32-pixel step per wave
+    int64_t splits = (768 + tiles - 1) / tiles;
+    if (splits > (M + 127) / 128) splits = (M + 127) / 128;
+    if (splits > work_floats / n) splits = work_floats / n;
+    if (splits < 1) return pf3d_fail(PF3D_E_ARG, "pf3d_nn_conv_dw: work must hold N * 9 * C floats");
+    int64_t chunk = (M + 4 * splits - 1) / (4 * splits);
+    chunk = (chunk + 31) / 32 * 32;
+    hipStream_t s = (hipStream_t)stream;
+    hipLaunchKernelGGL(conv3_dw, dim3(tiles, (unsigned)splits), dim3(256), 0, s, c, dy, M, chunk,
+                       work);
+    hipLaunchKernelGGL(dw_sum, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, n, (int)splits,
+                       work, dw);
+    return pf3d_hip_check(hipGetLastError(), "pf3d_nn_conv_dw");
+}
+
+int pf3d_nn_adam_many(int count, const int64_t *n, float *const *p, const float *const *g,
+                      float *const *m, float *const *v, float lr, float b1, float b2, float eps,
+                      int step, void *stream)
+{
+    if (count < 1 || count > MAX_TENSORS || !n || !p || !g || !m || !v || step < 1)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nn_adam_many: bad arguments");
+    Tensors a{};
+    int64_t most = 0;
+    for (int k = 0; k < count; k++) {
+        if (n[k] <= 0 || !p[k] || !g[k] || !m[k] || !v[k])
+            return pf3d_fail(PF3D_E_ARG, "pf3d_nn_adam_many: bad tensor %d", k);
+        a.n[k] = n[k]; a.p[k] = p[k]; a.g[k] = g[k]; a.m[k] = m[k]; a.v[k] = v[k];
+        most = n[k] > most ? n[k] : most;
+    }
+    const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
+    const unsigned gx = nb256(most) < 256 ? nb256(most) : 256;
+    hipLaunchKernelGGL(adam_many, dim3(gx, count), dim3(256), 0, (hipStream_t)stream, a, lr, b1,
+                       b2, eps, c1, c2);
+    return pf3d_hip_check(hipGetLastError(), "pf3d_nn_adam_many");
 }
 
 int pf3d_nn_relu_bwd(int64_t n, const float *y, float *dy, void *stream)

@@ -10,11 +10,13 @@ x0; a plate whose alpha is not positive starts from zero.  The solve
 itself, and its FP64 residual criterion, are unchanged: the network can only
 change how many iterations are needed.
 
-Everything runs through the library's own HIP kernels (im2col / col2im,
-bfloat16 GEMM on the matrix cores with FP32 accumulation, up-sampling,
+Everything runs through the library's own HIP kernels (direct 3x3
+convolutions and a bfloat16 GEMM on the matrix cores with FP32 accumulation, up-sampling,
 losses and Adam); torch only holds the buffers.  Training data are solves
 of the plain GPU solver (:mod:`pyfe3d_amd.sweep`).
 """
+import ctypes
+
 import numpy as np
 import torch
 
@@ -35,6 +37,9 @@ LAYERS = [
     ('head', 32, 6, 1, 1, False),
 ]
 SPEC = {l[0]: l[1:] for l in LAYERS}
+# 3x3 layers whose channels fill the matrix cores' K: direct convolutions; the
+# first layer (2 channels) goes through its patches, the head is a product
+DIRECT = [l[0] for l in LAYERS if l[4] == 3 and l[1] % 32 == 0 and l[2] % 32 == 0]
 
 
 def _s(stream):
@@ -65,6 +70,10 @@ class WarmStartNet:
             self.m[k] = torch.zeros_like(t)
             self.v[k] = torch.zeros_like(t)
         self.step_count = 0
+        # bfloat16 weights of the direct layers, [co][9][ci] and [ci][9][co]
+        half = lambda t: torch.empty(t.numel(), dtype=torch.bfloat16, device=self.dev)
+        self.wf = {k: half(self.p[k + '.w']) for k in DIRECT}
+        self.wb = {k: half(self.p[k + '.w']) for k in DIRECT}
         self._alloc(batch)
 
     # ------------------------------------------------------------ buffers
@@ -80,20 +89,15 @@ class WarmStartNet:
         n = self.n
         self.B = B
         self.act, self.col = {}, {}
-        self.dcol_size = 0
         for name, ci, co, s, k, _ in LAYERS:
             hi, ho = self._shape(name)
             self.act[name] = torch.empty((B, ho, ho, co), **f)
-            if k == 3:
+            if k == 3 and name not in DIRECT:
                 self.col[name] = torch.empty((B * ho * ho, 9 * ci), **f)
-                self.dcol_size = max(self.dcol_size, B * ho * ho * 9 * ci)
-            else:
-                self.dcol_size = max(self.dcol_size, B * ho * ho * ci)
         self.z = {3: torch.empty((B, n // 4, n // 4, 128), **f),
                   2: torch.empty((B, n // 2, n // 2, 64), **f),
                   1: torch.empty((B, n, n, 32), **f)}
         self.u = torch.empty((B, n + 1, n + 1, 6), **f)
-        self.dcol = torch.empty(self.dcol_size, **f)
         # gradients of activations (same shapes), split-K partials
         self.dact = {k: torch.empty_like(t) for k, t in self.act.items()}
         self.dz = {k: torch.empty_like(t) for k, t in self.z.items()}
@@ -108,11 +112,24 @@ class WarmStartNet:
                   C.data_ptr(), ldc, acc, None if bias is None else bias.data_ptr(), relu,
                   splits, self.partial.data_ptr() if splits > 1 else None, _s(stream))
 
+    def _pack(self, stream=None):
+        """bfloat16 copies of the direct layers' weights (one launch)."""
+        n = len(DIRECT)
+        ptrs = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])
+        _lib.call('pf3d_nn_pack', n, (ctypes.c_int * n)(*[SPEC[k][1] for k in DIRECT]),
+                  (ctypes.c_int * n)(*[SPEC[k][0] for k in DIRECT]),
+                  ptrs([self.p[k + '.w'] for k in DIRECT]), ptrs([self.wf[k] for k in DIRECT]),
+                  ptrs([self.wb[k] for k in DIRECT]), _s(stream))
+
     def _conv(self, name, x, stream=None):
         ci, co, s, k, relu = SPEC[name]
         B = self.B
         hi, ho = self._shape(name)
         y = self.act[name]
+        if name in DIRECT:
+            _lib.call('pf3d_nn_conv', B, hi, hi, ci, s, x.data_ptr(), self.wf[name].data_ptr(),
+                      self.p[name + '.b'].data_ptr(), int(relu), co, y.data_ptr(), _s(stream))
+            return y
         M = B * ho * ho
         if k == 3:
             col = self.col[name]
@@ -137,21 +154,23 @@ class WarmStartNet:
         st = _s(stream)
         if relu:
             _lib.call('pf3d_nn_relu_bwd', dy.numel(), y.data_ptr(), dy.data_ptr(), st)
-        col = self.col[name] if k == 3 else x
-        # dW[co][Kd] = sum_m dy[m][co] col[m][Kd]  (split-K over the pixels)
-        self._gemm(co, Kd, M, dy, 1, co, col, 1, Kd, self.g[name + '.w'], Kd,
-                   splits=min(self.splits, max(1, M // 256)), stream=stream)
+        if name in DIRECT:
+            _lib.call('pf3d_nn_conv_dw', B, hi, hi, ci, s, x.data_ptr(), dy.data_ptr(), co,
+                      self.g[name + '.w'].data_ptr(), self.partial.data_ptr(),
+                      self.partial.numel(), st)
+        else:
+            col = self.col[name] if k == 3 else x
+            # dW[co][Kd] = sum_m dy[m][co] col[m][Kd]  (split-K over the pixels)
+            self._gemm(co, Kd, M, dy, 1, co, col, 1, Kd, self.g[name + '.w'], Kd,
+                       splits=min(self.splits, max(1, M // 256)), stream=stream)
         _lib.call('pf3d_nn_bias_grad', M, co, dy.data_ptr(), self.g[name + '.b'].data_ptr(),
                   self.partial.data_ptr(), self.partial.numel(), st)
         if dx is None:
             return
-        if k == 3:
-            dcol = self.dcol[:M * Kd]
-            self._gemm(M, Kd, co, dy, co, 1, self.p[name + '.w'], 1, Kd, dcol, Kd,
-                       stream=stream)
-            _lib.call('pf3d_nn_col2im', B, hi, hi, ci, s, dcol.data_ptr(), dx.data_ptr(),
-                      int(dx_acc), st)
-        else:
+        if name in DIRECT:
+            _lib.call('pf3d_nn_conv_dx', B, hi, hi, ci, s, dy.data_ptr(),
+                      self.wb[name].data_ptr(), co, dx.data_ptr(), int(dx_acc), st)
+        else:  # (the head; the first layer has no input gradient)
             self._gemm(M, Kd, co, dy, co, 1, self.p[name + '.w'], 1, Kd, dx, Kd,
                        acc=int(dx_acc), stream=stream)
 
@@ -163,6 +182,7 @@ class WarmStartNet:
         x = x.contiguous()
         self._x = x
         n, B, st = self.n, self.B, _s(stream)
+        self._pack(stream)
         a0 = self._conv('c0', x, stream)
         a1 = self._conv('c1', a0, stream)
         a2 = self._conv('d1', a1, stream)
@@ -224,6 +244,7 @@ class WarmStartNet:
         n, B, st = self.n, self.B, _s(stream)
         de = self.dact['head']
         A, D = self.act, self.dact
+        self._pack(stream)  # (the parameters may have changed since forward)
         self._conv_bwd('head', A['u1'], de, D['u1'], stream=stream)
         self._conv_bwd('u1', self.z[1], D['u1'], self.dz[1], stream=stream)
         # z1 = up(a6) + a1
@@ -245,10 +266,11 @@ class WarmStartNet:
 
     def adam(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, stream=None):
         self.step_count += 1
-        for k, p in self.p.items():
-            _lib.call('pf3d_nn_adam', p.numel(), p.data_ptr(), self.g[k].data_ptr(),
-                      self.m[k].data_ptr(), self.v[k].data_ptr(), lr, b1, b2, eps,
-                      self.step_count, _s(stream))
+        n = len(self.p)
+        ptrs = lambda d: (ctypes.c_void_p * n)(*[d[k].data_ptr() for k in self.p])
+        _lib.call('pf3d_nn_adam_many', n, (ctypes.c_int64 * n)(*[p.numel() for p in self.p.values()]),
+                  ptrs(self.p), ptrs(self.g), ptrs(self.m), ptrs(self.v), lr, b1, b2, eps,
+                  self.step_count, _s(stream))
 
     def gemm_flops(self):
         """(forward, backward) floating-point operations of the matrix-core

@@ -300,3 +300,71 @@ def test_pcg_routes(rows, method):
         assert again['iters'] == 0
         _, few = s.solve(f.reshape(-1), method=method, rtol=1e-30, maxiter=3)
         assert few['iters'] == 3
+
+
+def _bf16(a):
+    return torch.as_tensor(a, dtype=torch.float32).to(torch.bfloat16).to(torch.float64)
+
+
+@pytest.mark.parametrize('B, H, W, C, N, stride', [
+    (1, 1, 1, 32, 32, 1), (1, 1, 1, 32, 64, 2), (2, 3, 5, 64, 32, 1), (3, 8, 8, 32, 96, 2),
+    (1, 7, 9, 96, 32, 2), (2, 16, 15, 32, 32, 1), (1, 33, 31, 64, 64, 2), (5, 2, 70, 32, 32, 2),
+    (40, 64, 64, 32, 32, 1), (2, 64, 64, 32, 64, 2)])
+def test_direct_convolutions(B, H, W, C, N, stride):
+    """3x3 convolution, input and weight gradients against float64 sums of
+    the same bfloat16 operands: 1 to 163,840 pixels (16 and 32 per wave), odd
+    grids (uneven parity classes), rows shorter than a lane's 8 pixels,
+    several channel tiles, one and many splits.  A sum of K products in FP32
+    is within K eps of the sum of their magnitudes; the order adds at most
+    another K."""
+    from pyfe3d_amd import _lib
+    import ctypes
+    rng = np.random.default_rng(H * W + C)
+    Ho, Wo = (H - 1) // stride + 1, (W - 1) // stride + 1
+    f32 = lambda *s: torch.as_tensor(rng.normal(size=s), dtype=torch.float32)
+    x, w, b, dy, dx0 = (f32(B, H, W, C), f32(N, 9, C), f32(N), f32(B, Ho, Wo, N),
+                        f32(B, H, W, C))
+    dev = lambda t: t.to(DEV).contiguous()
+    xd, wd, bd, dyd = dev(x), dev(w), dev(b), dev(dy)
+    wf = torch.empty(N * 9 * C, dtype=torch.bfloat16, device=DEV)
+    wb = torch.empty_like(wf)
+    st = torch.cuda.current_stream().cuda_stream
+    one = lambda t: (ctypes.c_void_p * 1)(t.data_ptr())
+    _lib.call('pf3d_nn_pack', 1, (ctypes.c_int * 1)(N), (ctypes.c_int * 1)(C), one(wd), one(wf),
+              one(wb), st)
+    y = torch.full((B, Ho, Wo, N), float('nan'), device=DEV)
+    _lib.call('pf3d_nn_conv', B, H, W, C, stride, xd.data_ptr(), wf.data_ptr(), bd.data_ptr(), 1,
+              N, y.data_ptr(), st)
+    dx = dev(dx0)
+    _lib.call('pf3d_nn_conv_dx', B, H, W, C, stride, dyd.data_ptr(), wb.data_ptr(), N,
+              dx.data_ptr(), 1, st)
+    n = N * 9 * C
+    eps = 2. ** -23
+    F = torch.nn.functional
+    nchw = lambda t: t.permute(0, 3, 1, 2)
+    wk = lambda t: t.reshape(N, 3, 3, C).permute(0, 3, 1, 2)
+
+    def both(fn, *ops):  # value and sum of magnitudes
+        return fn(*ops), fn(*[o.abs() for o in ops])
+
+    xb, wbf, dyb = _bf16(x), _bf16(w), _bf16(dy)
+    ref, mag = both(lambda p, q: F.conv2d(nchw(p), wk(q), stride=stride, padding=1), xb, wbf)
+    got = nchw(y.cpu().double())
+    tol = 2 * 9 * C * eps * (mag + b.abs().double()[None, :, None, None])
+    assert ((got - (ref + b.double()[None, :, None, None]).clamp(min=0)).abs() <= tol).all()
+    ref, mag = both(lambda p, q: torch.nn.grad.conv2d_input((B, C, H, W), wk(q), nchw(p),
+                                                            stride=stride, padding=1), dyb, wbf)
+    tol = 2 * 9 * N * eps * (mag + nchw(dx0).abs().double())
+    assert ((nchw(dx.cpu().double()) - (ref + nchw(dx0).double())).abs() <= tol).all()
+    ref, mag = both(lambda p, q: torch.nn.grad.conv2d_weight(nchw(p), (N, C, 3, 3), nchw(q),
+                                                             stride=stride, padding=1), xb, dyb)
+    K = B * Ho * Wo
+    for floats in (n, 3 * n, 1000 * n):
+        if floats * 4 > 1 << 30:
+            continue
+        dw = torch.full((N, 9, C), float('nan'), device=DEV)
+        work = torch.full((floats,), float('nan'), device=DEV)
+        _lib.call('pf3d_nn_conv_dw', B, H, W, C, stride, xd.data_ptr(), dyd.data_ptr(), N,
+                  dw.data_ptr(), work.data_ptr(), floats, st)
+        got = wk(dw.cpu().double())
+        assert ((got - ref).abs() <= 2 * K * eps * mag).all(), floats
