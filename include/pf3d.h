@@ -719,7 +719,7 @@ int pf3d_axpby(int64_t n, double a, const double *x, double b, double *y, void *
 /* ------------------------------------------------------------------ */
 
 /* C[m*ldc + n] (+)= sum_k A[m*sam + k*sak] B[n*sbn + k*sbk] (+ bias[n],
- * ReLU).  splits > 1 divides K into slices summed in slice order through
+ * ReLU).  splits > 1 divides K into slices summed in a fixed order through
  * partial (splits*M*N floats). */
 int pf3d_nn_gemm(int M, int N, int K, const float *A, int64_t sam, int64_t sak, const float *B,
                  int64_t sbn, int64_t sbk, float *C, int64_t ldc, int accumulate,
@@ -740,6 +740,10 @@ int pf3d_nn_conv_dx(int B, int H, int W, int C, int stride, const float *dy, con
                     int N, float *dx, int accumulate, void *stream);
 int pf3d_nn_conv_dw(int B, int H, int W, int C, int stride, const float *x, const float *dy, int N,
                     float *dw, float *work, int64_t work_floats, void *stream);
+/* dy <- dy * (y > 0) (y NULL: dy as it is) and db[c] = sum_rows dy[row][c]
+ * (C <= 256) in one pass; work as for pf3d_nn_bias_grad */
+int pf3d_nn_relu_bias_grad(int64_t rows, int C, const float *y, float *dy, float *db, float *work,
+                           int64_t work_floats, void *stream);
 /* pf3d_nn_adam on up to 32 tensors in one launch (host arrays) */
 int pf3d_nn_adam_many(int count, const int64_t *n, float *const *p, const float *const *g,
                       float *const *m, float *const *v, float lr, float b1, float b2, float eps,

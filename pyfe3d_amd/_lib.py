@@ -113,6 +113,7 @@ SIGNATURES = {
     'pf3d_nn_conv': [I32, I32, I32, I32, I32, P, P, P, I32, I32, P, P],
     'pf3d_nn_conv_dx': [I32, I32, I32, I32, I32, P, P, I32, P, I32, P],
     'pf3d_nn_conv_dw': [I32, I32, I32, I32, I32, P, P, I32, P, P, I64, P],
+    'pf3d_nn_relu_bias_grad': [I64, I32, P, P, P, P, I64, P],
     'pf3d_nn_adam_many': [I32, P, P, P, P, P, F32, F32, F32, F32, I32, P],
     'pf3d_nn_relu_bwd': [I64, P, P, P],
     'pf3d_nn_bias_grad': [I64, I32, P, P, P, I64, P],

@@ -135,17 +135,41 @@ __global__ void __launch_bounds__(256) gemm_bf16(Gemm g)
             }
 }
 
-// C = sum over the split-K slices in slice order (+ C, bias, ReLU)
-__global__ void splitk_reduce(Gemm g, int splits)
+// Sum of part[z * n + t] over the splits z: ZL threads per entry take every
+// ZL-th split in order, their sums are added in order.  To the ZL == 0
+// lanes.
+template <int ZL>
+__device__ __forceinline__ float split_sum(int64_t n, int splits, const float *__restrict__ part,
+                                           int64_t t, float *sh)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)g.M * g.N) return;
-    const int m = (int)(t / g.N), n = (int)(t - (int64_t)m * g.N);
+    constexpr int PB = 256 / ZL;
+    const int l = threadIdx.x % PB, w = threadIdx.x / PB;
     float v = 0.f;
-    for (int z = 0; z < splits; z++) v += g.partial[(int64_t)z * g.M * g.N + t];
-    float *c = g.C + (int64_t)m * g.ldc + n;
+    if (t < n)
+#pragma unroll 8
+        for (int z = w; z < splits; z += ZL) v += part[z * n + t];
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    if (w) return 0.f;
+    float r = sh[l];
+#pragma unroll
+    for (int k = 1; k < ZL; k++) r += sh[k * PB + l];
+    return r;
+}
+
+// C = sum over the split-K slices (+ C, bias, ReLU)
+template <int ZL>
+__global__ void __launch_bounds__(256) splitk_reduce(Gemm g, int splits)
+{
+    __shared__ float sh[256];
+    const int64_t n = (int64_t)g.M * g.N;
+    const int64_t t = (int64_t)blockIdx.x * (256 / ZL) + threadIdx.x % (256 / ZL);
+    float v = split_sum<ZL>(n, splits, g.partial, t, sh);
+    if (threadIdx.x >= 256 / ZL || t >= n) return;
+    const int m = (int)(t / g.N), c0 = (int)(t - (int64_t)m * g.N);
+    float *c = g.C + (int64_t)m * g.ldc + c0;
     if (g.accumulate) v += *c;
-    if (g.bias) v += g.bias[n];
+    if (g.bias) v += g.bias[c0];
     if (g.relu && v < 0.f) v = 0.f;
     *c = v;
 }
@@ -424,20 +448,15 @@ __global__ void __launch_bounds__(256)
         }
 }
 
-// out[t] = sum of part[z][t] over the splits, 4 threads per entry (splits
-// z = 0, 4, .. and so on, added in order)
+// out[t] = sum of part[z][t] over the splits
+template <int ZL>
 __global__ void __launch_bounds__(256)
     dw_sum(int64_t n, int splits, const float *__restrict__ part, float *__restrict__ out)
 {
-    __shared__ float sh[4][64];
-    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t t = (int64_t)blockIdx.x * 64 + l;
-    float v = 0.f;
-    if (t < n)
-        for (int z = w; z < splits; z += 4) v += part[z * n + t];
-    sh[w][l] = v;
-    __syncthreads();
-    if (w == 0 && t < n) out[t] = ((sh[0][l] + sh[1][l]) + sh[2][l]) + sh[3][l];
+    __shared__ float sh[256];
+    const int64_t t = (int64_t)blockIdx.x * (256 / ZL) + threadIdx.x % (256 / ZL);
+    const float v = split_sum<ZL>(n, splits, part, t, sh);
+    if (threadIdx.x < 256 / ZL && t < n) out[t] = v;
 }
 
 // bfloat16 copies of the weights w[co][9][ci], as they are and with input
@@ -489,6 +508,49 @@ __global__ void __launch_bounds__(256) bias_part(int64_t rows, int C, int64_t ch
     __syncthreads();
     if (q == 0 && c < C)
         part[(int64_t)blockIdx.x * C + c] = red[0][cl] + red[1][cl] + red[2][cl] + red[3][cl];
+}
+
+// The same partial sums with the ReLU mask of the layer's output y (null:
+// none) applied to dy on the way, in one pass over dy.  Threads (row lane,
+// V channels): every lane has work at any channel count up to 256 V, and the
+// row lanes' sums are added in order.
+template <int V>
+__global__ void __launch_bounds__(256) relu_bias_part(int64_t rows, int C, int64_t chunk,
+                                                      const float *__restrict__ y,
+                                                      float *__restrict__ dy,
+                                                      float *__restrict__ part)
+{
+    using vec = float __attribute__((ext_vector_type(V)));
+    __shared__ float red[256 * V];
+    const int tpr = C / V, rl = 256 / tpr;
+    const int q = threadIdx.x / tpr, c = threadIdx.x - q * tpr;
+    const int64_t r0 = (int64_t)blockIdx.x * chunk;
+    const int64_t r1 = r0 + chunk < rows ? r0 + chunk : rows;
+    float s[V];
+#pragma unroll
+    for (int k = 0; k < V; k++) s[k] = 0.f;
+    if (q < rl)
+#pragma unroll 4
+        for (int64_t r = r0 + q; r < r1; r += rl) {
+            vec *p = reinterpret_cast<vec *>(dy + r * C) + c;
+            vec d = *p;
+            if (y) {
+                const vec a = *(reinterpret_cast<const vec *>(y + r * C) + c);
+#pragma unroll
+                for (int k = 0; k < V; k++) d[k] = a[k] > 0.f ? d[k] : 0.f;
+                *p = d;
+            }
+#pragma unroll
+            for (int k = 0; k < V; k++) s[k] += d[k];
+        }
+#pragma unroll
+    for (int k = 0; k < V; k++) red[threadIdx.x * V + k] = s[k];
+    __syncthreads();
+    for (int t = threadIdx.x; t < C; t += 256) {
+        float v = 0.f;
+        for (int k = 0; k < rl; k++) v += red[k * C + t];
+        part[(int64_t)blockIdx.x * C + t] = v;
+    }
 }
 
 // one wave per channel: lane l adds chunks l, l + 64, ... in order, then a
@@ -772,7 +834,8 @@ int pf3d_nn_gemm(int M, int N, int K, const float *A, int64_t sam, int64_t sak, 
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL(gemm_bf16, grid, dim3(256), 0, s, g);
     if (z > 1)
-        hipLaunchKernelGGL(splitk_reduce, dim3(nb256((int64_t)M * N)), dim3(256), 0, s, g, z);
+        hipLaunchKernelGGL(splitk_reduce<16>, dim3(nb256((int64_t)M * N * 16)), dim3(256), 0, s, g,
+                           z);
     return pf3d_hip_check(hipGetLastError(), "pf3d_nn_gemm");
 }
 
@@ -866,8 +929,13 @@ int pf3d_nn_conv_dw(int B, int H, int W, int C, int stride, const float *x, cons
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL(conv3_dw, dim3(tiles, (unsigned)splits), dim3(256), 0, s, c, dy, M, chunk,
                        work);
-    hipLaunchKernelGGL(dw_sum, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, s, n, (int)splits,
-                       work, dw);
+    // (more threads per entry where few entries have many splits)
+    if (splits >= 64)
+        hipLaunchKernelGGL(dw_sum<16>, dim3(nb256(n * 16)), dim3(256), 0, s, n, (int)splits, work,
+                           dw);
+    else
+        hipLaunchKernelGGL(dw_sum<4>, dim3(nb256(n * 4)), dim3(256), 0, s, n, (int)splits, work,
+                           dw);
     return pf3d_hip_check(hipGetLastError(), "pf3d_nn_conv_dw");
 }
 
@@ -918,6 +986,29 @@ int pf3d_nn_bias_grad(int64_t rows, int C, const float *dy, float *db, float *wo
                        chunk, dy, work);
     hipLaunchKernelGGL(bias_sum, dim3((C + 3) / 4), dim3(256), 0, s, (int)nchunk, C, work, db);
     return pf3d_hip_check(hipGetLastError(), "pf3d_nn_bias_grad");
+}
+
+int pf3d_nn_relu_bias_grad(int64_t rows, int C, const float *y, float *dy, float *db, float *work,
+                           int64_t work_floats, void *stream)
+{
+    if (rows <= 0 || C <= 0 || C > 256 || !dy || !db || !work || work_floats < C)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_nn_relu_bias_grad: bad arguments");
+    // chunks of >= 128 rows, at most 1024 of them, as many as the work holds
+    int64_t nchunk = (rows + 127) / 128;
+    if (nchunk > 1024) nchunk = 1024;
+    if (nchunk > work_floats / C) nchunk = work_floats / C;
+    const int64_t chunk = (rows + nchunk - 1) / nchunk;
+    nchunk = (rows + chunk - 1) / chunk;
+    hipStream_t s = (hipStream_t)stream;
+    const uintptr_t al = (uintptr_t)y | (uintptr_t)dy;
+    if (C % 4 == 0 && (al & 15) == 0)
+        hipLaunchKernelGGL(relu_bias_part<4>, dim3((unsigned)nchunk), dim3(256), 0, s, rows, C,
+                           chunk, y, dy, work);
+    else
+        hipLaunchKernelGGL(relu_bias_part<1>, dim3((unsigned)nchunk), dim3(256), 0, s, rows, C,
+                           chunk, y, dy, work);
+    hipLaunchKernelGGL(bias_sum, dim3((C + 3) / 4), dim3(256), 0, s, (int)nchunk, C, work, db);
+    return pf3d_hip_check(hipGetLastError(), "pf3d_nn_relu_bias_grad");
 }
 
 int pf3d_nn_up2_add(int B, int H, int W, int C, const float *lo, const float *skip, float *y,

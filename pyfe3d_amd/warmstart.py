@@ -152,19 +152,20 @@ class WarmStartNet:
         Kd = k * k * ci
         y = self.act[name]
         st = _s(stream)
-        if relu:
-            _lib.call('pf3d_nn_relu_bwd', dy.numel(), y.data_ptr(), dy.data_ptr(), st)
+        _lib.call('pf3d_nn_relu_bias_grad', M, co, y.data_ptr() if relu else None, dy.data_ptr(),
+                  self.g[name + '.b'].data_ptr(), self.partial.data_ptr(), self.partial.numel(),
+                  st)
         if name in DIRECT:
             _lib.call('pf3d_nn_conv_dw', B, hi, hi, ci, s, x.data_ptr(), dy.data_ptr(), co,
                       self.g[name + '.w'].data_ptr(), self.partial.data_ptr(),
                       self.partial.numel(), st)
         else:
             col = self.col[name] if k == 3 else x
-            # dW[co][Kd] = sum_m dy[m][co] col[m][Kd]  (split-K over the pixels)
+            # dW[co][Kd] = sum_m dy[m][co] col[m][Kd]: one output tile, so the
+            # pixels are split over as many workgroups as keep the GPU busy
+            # (131,072 pixels in 64 slices took 300 us, in 1,024 of them 20)
             self._gemm(co, Kd, M, dy, 1, co, col, 1, Kd, self.g[name + '.w'], Kd,
-                       splits=min(self.splits, max(1, M // 256)), stream=stream)
-        _lib.call('pf3d_nn_bias_grad', M, co, dy.data_ptr(), self.g[name + '.b'].data_ptr(),
-                  self.partial.data_ptr(), self.partial.numel(), st)
+                       splits=max(1, min(1024, M // 128)), stream=stream)
         if dx is None:
             return
         if name in DIRECT:

@@ -368,3 +368,44 @@ def test_direct_convolutions(B, H, W, C, N, stride):
                   dw.data_ptr(), work.data_ptr(), floats, st)
         got = wk(dw.cpu().double())
         assert ((got - ref).abs() <= 2 * K * eps * mag).all(), floats
+
+
+@pytest.mark.parametrize('rows, C', [(1, 1), (1, 6), (41, 6), (43, 6), (129, 32), (1000, 128),
+                                     (131072, 32), (5, 256), (300, 37), (2500, 3)])
+@pytest.mark.parametrize('masked', [True, False])
+def test_relu_bias_gradient(rows, C, masked):
+    """Mask and column sums for 1 to 256 channels (a multiple of 4 or not,
+    dividing 256 or not), less and more rows than row lanes, one and many
+    chunks; dy changed only by the mask.  Sums of n FP32 terms: n eps."""
+    from pyfe3d_amd import _lib
+    rng = np.random.default_rng(rows + C)
+    dy, y = (rng.normal(size=(rows, C)).astype(np.float32) for _ in range(2))
+    y[rng.random((rows, C)) < 0.1] = 0.
+    want = np.where(y > 0, dy, 0.) if masked else dy
+    for floats in (C, 4 * C, 1024 * C):
+        d, db = T(dy, torch.float32), torch.full((C,), float('nan'), device=DEV)
+        work = torch.empty(floats, device=DEV)
+        ty = T(y, torch.float32)
+        _lib.call('pf3d_nn_relu_bias_grad', rows, C, ty.data_ptr() if masked else None,
+                  d.data_ptr(), db.data_ptr(), work.data_ptr(), floats,
+                  torch.cuda.current_stream().cuda_stream)
+        assert (d.cpu().numpy() == want).all()
+        tol = rows * 2. ** -23 * np.abs(want.astype(np.float64)).sum(axis=0)
+        assert (np.abs(db.cpu().numpy() - want.astype(np.float64).sum(axis=0)) <= tol).all()
+
+
+@pytest.mark.parametrize('splits', [2, 15, 16, 17, 300, 1024])
+def test_split_products(splits):
+    """Thin products divided into many slices (one output tile, slices of
+    32 to 131,072 / splits terms) against float64 on the same operands."""
+    from pyfe3d_amd import _lib
+    rng = np.random.default_rng(splits)
+    K, M, N = 131072 if splits > 64 else 4096, 32, 18
+    a, b = _bf16(rng.normal(size=(K, M))), _bf16(rng.normal(size=(K, N)))
+    ta, tb = T(a.numpy(), torch.float32), T(b.numpy(), torch.float32)
+    c = torch.full((M, N), 2., device=DEV)
+    part = torch.full((splits * M * N,), float('nan'), device=DEV)
+    _lib.call('pf3d_nn_gemm', M, N, K, ta.data_ptr(), 1, M, tb.data_ptr(), 1, N, c.data_ptr(), N,
+              1, None, 0, splits, part.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    tol = 2. ** -23 * K * (a.abs().T @ b.abs()).numpy()
+    assert (np.abs(c.cpu().numpy() - (a.T @ b).numpy() - 2.) <= tol).all()
