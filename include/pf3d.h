@@ -431,6 +431,19 @@ int pf3d_cg_update_xr(int64_t n, const double *s, const double *p, const double 
 int pf3d_cg_beta(double *s, int flexible, void *stream);
 int pf3d_cg_update_p(int64_t n, const double *s, const double *z, double *p, void *stream);
 
+/* The same iteration in fewer launches: the dot products stay partial sums
+ * (part: 3 * 1024 doubles) that the kernel needing them adds.  s[7] holds
+ * r.z before the first step; pf3d_cg_step_xr forms p.q, alpha and updates x
+ * and r (s[0] = s[7]); pf3d_cg_dots forms the partials of a.b, a.a and a.c
+ * (c may be NULL); pf3d_cg_step_p takes those of r.z, r.r and r.z_old, sets
+ * s[7], s[4] = beta and s[5] = r.r and updates p. */
+int pf3d_cg_dots(int64_t n, const double *a, const double *b, const double *c, double *part,
+                 void *stream);
+int pf3d_cg_step_xr(int64_t n, double *s, double *part, const double *p, const double *q,
+                    double *x, double *r, void *stream);
+int pf3d_cg_step_p(int64_t n, double *s, const double *part, int flexible, const double *z,
+                   double *p, void *stream);
+
 /* Fused multigrid vector step over the nb block rows of a 6x6 BSR matrix
  * A (no reference counterpart): q = A xin (xin NULL: q = 0),
  * r = sa * (b ? b : r) + sb * q, then dnew = c1 * Dinv r + c2 * dold (when
@@ -446,6 +459,18 @@ int pf3d_bsr_fused_f32(int64_t nb, const int32_t *row_ptr, const int32_t *col_id
                        const float *val, const float *xin, const float *b, float *r,
                        const float *dinv, const float *dold, float *dnew, float *xacc, double sa,
                        double sb, double c1, double c2, void *stream);
+
+/* pf3d_bsr_fused with a choice for xacc: xmode & 1 starts it from zero
+ * instead of its values, xmode & 2 adds dnew as well (after dold).
+ * sa == 0 reads neither b nor r. */
+int pf3d_bsr_smooth(int64_t nb, const int32_t *row_ptr, const int32_t *col_idx, const double *val,
+                    const double *xin, const double *b, double *r, const double *dinv,
+                    const double *dold, double *dnew, double *xacc, double sa, double sb,
+                    double c1, double c2, int xmode, void *stream);
+int pf3d_bsr_smooth_f32(int64_t nb, const int32_t *row_ptr, const int32_t *col_idx,
+                        const float *val, const float *xin, const float *b, float *r,
+                        const float *dinv, const float *dold, float *dnew, float *xacc, double sa,
+                        double sb, double c1, double c2, int xmode, void *stream);
 
 /* pf3d_bsr_fused for nv <= 8 vectors at once, vector v of xin at offset
  * v * ldx and of every other vector operand at v * ld (ld >= 6 nb; the

@@ -64,6 +64,11 @@ SIGNATURES = {
                           P],
     'pf3d_bsr_fused_mv_f32': [I64, P, P, P, I32, I64, P, I64, P, P, P, P, P, P, F64, F64, F64,
                               F64, P],
+    'pf3d_bsr_smooth': [I64, P, P, P, P, P, P, P, P, P, P, F64, F64, F64, F64, I32, P],
+    'pf3d_bsr_smooth_f32': [I64, P, P, P, P, P, P, P, P, P, P, F64, F64, F64, F64, I32, P],
+    'pf3d_cg_dots': [I64, P, P, P, P, P],
+    'pf3d_cg_step_xr': [I64, P, P, P, P, P, P, P],
+    'pf3d_cg_step_p': [I64, P, P, I32, P, P, P],
     'pf3d_cg_update_xr': [I64, P, P, P, P, P, P],
     'pf3d_cg_beta': [P, I32, P],
     'pf3d_cg_update_p': [I64, P, P, P, P],

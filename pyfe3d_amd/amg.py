@@ -356,29 +356,37 @@ class SAAMG:
         _axpby(1., self.g_out, 0., z)
         return z
 
-    def _cheb(self, L, b, x, x_zero=False):
-        """x += Chebyshev(D^-1 A) correction for A x = b (degree k, bounds
-        [lower, 1.1] lambda_max); x_zero: x is known to be 0 (r = b, no
-        product).  Each step is one fused pass (pf3d_bsr_fused): x += d,
-        r -= A d and the next d = a D^-1 r + c d together."""
+    def _cheb_scale(self, L):
+        """(theta, delta) of the Chebyshev smoother on D^-1 A: bounds
+        [cheb_lower, 1.1] lambda_max."""
         lmax = 1.1 * L['lam']
         lmin = self.cheb_lower * L['lam']
-        theta, delta = 0.5 * (lmax + lmin), 0.5 * (lmax - lmin)
+        return 0.5 * (lmax + lmin), 0.5 * (lmax - lmin)
+
+    def _cheb(self, L, b, x, x_zero=False, started=False):
+        """x += Chebyshev(D^-1 A) correction for A x = b (degree k);
+        x_zero: x is taken as 0 (r = b, no product; x is only written).  Each
+        step is one fused pass (pf3d_bsr_smooth): x += d, r -= A d and the next
+        d = a D^-1 r + c d together; the last one also adds that d.  started:
+        L['d'] already holds D^-1 b / theta."""
+        theta, delta = self._cheb_scale(L)
         sigma = theta / delta
         rho_old = 1. / sigma
         A, D = L['A'], L['Dinv'].val
         r, cur, nxt = L['r'], L['d'], L['t']
         # r = b - A x (r = b from a zero x); d = D^-1 r / theta
-        _fused(A, None if x_zero else x, b, r, dinv=D, dnew=cur, sa=1., sb=-1.,
-               c1=1. / theta)
-        for k in range(self.cheb_degree):
-            if k == self.cheb_degree - 1:
-                _axpby(1., cur, 1., x)             # x += d
-                break
+        if not started:
+            _fused(A, None if x_zero else x, b, r, dinv=D, dnew=cur, sa=1., sb=-1.,
+                   c1=1. / theta)
+        if self.cheb_degree == 1:
+            _axpby(1., cur, 0. if x_zero else 1., x)
+        for k in range(self.cheb_degree - 1):
             rho = 1. / (2. * sigma - rho_old)
             # x += d; r -= A d; d = 2 rho / delta D^-1 r + rho rho_old d
-            _fused(A, cur, None, r, dinv=D, dold=cur, dnew=nxt, xacc=x, sa=1., sb=-1.,
-                   c1=2. * rho / delta, c2=rho * rho_old)
+            # (from a zero x the first residual is b itself)
+            _fused(A, cur, b if x_zero and k == 0 else None, r, dinv=D, dold=cur, dnew=nxt,
+                   xacc=x, sa=1., sb=-1., c1=2. * rho / delta, c2=rho * rho_old,
+                   xmode=(1 if x_zero and k == 0 else 0) + (2 if k == self.cheb_degree - 2 else 0))
             cur, nxt = nxt, cur
             rho_old = rho
 
@@ -473,8 +481,8 @@ class SAAMG:
             _lib.call('pf3d_to_f64', zf.numel(), z32.data_ptr(), zf.data_ptr(), _s())
         return Z
 
-    def vcycle(self, b, x, lvl=0):
-        """x = M^-1 b (x is overwritten)."""
+    def vcycle(self, b, x, lvl=0, started=False):
+        """x = M^-1 b (x is overwritten); started: see _cheb."""
         if lvl == len(self.levels):
             if b.dtype == torch.float64:
                 _lib.call('pf3d_gemv_t', self.nc, self.nc, self.coarse_inv.data_ptr(), self.nc,
@@ -487,13 +495,18 @@ class SAAMG:
                 _lib.call('pf3d_to_f32', self.nc, x64.data_ptr(), x.data_ptr(), _s())
             return x
         L = self.levels[lvl]
-        _axpby(0., b, 0., x)                       # x = 0
-        self._cheb(L, b, x, x_zero=True)
+        self._cheb(L, b, x, x_zero=True, started=started)
         r = L['r']
         _fused(L['A'], x, b, r, sa=1., sb=-1.)     # r = b - A x
         bc, xc = L['bc'], L['xc']
-        L['R'](r, bc)
-        self.vcycle(bc, xc, lvl + 1)
+        last = lvl + 1 == len(self.levels)
+        if last:
+            L['R'](r, bc)
+        else:  # the restriction also starts the next level's smoother
+            N = self.levels[lvl + 1]
+            _fused(L['R'], r, None, bc, dinv=N['Dinv'].val, dnew=N['d'], sa=0., sb=1.,
+                   c1=1. / self._cheb_scale(N)[0])
+        self.vcycle(bc, xc, lvl + 1, started=not last)
         _fused(L['P'], xc, None, x, sa=1., sb=1.)  # x += P xc
         self._cheb(L, b, x)
         return x
@@ -537,13 +550,14 @@ def _fused_mv(M, nv, ldx, xin, ld, b, r, dinv=None, dold=None, dnew=None, xacc=N
 
 
 def _fused(M, xin, b, r, dinv=None, dold=None, dnew=None, xacc=None, sa=1., sb=1., c1=0.,
-           c2=0.):
-    """One pf3d_bsr_fused(_f32) pass with the operator M (a _Dev):
-    r = sa (b or r) + sb M xin; dnew = c1 Dinv r + c2 dold; xacc += dold."""
-    fn = 'pf3d_bsr_fused' if M.fn == 'pf3d_bsr_spmv' else 'pf3d_bsr_fused_f32'
+           c2=0., xmode=0):
+    """One pf3d_bsr_smooth(_f32) pass with the operator M (a _Dev):
+    r = sa (b or r) + sb M xin; dnew = c1 Dinv r + c2 dold; xacc += dold
+    (xmode & 1: xacc = dold; xmode & 2: then += dnew)."""
+    fn = 'pf3d_bsr_smooth' if M.fn == 'pf3d_bsr_spmv' else 'pf3d_bsr_smooth_f32'
     _lib.call(fn, M.nb, M.row_ptr.data_ptr(), M.col_idx.data_ptr(), M.val.data_ptr(), _ptr(xin),
               _ptr(b), r.data_ptr(), _ptr(dinv), _ptr(dold), _ptr(dnew), _ptr(xacc), float(sa),
-              float(sb), float(c1), float(c2), _s())
+              float(sb), float(c1), float(c2), int(xmode), _s())
 
 
 def _dot(a, b, out):
@@ -558,8 +572,8 @@ class _CGIteration:
     """Buffers of one preconditioned-CG solve and one iteration captured in
     a HIP graph: q = A p, p.q, x and r updated, z = V-cycle(r), r.z (and
     r.z_old), r.r, beta, p updated -- scalars on the device
-    (pf3d_cg_update_xr, pf3d_cg_beta, pf3d_cg_update_p), so replays need no
-    host round trip.  Kept on the system per preconditioner and reused by
+    (pf3d_cg_step_xr, pf3d_cg_dots, pf3d_cg_step_p), so replays need no host
+    round trip.  Kept on the system per preconditioner and reused by
     later solves."""
 
     def __init__(self, system, amg):
@@ -574,8 +588,8 @@ class _CGIteration:
         self.flexible = amg.precision != 'fp64'
         self.x, self.r, self.p, self.q, self.z = (zeros(n) for _ in range(5))
         self.zold = zeros(n) if self.flexible else None
-        self.s = zeros(8)           # r.z, p.q, -, r.z new, beta, r.r, r.z_old
-        self.work = zeros(1024)
+        self.s = zeros(8)           # r.z, p.q, -, -, beta, r.r, -, r.z of the next step
+        self.work = zeros(3 * 1024)
         self.graph = None
 
     @property
@@ -589,21 +603,18 @@ class _CGIteration:
     def step(self):
         """One iteration's launches (eager, or recorded by capture())."""
         self.system.matvec(self.p, self.q)
-        self._dot_into(self.p, self.q, 1)
-        _lib.call('pf3d_cg_update_xr', self.n, self.s.data_ptr(), self.p.data_ptr(),
-                  self.q.data_ptr(), self.x.data_ptr(), self.r.data_ptr(), _s())
+        s, w, st = self.s.data_ptr(), self.work.data_ptr(), _s()
+        _lib.call('pf3d_cg_step_xr', self.n, s, w, self.p.data_ptr(), self.q.data_ptr(),
+                  self.x.data_ptr(), self.r.data_ptr(), st)
         if self.flexible:
             _axpby(1., self.z, 0., self.zold)
         self.amg._apply(self.r, self.z)
-        self._dot_into(self.r, self.z, 3)
-        if self.flexible:
-            # beta = r.(z_new - z_old) / r_old.z_old keeps CG's rate with a
-            # preconditioner that is linear only up to FP32 rounding
-            self._dot_into(self.r, self.zold, 6)
-        self._dot_into(self.r, self.r, 5)
-        _lib.call('pf3d_cg_beta', self.s.data_ptr(), int(self.flexible), _s())
-        _lib.call('pf3d_cg_update_p', self.n, self.s.data_ptr(), self.z.data_ptr(),
-                  self.p.data_ptr(), _s())
+        # flexible: beta = r.(z_new - z_old) / r_old.z_old keeps CG's rate with
+        # a preconditioner that is linear only up to FP32 rounding
+        _lib.call('pf3d_cg_dots', self.n, self.r.data_ptr(), self.z.data_ptr(), _ptr(self.zold), w,
+                  st)
+        _lib.call('pf3d_cg_step_p', self.n, s, w, int(self.flexible), self.z.data_ptr(),
+                  self.p.data_ptr(), st)
 
     def capture(self):
         with _capture_guard():
@@ -620,10 +631,10 @@ class _CGIteration:
         self.graph = g
 
     def restart(self):
-        """p = z = V-cycle(r), s[0] = r.z (r holds the true residual)."""
+        """p = z = V-cycle(r), s[7] = r.z (r holds the true residual)."""
         self.amg._apply(self.r, self.z)
         _axpby(1., self.z, 0., self.p)
-        self._dot_into(self.r, self.z, 0)
+        self._dot_into(self.r, self.z, 7)
 
 
 def amg_pcg(system, amg, f, rtol=1e-8, maxiter=2000, x0=None, log=None, stall=400, check=None,

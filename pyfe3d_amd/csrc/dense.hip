@@ -133,6 +133,108 @@ __global__ void __launch_bounds__(256) dot_finish(int nparts, const double *__re
     if (threadIdx.x == 0) out[0] = sh[0];
 }
 
+// The conjugate-gradient iteration without finishing launches: the dot
+// products stay as dot_partial's partial sums, and the kernel that needs one
+// adds them in every workgroup, in dot_finish's order (the same bits).
+// Slots: s[7] r.z of the coming step, s[0] r.z of the current one (set by
+// cg_step_xr, which no workgroup of that launch reads), s[1] p.q, s[4] beta,
+// s[5] r.r.
+__device__ __forceinline__ double partial_total(int nparts, const double *__restrict__ part,
+                                                double *sh)
+{
+    double v = 0.;
+    for (int k = threadIdx.x; k < nparts; k += 256) v += part[k];
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        // the tree 128, 64, 32, ... of dot_finish
+        const int l = threadIdx.x;
+        double t = (sh[l] + sh[l + 128]) + (sh[l + 64] + sh[l + 192]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o, 64);
+        if (l == 0) sh[256] = t;
+    }
+    __syncthreads();
+    const double r = sh[256];
+    __syncthreads();
+    return r;
+}
+
+__global__ void __launch_bounds__(256)
+    cg_step_xr(int64_t n, double *__restrict__ s, int nparts, const double *__restrict__ part,
+               const double *__restrict__ p, const double *__restrict__ q, double *__restrict__ x,
+               double *__restrict__ r)
+{
+    __shared__ double sh[257];
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    double pv = 0., qv = 0., xv = 0., rv = 0.;
+    if (i < n) {
+        pv = p[i];
+        qv = q[i];
+        xv = x[i];
+        rv = r[i];
+    }
+    const double rz = s[7];
+    const double pq = partial_total(nparts, part, sh);
+    const double alpha = pq != 0. ? rz / pq : 0.;
+    if (i < n) {
+        x[i] = xv + alpha * pv;
+        r[i] = rv - alpha * qv;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        s[0] = rz;
+        s[1] = pq;
+    }
+}
+
+// partial sums of a.b, a.c and a.a (c may be null)
+__global__ void __launch_bounds__(256)
+    cg_dots(int64_t n, const double *__restrict__ a, const double *__restrict__ b,
+            const double *__restrict__ c, double *__restrict__ part)
+{
+    __shared__ double sh[3][256];
+    double s[3] = {0., 0., 0.};
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * 256) {
+        const double v = a[i];
+        s[0] += v * b[i];
+        s[1] += v * v;
+        if (c) s[2] += v * c[i];
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++) sh[k][threadIdx.x] = s[k];
+    __syncthreads();
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    if (w < 3) {
+        double t = (sh[w][l] + sh[w][l + 128]) + (sh[w][l + 64] + sh[w][l + 192]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o, 64);
+        if (l == 0) part[w * DOT_BLOCKS + blockIdx.x] = t;
+    }
+}
+
+__global__ void __launch_bounds__(256)
+    cg_step_p(int64_t n, double *__restrict__ s, int nparts, const double *__restrict__ part,
+              int flexible, const double *__restrict__ z, double *__restrict__ p)
+{
+    __shared__ double sh[257];
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const double zv = i < n ? z[i] : 0., pv = i < n ? p[i] : 0.;
+    const double old = s[0];
+    const double rz = partial_total(nparts, part, sh);
+    const double num = rz - (flexible ? partial_total(nparts, part + 2 * DOT_BLOCKS, sh) : 0.);
+    const double beta = old != 0. ? num / old : 0.;
+    if (i < n) p[i] = zv + beta * pv;
+    if (blockIdx.x == 0) {
+        const double rr = partial_total(nparts, part + DOT_BLOCKS, sh);
+        if (threadIdx.x == 0) {
+            s[7] = rz;
+            s[4] = beta;
+            s[5] = rr;
+        }
+    }
+}
+
 // C = A B^T for p vectors A[i][0:n] (row stride lda) and q vectors
 // B[j][0:n] (row stride ldb), p, q <= 32: the Gram matrices of a block
 // eigensolver.  Stage 1: block (g, ti, tj) accumulates a 4 x 4 tile over
@@ -258,6 +360,43 @@ int pf3d_to_f64(int64_t n, const float *a, double *b, void *stream)
     hipLaunchKernelGGL(widen, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                        (hipStream_t)stream, n, a, b);
     return pf3d_hip_check(hipGetLastError(), "pf3d_to_f64");
+}
+
+static int dot_blocks(int64_t n)
+{
+    const int64_t b = (n + 255) / 256;
+    return (int)(b < DOT_BLOCKS ? (b < 1 ? 1 : b) : DOT_BLOCKS);
+}
+
+int pf3d_cg_dots(int64_t n, const double *a, const double *b, const double *c, double *part,
+                 void *stream)
+{
+    if (n <= 0 || !a || !b || !part) return pf3d_fail(PF3D_E_ARG, "pf3d_cg_dots: bad arguments");
+    hipLaunchKernelGGL(cg_dots, dim3(dot_blocks(n)), dim3(256), 0, (hipStream_t)stream, n, a, b, c,
+                       part);
+    return pf3d_hip_check(hipGetLastError(), "pf3d_cg_dots");
+}
+
+int pf3d_cg_step_xr(int64_t n, double *s, double *part, const double *p, const double *q,
+                    double *x, double *r, void *stream)
+{
+    if (n <= 0 || !s || !part || !p || !q || !x || !r)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_cg_step_xr: bad arguments");
+    const int nb = dot_blocks(n);
+    hipLaunchKernelGGL(dot_partial, dim3(nb), dim3(256), 0, (hipStream_t)stream, n, p, q, part);
+    hipLaunchKernelGGL(cg_step_xr, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, n, s, nb, part, p, q, x, r);
+    return pf3d_hip_check(hipGetLastError(), "pf3d_cg_step_xr");
+}
+
+int pf3d_cg_step_p(int64_t n, double *s, const double *part, int flexible, const double *z,
+                   double *p, void *stream)
+{
+    if (n <= 0 || !s || !part || !z || !p)
+        return pf3d_fail(PF3D_E_ARG, "pf3d_cg_step_p: bad arguments");
+    hipLaunchKernelGGL(cg_step_p, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, n, s, dot_blocks(n), part, flexible, z, p);
+    return pf3d_hip_check(hipGetLastError(), "pf3d_cg_step_p");
 }
 
 int pf3d_dot(int64_t n, const double *a, const double *b, double *out, double *work,

@@ -409,3 +409,39 @@ def test_split_products(splits):
               1, None, 0, splits, part.data_ptr(), torch.cuda.current_stream().cuda_stream)
     tol = 2. ** -23 * K * (a.abs().T @ b.abs()).numpy()
     assert (np.abs(c.cpu().numpy() - (a.T @ b).numpy() - 2.) <= tol).all()
+
+
+@pytest.mark.parametrize('rows', [1, 3, 4, 5, 12287, 12288, 12301])
+def test_product_row_routes(rows):
+    """One and four block rows per wave at the line between them and at the
+    ends: the product and a smoothing step (with the choices of xacc) against
+    float64 sums of the same chain matrix."""
+    from pyfe3d_amd import _lib
+    rng = np.random.default_rng(rows)
+    nb = [[j for j in (i - 1, i, i + 1) if 0 <= j < rows] for i in range(rows)]
+    rp = np.concatenate([[0], np.cumsum([len(s) for s in nb])])
+    ci = np.concatenate(nb)
+    val = rng.normal(size=(ci.size, 6, 6))
+    x, b, d, D = (rng.normal(size=s) for s in ((rows, 6), (rows, 6), (rows, 6), (rows, 6, 6)))
+    q = np.zeros((rows, 6))
+    np.add.at(q, np.repeat(np.arange(rows), np.diff(rp)), np.einsum('nij,nj->ni', val, x[ci]))
+    t = lambda a: T(np.ascontiguousarray(a).reshape(-1), torch.float64)
+    trp, tci, tv, tx, tb, td, tD = (T(rp, torch.int32), T(ci, torch.int32), t(val), t(x), t(b),
+                                    t(d), t(D))
+    st = torch.cuda.current_stream().cuda_stream
+    y = torch.full((6 * rows,), float('nan'), dtype=torch.float64, device=DEV)
+    _lib.call('pf3d_bsr_spmv', rows, trp.data_ptr(), tci.data_ptr(), tv.data_ptr(), tx.data_ptr(),
+              y.data_ptr(), st)
+    # 18 products of unit size: a few eps of their sum
+    assert np.abs(y.cpu().numpy() - q.ravel()).max() <= 1e-13
+    r = b - q
+    dn = 0.7 * np.einsum('nij,nj->ni', D, r) + 0.3 * d
+    for xmode in range(4):
+        tr, tn, acc = y.clone(), torch.full_like(y, float('nan')), t(b)
+        _lib.call('pf3d_bsr_smooth', rows, trp.data_ptr(), tci.data_ptr(), tv.data_ptr(),
+                  tx.data_ptr(), tb.data_ptr(), tr.data_ptr(), tD.data_ptr(), td.data_ptr(),
+                  tn.data_ptr(), acc.data_ptr(), 1., -1., 0.7, 0.3, xmode, st)
+        want = (0. if xmode & 1 else b) + d + (dn if xmode & 2 else 0.)
+        assert np.abs(tr.cpu().numpy() - r.ravel()).max() <= 1e-13
+        assert np.abs(tn.cpu().numpy() - dn.ravel()).max() <= 1e-12
+        assert np.abs(acc.cpu().numpy() - want.ravel()).max() <= 1e-12
