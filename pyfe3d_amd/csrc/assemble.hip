@@ -8,6 +8,8 @@
 // it in an LDS tile; the wave then streams the element's slots out in the
 // reference's slot order with unit-stride stores, so every store
 // instruction writes 64 consecutive doubles of the COO value array.
+#include <type_traits>
+
 #include "pf3d_device.hpp"
 
 // unroll factor of the 2x2 Gauss loop of the Quad4 KC0 block integral
@@ -435,10 +437,19 @@ __device__ __forceinline__ void membrane_forces(const Shell &s, const double *Nx
 // scalar per pair times one 6x6 pattern per element (KG: G_IJ n n^T on the
 // translations, n the element normal; M: H_IJ R6 m R6^T), so the work is
 // split in two phases.  Phase 1: one lane per element (64 elements per
-// wave; 32 for M) computes the geometry, the per-pair scalars and the
-// pattern into LDS.  Phase 2: the wave streams its elements' slots in the
-// reference layout, consecutive lanes computing consecutive slots from LDS,
-// so the stores are contiguous across lanes.
+// block; 32 for M) computes the geometry, the per-pair scalars and the
+// pattern into LDS.  Phase 2: the block's four waves stream its elements'
+// slots in the reference layout, consecutive lanes computing consecutive
+// slots from LDS, so the stores are contiguous across lanes.
+// What bounds it: the stores, once enough waves stream.  With one wave per
+// block phase 2 had 7 waves a CU on a 60,600-element mesh, each recomputing
+// two slot maps with a division per pair: M 60 us (3.9 TB/s), and 39 us on
+// 361 elements; four waves per block and the maps out of the loop: 36 us
+// (6.4 TB/s) and 10 us, lumped M 44 -> 24 us, 490,000 elements 384 -> 360 us.
+// KG spends as long in phase 1, whose 160 registers four waves would hold for
+// nothing (490,000 elements: 140 us with 256 threads, 135 with 64): two waves,
+// 24 -> 17 us and 129 us.  With beams in the same launch two waves are slower
+// (92 us for 512 panels against 84), so the mixed KG keeps one wave a block.
 // ------------------------------------------------------------------------
 // 16-byte vectors for the slot streaming; F_VEC (internal launch flag):
 // every element's first slot is even and v, r, c are 16-byte aligned
@@ -462,19 +473,25 @@ __device__ __forceinline__ void store2(T *p, T v)
 #endif
 }
 
+// threads per block of the stream kernels: one element type, mixed types
+constexpr int stream_threads(int mat) { return mat == MASS ? 256 : 128; }
+constexpr int mixed_threads(int mat) { return mat == MASS ? 256 : 64; }
+
 // LDS layout of one shell_stream block (also sizes the mixed-type kernels)
 template <int ET, int MAT>
 struct StreamLds {
     static constexpr int NN = (ET == TRIA3R) ? 3 : 4;
     static constexpr int NP = NN * NN;
-    static constexpr int W = (MAT == MASS) ? NP + 36 : NP + 3;  // per-element LDS doubles
-    // elements per 64-lane block: the mass pattern needs 4x the LDS of KG,
-    // so mass blocks take 32 elements to keep several waves per CU
+    // per-element LDS doubles, an odd number: the lanes of phase 1 write one
+    // element each
+    static constexpr int W = ((MAT == MASS) ? NP + 36 : NP + 3) | 1;
+    // elements per block: the mass pattern needs 4x the LDS of KG, so mass
+    // blocks take 32 elements to keep several blocks per CU
     static constexpr int EPB = (MAT == MASS) ? 32 : 64;
     static constexpr int BYTES = EPB * (W * 8 + NN * 8 + 8);
 };
 
-template <int ET, int MAT>
+template <int ET, int MAT, int T>
 __device__ __forceinline__ void shell_stream_body(const AsmArgs &a, int64_t blk, char *lds)
 {
     using L = StreamLds<ET, MAT>;
@@ -670,45 +687,74 @@ __device__ __forceinline__ void shell_stream_body(const AsmArgs &a, int64_t blk,
         if (kg_like(MAT)) return (d[NP + dr] * d[I * NN + J]) * d[NP + dc];
         return d[I * NN + J] * d[NP + 6 * dr + dc];
     };
-    const int total = nel * nslot;
-    if (NN == 4 && (a.flags & F_VEC)) {
-        // pairs of consecutive slots (every row of these layouts has an even
-        // length, so a pair never crosses a row): one 16-byte store per pair;
-        // F_VEC: contiguous 16-byte aligned blocks of an even slot count
-        for (int t2 = lane; 2 * t2 < total; t2 += 64) {
-            const int t = 2 * t2;
-            const int el = t / nslot, k = t - el * nslot;
+    // the slot count as a constant: nslot is one of two, so the divisions by
+    // it become multiplications
+    auto stream = [&](auto slots) {
+        constexpr int NS = decltype(slots)::value;
+        if constexpr (NN == 4) if (a.flags & F_VEC) {
+            // pairs of consecutive slots (every row of these layouts has an
+            // even length, so a pair never crosses a row): one 16-byte store
+            // per pair; F_VEC: contiguous 16-byte aligned blocks of an even
+            // slot count
+            auto put = [&](int el, int k, int I0, int J0, int dr0, int dc0, int I1, int J1,
+                           int dr1, int dc1) {
+                const dbl2 val = {slot_val(el, I0, J0, dr0, dc0),
+                                  slot_val(el, I1, J1, dr1, dc1)};
+                const int64_t slot = (e0 + el) * NS + k;
+                dbl2 *dst = reinterpret_cast<dbl2 *>(a.v + slot);
+                if (overwrite) store2(dst, val);
+                else *dst = *dst + val;
+                if (write_idx) {
+                    store2(reinterpret_cast<lng2 *>(a.r + slot),
+                           lng2{sconn[el][I0] + dr0, sconn[el][I1] + dr1});
+                    store2(reinterpret_cast<lng2 *>(a.c + slot),
+                           lng2{sconn[el][J0] + dc0, sconn[el][J1] + dc1});
+                }
+            };
+            constexpr int NPR = NS / 2, G = T / NPR;
             int I0, J0, dr0, dc0, I1, J1, dr1, dc1;
-            slot_map(k, I0, J0, dr0, dc0);
-            slot_map(k + 1, I1, J1, dr1, dc1);
-            const dbl2 val = {slot_val(el, I0, J0, dr0, dc0), slot_val(el, I1, J1, dr1, dc1)};
+            if constexpr (G >= 1) {
+                // a lane keeps one pair and walks the elements, so the slot
+                // map is out of the loop: 240 of 256 lanes work for the
+                // consistent M, 144 for the lumped one, 72 of 128 for KG
+                const int first = lane / NPR, k = 2 * (lane - first * NPR);
+                if (first >= G) return;
+                slot_map(k, I0, J0, dr0, dc0);
+                slot_map(k + 1, I1, J1, dr1, dc1);
+#pragma unroll 4
+                for (int el = first; el < nel; el += G)
+                    put(el, k, I0, J0, dr0, dc0, I1, J1, dr1, dc1);
+            } else {
+                for (int t = lane; t < nel * NPR; t += T) {
+                    const int el = t / NPR, k = 2 * (t - el * NPR);
+                    slot_map(k, I0, J0, dr0, dc0);
+                    slot_map(k + 1, I1, J1, dr1, dc1);
+                    put(el, k, I0, J0, dr0, dc0, I1, J1, dr1, dc1);
+                }
+            }
+            return;
+        }
+        // consecutive lanes write consecutive slots of the block's elements
+        for (int t = lane; t < nel * NS; t += T) {
+            const int el = t / NS, k = t - el * NS;
+            int I, J, dr, dc;
+            slot_map(k, I, J, dr, dc);
+            const double val = slot_val(el, I, J, dr, dc);
             const int64_t slot = sk0[el] + k;
-            dbl2 *dst = reinterpret_cast<dbl2 *>(a.v + slot);
-            if (overwrite) store2(dst, val);
-            else *dst = *dst + val;
+            if (overwrite) __builtin_nontemporal_store(val, a.v + slot);
+            else a.v[slot] += val;
             if (write_idx) {
-                store2(reinterpret_cast<lng2 *>(a.r + slot),
-                       lng2{sconn[el][I0] + dr0, sconn[el][I1] + dr1});
-                store2(reinterpret_cast<lng2 *>(a.c + slot),
-                       lng2{sconn[el][J0] + dc0, sconn[el][J1] + dc1});
+                a.r[slot] = sconn[el][I] + dr;
+                a.c[slot] = sconn[el][J] + dc;
             }
         }
-        return;
-    }
-    // consecutive lanes write consecutive slots of the block's elements
-    for (int t = lane; t < total; t += 64) {
-        const int el = t / nslot, k = t - el * nslot;
-        int I, J, dr, dc;
-        slot_map(k, I, J, dr, dc);
-        const double val = slot_val(el, I, J, dr, dc);
-        const int64_t slot = sk0[el] + k;
-        if (overwrite) __builtin_nontemporal_store(val, a.v + slot);
-        else a.v[slot] += val;
-        if (write_idx) {
-            a.r[slot] = sconn[el][I] + dr;
-            a.c[slot] = sconn[el][J] + dc;
+    };
+    if constexpr (MAT == MASS)
+        if (mtype == 2) {
+            stream(std::integral_constant<int, slot_count<NN>(MASS, 2)>());
+            return;
         }
-    }
+    stream(std::integral_constant<int, slot_count<NN>(MAT, 0)>());
 }
 
 // ------------------------------------------------------------------------
@@ -732,10 +778,10 @@ __device__ __forceinline__ void upper_pair(int sub, int &I, int &J)
 
 
 template <int ET, int MAT>
-__global__ void __launch_bounds__(64) shell_stream(AsmArgs a)
+__global__ void __launch_bounds__(stream_threads(MAT)) shell_stream(AsmArgs a)
 {
     __shared__ __align__(16) char lds[StreamLds<ET, MAT>::BYTES];
-    shell_stream_body<ET, MAT>(a, blockIdx.x, lds);
+    shell_stream_body<ET, MAT, stream_threads(MAT)>(a, blockIdx.x, lds);
 }
 
 // waves per SIMD the register allocation of the KC0 kernel targets
@@ -1428,13 +1474,14 @@ __device__ __forceinline__ void beam_slot(int lumped, int k, int &rl, int &cl)
     }
 }
 
-// beams per block BPB (4 lanes each, BPB <= 16)
+// beams per block BPB (4 lanes each, BPB <= 16); NT threads in the block, at
+// least 4 BPB
 template <int BPB>
 struct BeamLds {
     static constexpr int BYTES = BPB * (144 * 8 + 2 * 8 + 8 + 9 * 8);
 };
 
-template <int ET, int MAT, int BPB>
+template <int ET, int MAT, int BPB, int NT = 64>
 __device__ __forceinline__ void beam_body(const AsmArgs &a, int64_t blk, char *lds)
 {
     double (*tile)[144] = reinterpret_cast<double (*)[144]>(lds);
@@ -1507,7 +1554,7 @@ __device__ __forceinline__ void beam_body(const AsmArgs &a, int64_t blk, char *l
     const bool overwrite = (a.flags & F_OVERWRITE);
     for (int el = 0; el < nel; el++) {
         const int64_t k0 = sk0[el];
-        for (int k = lane; k < nslot; k += 64) {
+        for (int k = lane; k < nslot; k += NT) {
             int rl, cl;
             beam_slot(lumped, k, rl, cl);
             const double val = tile[el][rl * 12 + cl];
@@ -1780,14 +1827,15 @@ mixed_kc0(MixedArgs m)
 
 // KG from displacements or mass (MAT = KG or MASS)
 template <int MAT>
-__global__ void __launch_bounds__(64) mixed_stream(MixedArgs m)
+__global__ void __launch_bounds__(mixed_threads(MAT)) mixed_stream(MixedArgs m)
 {
+    constexpr int T = mixed_threads(MAT);
     __shared__ __align__(16) char lds[mixed_stream_lds<MAT>()];
     const int64_t b = blockIdx.x;
-    if (b < m.blk0[1]) shell_stream_body<QUAD4, MAT>(m.g[0], b, lds);
-    else if (b < m.blk0[2]) shell_stream_body<QUAD4R, MAT>(m.g[1], b - m.blk0[1], lds);
-    else if (b < m.blk0[3]) shell_stream_body<TRIA3R, MAT>(m.g[2], b - m.blk0[2], lds);
-    else beam_body<BEAMC, MAT, MIXED_BPB>(m.g[3], b - m.blk0[3], lds);
+    if (b < m.blk0[1]) shell_stream_body<QUAD4, MAT, T>(m.g[0], b, lds);
+    else if (b < m.blk0[2]) shell_stream_body<QUAD4R, MAT, T>(m.g[1], b - m.blk0[1], lds);
+    else if (b < m.blk0[3]) shell_stream_body<TRIA3R, MAT, T>(m.g[2], b - m.blk0[2], lds);
+    else beam_body<BEAMC, MAT, MIXED_BPB, T>(m.g[3], b - m.blk0[3], lds);
 }
 
 }  // namespace pf3d
@@ -1822,7 +1870,7 @@ static hipError_t launch_shell(const AsmArgs &a, hipStream_t s)
         }
         return hipGetLastError();
     } else {
-        constexpr int EPB = (MAT == MASS) ? 32 : 64;
+        constexpr int EPB = StreamLds<ET, MAT>::EPB;
         const int64_t blocks = (a.n_elem + EPB - 1) / EPB;
         if (blocks == 0) return hipSuccess;
         // paired 16-byte stores: contiguous blocks (no init_k) of an even
@@ -1833,7 +1881,8 @@ static hipError_t launch_shell(const AsmArgs &a, hipStream_t s)
                           ((reinterpret_cast<uintptr_t>(a.r) & 15) == 0 &&
                            (reinterpret_cast<uintptr_t>(a.c) & 15) == 0));
         if (vec) b.flags |= F_VEC;
-        hipLaunchKernelGGL((shell_stream<ET, MAT>), dim3((unsigned)blocks), dim3(64), 0, s, b);
+        hipLaunchKernelGGL((shell_stream<ET, MAT>), dim3((unsigned)blocks),
+                           dim3(stream_threads(MAT)), 0, s, b);
         return hipGetLastError();
     }
 }
@@ -1922,7 +1971,7 @@ hipError_t pf3d_launch_mixed(int mat, const AsmArgs *groups, hipStream_t s)
     MixedArgs m;
     int64_t per_kc0[4] = {Kc0Lds<QUAD4>::EPW, Kc0Lds<QUAD4R>::EPW, Kc0Lds<TRIA3R>::EPW,
                           MIXED_BPB};
-    const int epb = mat == MASS ? 32 : 64;
+    const int epb = mat == MASS ? StreamLds<QUAD4, MASS>::EPB : StreamLds<QUAD4, KG>::EPB;
     int64_t per_stream[4] = {epb, epb, epb, MIXED_BPB};
     m.blk0[0] = 0;
     bool vec = true;
@@ -1954,9 +2003,9 @@ hipError_t pf3d_launch_mixed(int mat, const AsmArgs *groups, hipStream_t s)
         default: hipLaunchKernelGGL(mixed_kc0<7>, grid, blk, 0, s, m);
         }
     } else if (mat == KG) {
-        hipLaunchKernelGGL(mixed_stream<KG>, grid, blk, 0, s, m);
+        hipLaunchKernelGGL(mixed_stream<KG>, grid, dim3(mixed_threads(KG)), 0, s, m);
     } else {
-        hipLaunchKernelGGL(mixed_stream<MASS>, grid, blk, 0, s, m);
+        hipLaunchKernelGGL(mixed_stream<MASS>, grid, dim3(mixed_threads(MASS)), 0, s, m);
     }
     return hipGetLastError();
 }

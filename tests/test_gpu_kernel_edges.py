@@ -445,3 +445,35 @@ def test_product_row_routes(rows):
         assert np.abs(tr.cpu().numpy() - r.ravel()).max() <= 1e-13
         assert np.abs(tn.cpu().numpy() - dn.ravel()).max() <= 1e-12
         assert np.abs(acc.cpu().numpy() - want.ravel()).max() <= 1e-12
+
+
+@pytest.mark.parametrize('etype', ['quad4', 'quad4r', 'tria3r'])
+@pytest.mark.parametrize('n_elem', [1, 31, 32, 33, 63, 64, 65, 97])
+def test_stream_block_edges(etype, n_elem):
+    """KG and M of a last block of 1 to 64 elements (32 for M) against the
+    oracle, with and without slot offsets, nothing written past the end."""
+    from pyfe3d_amd import assembly as A
+    from test_gpu_assembly import TOL, element_errors
+    x, conn, props, u, kw = _mixed_mesh(etype)
+    conn, pid, xmat = conn[:n_elem], kw['pid'][:n_elem], kw['xmat'][:n_elem]
+    args = T(x, torch.float64), T(6 * conn, torch.int64)
+    gkw = dict(pid=T(pid, torch.int32), xmat=T(xmat, torch.float64))
+    rec = T(props, torch.float64)
+    for mat, mtype in (('KG', 0), ('M', 0), ('M', 1), ('M', 2)):
+        size = O.slot_count(etype, mat, mtype)
+        k0 = size * np.arange(n_elem)
+        rr = np.zeros(size * n_elem, np.int64); cc = np.zeros_like(rr); vv = np.zeros(rr.size)
+        O.assemble(etype, mat, x, conn, k0, xmat, pid, props, rr, cc, vv, mtype=mtype,
+                   k6rot=kw['k6rot'][:n_elem], alpha=kw['alpha'][:n_elem],
+                   hg=kw['hg'][:n_elem], u=u)
+        for init_k in (None, T(k0, torch.int64)):
+            r = torch.full((rr.size + 2,), -7, dtype=torch.int64, device=DEV)
+            c, v = r.clone(), torch.full((rr.size + 2,), -7., dtype=torch.float64, device=DEV)
+            kk = dict(gkw, init_k=init_k, overwrite=True)
+            if mat == 'KG':
+                A.shell_kg(etype, *args, T(u, torch.float64), r, c, v, rec, **kk)
+            else:
+                A.shell_m(etype, *args, r, c, v, rec, mtype=mtype, **kk)
+            assert (r[-2:] == -7).all() and (c[-2:] == -7).all() and (v[-2:] == -7.).all()
+            assert (r[:-2].cpu().numpy() == rr).all() and (c[:-2].cpu().numpy() == cc).all()
+            assert element_errors(v[:-2].cpu().numpy(), vv, size, np.arange(n_elem)) <= TOL
