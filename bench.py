@@ -12,7 +12,7 @@ same assembly with int64 row/col indices and accumulating, KG (given
 stress), M, internal forces, and static solves per second at 1e-8 relative
 residual (plain FP64 block-Jacobi PCG against multigrid CG with FP64 and
 FP32 V-cycles, the double-double refinement where an FP64 vector cannot
-reach 1e-8, banded direct solves of a design sweep, the stiffened panel,
+reach 1e-8, direct solves of a design sweep, the stiffened panel,
 the 6M-DOF plate, the learned warm start), with the panel's lowest natural
 frequencies; the CPU baseline times the reference-equivalent path on the
 host.
@@ -240,7 +240,7 @@ def sweep_rates(n_var, log, steps=2, modes=('direct', 'fp64', 'mixed')):
     """Batched design sweep: n_var clamped isotropic plates with smooth
     seeded thickness fields and a central point load, assembled and solved
     to 1e-8 (every variant) per step, as one captured graph per mode:
-    banded Cholesky per plate ('direct'), FP64 block-Jacobi PCG ('fp64'),
+    sparse Cholesky per plate ('direct'), FP64 block-Jacobi PCG ('fp64'),
     PCG reading the operator in FP32 ('mixed').  A step is the whole
     captured graph: property records, KC0, BSR, Dirichlet, block Jacobi,
     FP32 copies and the solve."""
@@ -347,7 +347,7 @@ def factor_roofline(sw, log, reps=3):
 def modal_rates(n, log, k=6):
     """First k natural frequencies of an n x n simply supported isotropic
     plate (u, v, w fixed on the edges, consistent mass): assembly of KC0 and
-    M, BSR, banded Cholesky of K + M and shift-invert Lanczos."""
+    M, BSR, sparse Cholesky of K + M and shift-invert Lanczos."""
     import torch
     from pyfe3d_amd import assembly as A
     from pyfe3d_amd.eigen import GeneralizedEigen
@@ -635,7 +635,7 @@ def profile_kc0(n, launches=3):
 
 def profile_sweep(n_var, steps=3, config=(512, 448, 512, 256)):
     """`steps` direct-solve steps of the n_var-plate design sweep (records,
-    KC0, BSR, Dirichlet, band fill, banded Cholesky, triangular solves) with
+    KC0, BSR, Dirichlet, sparse Cholesky, triangular solves) with
     the launch shape given (factor threads, panel bandwidth, solve threads,
     factor threads of the plates whose band fits the 256-wide panel; default
     the one the autotuner picks for the 4,096-plate sweep), for kernel
@@ -1008,7 +1008,7 @@ def solve_summary(extra):
     if sw:
         out['design_sweep_4096'] = dict(solves_per_s=sw['solves_per_s'],
                                         all_converged=sw['converged'] == sw.get('variants', 4096),
-                                        method='batched banded Cholesky, autotuned launch shape')
+                                        method='batched nested-dissection Cholesky')
     ws = extra.get('warm_start_64x64', {})
     if 'summary' in ws:
         out['learned_warm_start_64x64'] = ws['summary']

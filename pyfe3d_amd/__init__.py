@@ -11,7 +11,7 @@ there is no CPU fallback):
 * ``sparse``    -- COO slots to 6x6 block-sparse rows (slot and element-block
                    plans);
 * ``solver``    -- the static solve (block-Jacobi PCG in FP64 or mixed
-                   precision, refinement, banded direct, multigrid CG);
+                   precision, refinement, nested-dissection direct, multigrid CG);
 * ``amg``       -- smoothed-aggregation multigrid (setup on the GPU) and its
                    CG; ``lobpcg`` / ``eigen`` -- natural frequencies and
                    linear buckling;

@@ -5,13 +5,13 @@
 // solve whose result is still judged by the FP64 residual.
 //
 // Layout: activations NHWC in FP32, weights [C_out][9*C_in] (ky, kx, c_in
-// fastest) in FP32 as the optimiser's master copy.  Every convolution is an
-// im2col gather followed by one GEMM on the matrix cores: operands are
-// rounded to bfloat16 when they are staged into LDS, products accumulate in
-// FP32 (gfx950's v_mfma_f32_16x16x32_bf16: the whole 32-deep LDS tile in
-// one instruction per 16x16 output tile).  The backward pass uses the same GEMM
-// with other strides (dW = dY^T col, dcol = dY W) and a gather col2im, so
-// every gradient is a fixed-order sum.
+// fastest) in FP32 as the optimiser's master copy.  3x3 convolutions between
+// multiples of 32 channels run on the matrix cores straight from the NHWC
+// activations (conv3, conv3_dw); the others are an im2col gather followed by
+// one GEMM: operands are rounded to bfloat16 when they are staged, products
+// accumulate in FP32 (gfx950's v_mfma_f32_16x16x32_bf16).  Their backward
+// pass uses the same GEMM with other strides (dW = dY^T col, dcol = dY W) and
+// a gather col2im.  Every gradient is a fixed-order sum.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>

@@ -357,10 +357,11 @@ class PlateSweep:
 
         Without config: nested dissection (pyfe3d_amd.direct), or, for sweeps
         of bands up to BANDED_MAX whose launch shape :meth:`autotune_direct`
-        has chosen, the banded kernels with that shape.  config: the banded kernels with (factor threads, panel bandwidth,
-        solve threads[, narrow-band factor threads]): banded Cholesky of every
-        variant (one workgroup each) with the forward substitution fused into
-        it, then the backward substitution."""
+        has chosen, the banded kernels with that shape.  config: the banded
+        kernels with (factor threads, panel bandwidth, solve threads[,
+        narrow-band factor threads]): banded Cholesky of every variant (one
+        workgroup each) with the forward substitution fused into it, then
+        the backward substitution."""
         s = _s(stream)
         batch = None if config is not None else self._dissection()
         if batch is not None:
