@@ -262,7 +262,9 @@ struct Conv {
 // columns of a pixel: one 16-byte store.
 //   forward:  row = output pixel, source x at (oy s - 1 + ky, ...)
 //   gradient: row = input pixel,  source dy; with stride 2 the launch's z is
-//   the pixel's parity class, whose pixels share the taps that reach them
+//   the pixel's parity class, whose pixels share the taps that reach them.
+//   Each tap is a sum of its own, the taps are added in order: the bits of
+//   the product with a column matrix and its gather (gemm_bf16, col2im3).
 template <int R, bool GRAD>
 __global__ void __launch_bounds__(256) conv3(Conv c, int64_t M)
 {
@@ -292,11 +294,11 @@ __global__ void __launch_bounds__(256) conv3(Conv c, int64_t M)
         src[r] = c.x + (int64_t)b * Hs * Ws * K + k8;
         out[r] = cls ? ((int64_t)b * c.H + 2 * y + py) * c.W + 2 * x + px : m;
     }
-    f32x4 acc[R][2];
+    f32x4 acc[R][2], sum[R][2];  // (sum: of the taps, gradient only)
 #pragma unroll
     for (int r = 0; r < R; r++)
 #pragma unroll
-        for (int t = 0; t < 2; t++) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < 2; t++) acc[r][t] = sum[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     const __bf16 *wp[2];
 #pragma unroll
     for (int t = 0; t < 2; t++) wp[t] = c.w + (int64_t)min(n0 + 16 * t + li, cols - 1) * 9 * K + k8;
@@ -335,6 +337,14 @@ __global__ void __launch_bounds__(256) conv3(Conv c, int64_t M)
                         acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b[r], acc[r][t],
                                                                              0, 0, 0);
             }
+            if (GRAD)
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int t = 0; t < 2; t++) {
+                        sum[r][t] += acc[r][t];
+                        acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
         }
     }
     // lane: columns n0 + 16 t + 4 (lane / 16) + 0..3 of pixel li
@@ -346,7 +356,7 @@ __global__ void __launch_bounds__(256) conv3(Conv c, int64_t M)
             const int n = n0 + 16 * t + 4 * (lane >> 4);
             if (n >= cols) continue;
             f32x4 *o = reinterpret_cast<f32x4 *>(c.y + out[r] * cols + n);
-            f32x4 v = acc[r][t];
+            f32x4 v = GRAD ? sum[r][t] : acc[r][t];
             if (c.bias) v += *reinterpret_cast<const f32x4 *>(c.bias + n);
             if (c.accumulate) v += *o;
             if (c.relu)

@@ -370,6 +370,46 @@ def test_direct_convolutions(B, H, W, C, N, stride):
         assert ((got - ref).abs() <= 2 * K * eps * mag).all(), floats
 
 
+@pytest.mark.parametrize('B, H, W, C, N, stride', [
+    (1, 1, 1, 32, 32, 1), (2, 3, 5, 64, 32, 1), (3, 8, 8, 32, 96, 2), (1, 7, 9, 96, 64, 2),
+    (2, 16, 15, 32, 32, 1), (40, 64, 64, 32, 32, 1), (2, 64, 64, 64, 128, 2)])
+@pytest.mark.parametrize('accumulate', [0, 1])
+def test_direct_convolutions_bits(B, H, W, C, N, stride, accumulate):
+    """The forward pass and the input gradient against the products with the
+    column matrix, bit for bit: a backward pass rounds each layer's gradient
+    to bfloat16, so that a last bit changed in one layer is a change of 1e-3
+    some layers on."""
+    from pyfe3d_amd import _lib
+    import ctypes
+    rng = np.random.default_rng(H * W + C)
+    Ho, Wo = (H - 1) // stride + 1, (W - 1) // stride + 1
+    f32 = lambda *s: T(rng.normal(size=s), torch.float32)
+    x, w, dy, dx0 = f32(B, H, W, C), f32(N, 9, C), f32(B, Ho, Wo, N), f32(B, H, W, C)
+    wf = torch.empty(N * 9 * C, dtype=torch.bfloat16, device=DEV)
+    wb = torch.empty_like(wf)
+    st = torch.cuda.current_stream().cuda_stream
+    one = lambda t: (ctypes.c_void_p * 1)(t.data_ptr())
+    _lib.call('pf3d_nn_pack', 1, (ctypes.c_int * 1)(N), (ctypes.c_int * 1)(C), one(w), one(wf),
+              one(wb), st)
+    y, y0 = (torch.full((B, Ho, Wo, N), float('nan'), device=DEV) for _ in range(2))
+    dx, dxc = dx0.clone(), dx0.clone()
+    M, Kd = B * Ho * Wo, 9 * C
+    col = torch.empty((M, Kd), device=DEV)
+    gemm = lambda n, k, a, sb, o: _lib.call('pf3d_nn_gemm', M, n, k, a.data_ptr(), k, 1,
+                                            w.data_ptr(), sb[0], sb[1], o.data_ptr(), n, 0, None,
+                                            0, 1, None, st)
+    _lib.call('pf3d_nn_conv', B, H, W, C, stride, x.data_ptr(), wf.data_ptr(), None, 0, N,
+              y.data_ptr(), st)
+    _lib.call('pf3d_nn_im2col', B, H, W, C, stride, x.data_ptr(), col.data_ptr(), st)
+    gemm(N, Kd, col, (Kd, 1), y0)
+    assert torch.equal(y, y0)
+    _lib.call('pf3d_nn_conv_dx', B, H, W, C, stride, dy.data_ptr(), wb.data_ptr(), N,
+              dx.data_ptr(), accumulate, st)
+    gemm(Kd, N, dy, (1, Kd), col)
+    _lib.call('pf3d_nn_col2im', B, H, W, C, stride, col.data_ptr(), dxc.data_ptr(), accumulate, st)
+    assert torch.equal(dx, dxc)
+
+
 @pytest.mark.parametrize('rows, C', [(1, 1), (1, 6), (41, 6), (43, 6), (129, 32), (1000, 128),
                                      (131072, 32), (5, 256), (300, 37), (2500, 3)])
 @pytest.mark.parametrize('masked', [True, False])
