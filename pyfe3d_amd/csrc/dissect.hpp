@@ -17,6 +17,7 @@ namespace nd {
 constexpr int NF = 32;    // panel width (DOFs)
 constexpr int RB = 128;   // rows below the diagonal block per workgroup
 constexpr int TS = 64;    // update tile
+constexpr double MAX_SIDE = 0.7;  // largest share of a part on one side of a cut
 
 // column length of a panel (n rows and the right-hand side's) and of an
 // update matrix: whole 128-byte lines
@@ -77,10 +78,18 @@ class Dissection {
     {
         std::vector<int32_t> all(n1 - n0);
         for (size_t i = 0; i < all.size(); i++) all[i] = (int32_t)(n0 + i);
-        if (!all.empty()) root = split(std::move(all), 0);
+        if (all.empty()) return;
+        if (xy_) {
+            grow(std::move(all));
+            return;
+        }
+        for (auto &part : parts(all)) {
+            std::sort(part.begin(), part.end());  // (the tree it has alone)
+            grow(std::move(part));
+        }
     }
     std::vector<TreeNode> tree;
-    int root = -1;
+    std::vector<int> roots;  // one for each connected part
 
   private:
     const int32_t *rp_, *ci_, *xy_;
@@ -143,12 +152,15 @@ class Dissection {
     }
 
     // cost of the separator q[c.first .. c.second): its size, raised where
-    // one side is much the larger
+    // one side is much the larger, above that of every other cut where it
+    // holds more than MAX_SIDE of the vertices: a tree of slivers is as deep
+    // as the part is long (1,000 levels for a comb of 1,000 teeth)
     static double cut_cost(size_t n, std::pair<size_t, size_t> c)
     {
         if (c.second <= c.first) return 1e300;
         const double big = (double)std::max(c.first, n - c.second) / (double)n;
-        return (double)(c.second - c.first) * (1. + 8. * std::max(0., big - 0.55));
+        return (double)(c.second - c.first) * (1. + 8. * std::max(0., big - 0.55)) +
+               (big > MAX_SIDE ? (double)n : 0.);
     }
 
     // the cheapest inner level of q (in level order): its [begin, end), or
@@ -166,18 +178,50 @@ class Dissection {
         return best;
     }
 
-    int split(std::vector<int32_t> V, int depth)
+    // the connected parts of V (V itself if there is one)
+    std::vector<std::vector<int32_t>> parts(const std::vector<int32_t> &V)
     {
-        if ((int)V.size() <= leaf_) return add(std::move(V), depth);
-        std::vector<int32_t> S, A, B;
-        if (!(xy_ ? by_coordinates(V, S, A, B) : by_levels(V, S, A, B))) return add(std::move(V), depth);
-        const int t = add(std::move(S), depth);
-        std::vector<int32_t>().swap(V);
-        const int a = A.empty() ? -1 : split(std::move(A), depth + 1);
-        const int b = B.empty() ? -1 : split(std::move(B), depth + 1);
-        tree[t].kid[0] = a;
-        tree[t].kid[1] = b;
-        return t;
+        const int todo = ++stamp_, done = ++stamp_;
+        for (int32_t v : V) in(v) = todo;
+        std::vector<std::vector<int32_t>> out;
+        for (int32_t v : V) {
+            if (in(v) != todo) continue;
+            std::vector<int32_t> q{v};
+            in(v) = done;
+            for (size_t h = 0; h < q.size(); h++)
+                for (int p = rp_[q[h]]; p < rp_[q[h] + 1]; p++)
+                    if (in(ci_[p]) == todo) {
+                        in(ci_[p]) = done;
+                        q.push_back(ci_[p]);
+                    }
+            out.push_back(q.size() == V.size() ? V : std::move(q));
+        }
+        return out;
+    }
+
+    // the tree of V, its root at depth 0 (a list of parts to divide: the tree
+    // may be deeper than a thread's stack)
+    void grow(std::vector<int32_t> V)
+    {
+        struct Part {
+            std::vector<int32_t> v;
+            int parent, side, depth;
+        };
+        std::vector<Part> todo;
+        todo.push_back({std::move(V), -1, 0, 0});
+        while (!todo.empty()) {
+            Part p = std::move(todo.back());
+            todo.pop_back();
+            std::vector<int32_t> S, A, B;
+            const bool cut = (int)p.v.size() > leaf_ &&
+                             (xy_ ? by_coordinates(p.v, S, A, B) : by_levels(p.v, S, A, B));
+            const int t = add(std::move(cut ? S : p.v), p.depth);
+            if (p.parent < 0) roots.push_back(t);
+            else tree[p.parent].kid[p.side] = t;
+            if (!cut) continue;
+            if (!B.empty()) todo.push_back({std::move(B), t, 1, p.depth + 1});
+            if (!A.empty()) todo.push_back({std::move(A), t, 0, p.depth + 1});
+        }
     }
 
     // the middle line of the longer direction of a structured grid; vertices
@@ -210,7 +254,8 @@ class Dissection {
     // A level of a breadth-first search is a separator.  Several searches are
     // tried: from the far side of a search, and from what two far sides have
     // in common (on a square grid the far side of a corner is two edges; the
-    // common one gives straight levels).
+    // common one gives straight levels).  The cheapest level may still be a
+    // short diagonal one, within MAX_SIDE.
     bool by_levels(const std::vector<int32_t> &V, std::vector<int32_t> &S,
                    std::vector<int32_t> &A, std::vector<int32_t> &B)
     {
@@ -221,9 +266,18 @@ class Dissection {
         const size_t n = V.size();
         stamp();
         std::vector<int32_t> q = bfs({V[0]}, n);
-        if (q.size() < n) {  // not connected: this part and the rest, no separator
-            const int part = stamp_;
-            for (int32_t v : V) (in(v) == part ? A : B).push_back(v);
+        if (q.size() < n) {
+            // not connected: the parts go to the two sides, a part of more
+            // than half of V is cut as well
+            auto some = parts(V);
+            std::stable_sort(some.begin(), some.end(),
+                             [](auto &x, auto &y) { return x.size() > y.size(); });
+            const bool cut = 2 * some[0].size() > n && (int)some[0].size() > leaf_ &&
+                             by_levels(some[0], S, A, B);
+            for (size_t i = cut; i < some.size(); i++) {
+                auto &to = A.size() <= B.size() ? A : B;
+                to.insert(to.end(), some[i].begin(), some[i].end());
+            }
             return true;
         }
         const int32_t a = least_degree(last_level(q, lev_, n0_));
@@ -295,16 +349,18 @@ inline SystemFronts analyse_system(const int32_t *rp, const int32_t *ci, const i
 {
     Dissection D(rp, ci, coord, n0, n1, leaf);
     SystemFronts out;
-    if (D.root < 0) return out;
-    // post-order: children, then their separator
-    std::vector<int> post, at(D.tree.size(), -1);
-    std::function<void(int)> walk = [&](int t) {
-        for (int c : D.tree[t].kid)
-            if (c >= 0) walk(c);
-        at[t] = (int)post.size();
+    // post-order: children, then their separator (the reverse of a walk that
+    // takes a separator, then its second child's part, then its first's)
+    std::vector<int> post, at(D.tree.size(), -1), todo(D.roots);
+    while (!todo.empty()) {
+        const int t = todo.back();
+        todo.pop_back();
         post.push_back(t);
-    };
-    walk(D.root);
+        for (int c : D.tree[t].kid)
+            if (c >= 0) todo.push_back(c);
+    }
+    std::reverse(post.begin(), post.end());
+    for (size_t i = 0; i < post.size(); i++) at[post[i]] = (int)i;
     std::vector<int32_t> perm(n1 - n0);  // permuted position of each node
     for (int t : post)
         for (int32_t v : D.tree[t].own) {

@@ -187,6 +187,29 @@ def test_dissection_against_dense(name, leaf):
     assert int(bad.item()) > 0
 
 
+def test_dissection_of_separate_parts():
+    """Plates that are not connected, in one system: level by level beside
+    each other, each with the bits of its solution alone."""
+    from types import SimpleNamespace
+    from pyfe3d_amd.solver import StaticSystem
+    grid, copies = _graph('14x11'), 9
+    rp, ci, val, _ = _block_system(grid, 4)
+    f = np.random.default_rng(5).normal(size=6 * len(grid))
+
+    def solve(k):
+        plan = SimpleNamespace(
+            row_ptr=T(np.concatenate([[0]] + [rp[1:] + s * ci.size for s in range(k)]), torch.int32),
+            col_idx=T(np.concatenate([ci + s * len(grid) for s in range(k)]), torch.int32),
+            n_nodes=k * len(grid))
+        system = StaticSystem(plan, T(np.tile(val.reshape(-1), k), torch.float64),
+                              np.zeros(6 * plan.n_nodes))
+        u, info = system.solve(np.tile(f, k), method='direct')
+        assert info['converged']
+        return u.cpu().numpy()
+
+    assert (solve(copies) == np.tile(solve(1), copies)).all()
+
+
 def test_dissection_sweep_matches_banded(monkeypatch):
     """The sweep's route by nested dissection against the banded kernels
     (an explicit launch shape) on uneven plates: every variant within 1e-9
