@@ -614,7 +614,8 @@ int pf3d_batch_solve(int64_t n_var, int64_t nb, const int64_t *row0, const int32
  * pf3d_nd_create analyses the pattern on the host (no device call): host
  * arrays row_ptr, col_idx; system s owns block rows [node0[s],
  * node0[s + 1]), which must cover all n_nodes and reference only each
- * other; coord NULL or the grid position (2 int32 per node) of structured
+ * other (a block stored on one side of the diagonal only stands for both
+ * sides); coord NULL or the grid position (2 int32 per node) of structured
  * plates; parts of at most `leaf` nodes are not divided further.  *plan is
  * an opaque handle for the calls below, read-only after creation, released
  * by pf3d_nd_free.

@@ -119,7 +119,9 @@ __global__ void nd_scatter(Image g, int64_t nnzb, int64_t n_nodes, const double 
         if (d < 0) return;
         // consecutive lanes: consecutive rows of a column
         const int e = (int)(t - b * 36), c = e / 6, r = e - 6 * c;
-        L[d + (int64_t)c * g.ld[b] + r] = val[b * 36 + 6 * r + c];
+        const int ld = g.ld[b];
+        if (ld > 0) L[d + (int64_t)c * ld + r] = val[b * 36 + 6 * r + c];
+        else L[d - (int64_t)c * ld + r] = val[b * 36 + 6 * c + r];
         return;
     }
     const int64_t q = t - nnzb * 36, node = q / 6;

@@ -8,6 +8,7 @@
 #include <atomic>
 #include <functional>
 #include <new>
+#include <stdexcept>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -53,7 +54,7 @@ struct Plan {
     std::vector<int32_t> cmap;    // 2 per list entry: boundary position in child 0, 1 or -1
     std::vector<int32_t> pnode;   // original node of each permuted one
     std::vector<int64_t> dest;    // panel offset of each BSR block, -1: the upper one of its pair
-    std::vector<int32_t> ld;      // its panel's column length
+    std::vector<int32_t> ld;      // its panel's column length, negative: the block goes in transposed
     std::vector<int64_t> rdest;   // right-hand side entry of each permuted node's first column
     std::vector<int32_t> rld;
     std::vector<Task> tasks;
@@ -393,6 +394,32 @@ inline SystemFronts analyse_system(const int32_t *rp, const int32_t *ci, const i
     return out;
 }
 
+// is the block (r, c) in the pattern?
+inline bool stored(const int32_t *rp, const int32_t *ci, int32_t r, int32_t c)
+{
+    return std::find(ci + rp[r], ci + rp[r + 1], c) != ci + rp[r + 1];
+}
+
+// the pattern with the transposes of its one-sided blocks
+inline void symmetric_pattern(int64_t n, const int32_t *rp, const int32_t *ci,
+                              std::vector<int32_t> &srp, std::vector<int32_t> &sci)
+{
+    std::vector<int64_t> at(n + 1, 0);
+    for (int64_t r = 0; r < n; r++) {
+        at[r + 1] += rp[r + 1] - rp[r];
+        for (int b = rp[r]; b < rp[r + 1]; b++) at[ci[b] + 1] += !stored(rp, ci, ci[b], (int32_t)r);
+    }
+    for (int64_t r = 0; r < n; r++) at[r + 1] += at[r];
+    if (at[n] > INT32_MAX) throw std::length_error("pattern");
+    srp.assign(at.begin(), at.end());
+    sci.resize(at[n]);
+    for (int64_t r = 0; r < n; r++)
+        for (int b = rp[r]; b < rp[r + 1]; b++) {
+            sci[at[r]++] = ci[b];
+            if (!stored(rp, ci, ci[b], (int32_t)r)) sci[at[ci[b]]++] = (int32_t)r;
+        }
+}
+
 inline void build(Plan &P, int64_t n_nodes, const int32_t *rp, const int32_t *ci,
                   const int32_t *coord, int64_t n_sys, const int64_t *node0, int leaf)
 {
@@ -425,8 +452,19 @@ inline void build(Plan &P, int64_t n_nodes, const int32_t *rp, const int32_t *ci
         for (auto &t : th) t.join();
         if (failed) throw std::bad_alloc();
     };
+    // the analysis takes a block that is stored on one side of the diagonal
+    // only for both
+    std::atomic<bool> one_sided{false};
     each(n_sys, 1, [&](int64_t s) {
-        S[s] = analyse_system(rp, ci, coord, node0[s], node0[s + 1], leaf);
+        for (int64_t r = node0[s]; r < node0[s + 1] && !one_sided; r++)
+            for (int b = rp[r]; b < rp[r + 1]; b++)
+                if (!stored(rp, ci, ci[b], (int32_t)r)) one_sided = true;
+    });
+    std::vector<int32_t> srp, sci;
+    if (one_sided) symmetric_pattern(n_nodes, rp, ci, srp, sci);
+    each(n_sys, 1, [&](int64_t s) {
+        S[s] = analyse_system(one_sided ? srp.data() : rp, one_sided ? sci.data() : ci, coord,
+                              node0[s], node0[s + 1], leaf);
     });
     // fronts of all systems by depth, deepest first
     int maxd = 0;
@@ -539,14 +577,19 @@ inline void build(Plan &P, int64_t n_nodes, const int32_t *rp, const int32_t *ci
     each(n_sys, 1, [&](int64_t s) {
         for (int64_t R = node0[s]; R < node0[s + 1]; R++)
             for (int b = rp[R]; b < rp[R + 1]; b++) {
-                const int32_t p = perm[R], q = perm[ci[b]];
-                if (p < q) continue;
+                int32_t p = perm[R], q = perm[ci[b]];
+                const bool upper = p < q;
+                if (upper) {
+                    if (!one_sided || stored(rp, ci, ci[b], (int32_t)R)) continue;
+                    std::swap(p, q);
+                }
                 const Front &F = P.fronts[owner[q]];
                 const int32_t *mine = P.nodes.data() + F.noff;
                 const int cnt = (F.k + F.m) / 6;
                 const int64_t row = std::lower_bound(mine, mine + cnt, p) - mine;
-                P.ld[b] = column(F.k + F.m + 1);
-                P.dest[b] = F.loff + (int64_t)6 * (q - F.own0) * P.ld[b] + 6 * row;
+                const int32_t ld = column(F.k + F.m + 1);
+                P.ld[b] = upper ? -ld : ld;
+                P.dest[b] = F.loff + (int64_t)6 * (q - F.own0) * ld + 6 * row;
             }
     });
 }

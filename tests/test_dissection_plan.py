@@ -176,3 +176,29 @@ def test_tree_of_a_comb_is_flat(spine, tooth):
     log(1 / 0.7) levels."""
     n, edges = _comb(spine, tooth)
     assert Plan(*_pattern(n, edges)).levels <= np.log(n / 16) / np.log(1 / 0.7) + 2
+
+
+@pytest.mark.parametrize('keep', ['lower', 'upper', 'random'])
+@pytest.mark.parametrize('name', sorted(GRAPHS))
+def test_one_sided_blocks(name, keep):
+    """Blocks stored on one side of the diagonal only stand for both: no map
+    entry leaves its front, and the solution is the symmetric matrix's."""
+    n, edges = GRAPHS[name]
+    rp, ci = _pattern(n, edges)
+    rng = np.random.default_rng(n)
+    val, A = _values(n, rp, ci, rng)
+    rows = np.repeat(np.arange(n), np.diff(rp))
+    if keep == 'random':  # of every third pair, one block, either one
+        pair = {(r, c): rng.integers(3) for r, c in zip(rows, ci) if r > c}
+        on = np.array([r == c or pair[max(r, c), min(r, c)] != int(r > c) for r, c in zip(rows, ci)])
+    else:
+        on = rows >= ci if keep == 'lower' else rows <= ci
+    orp = np.concatenate([[0], np.cumsum(np.bincount(rows[on], minlength=n))])
+    plan = Plan(orp, ci[on])
+    front = np.searchsorted(plan.fronts['loff'], plan.dest, side='right') - 1
+    for b in np.flatnonzero(plan.dest >= 0):
+        F = plan.fronts[front[b]]
+        col, row = divmod(plan.dest[b] - F['loff'], abs(plan.ld[b]))
+        assert col + 6 <= F['k'] and row + 6 <= F['k'] + F['m']
+    f = rng.normal(size=6 * n)
+    assert np.abs(plan.solve(val[on], f) - np.linalg.solve(A, f)).max() <= 1e-12

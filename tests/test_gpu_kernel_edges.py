@@ -187,6 +187,32 @@ def test_dissection_against_dense(name, leaf):
     assert int(bad.item()) > 0
 
 
+@pytest.mark.parametrize('keep', ['lower', 'upper'])
+def test_dissection_of_one_sided_blocks(keep):
+    """Blocks stored on one side of the diagonal only: the bits of the whole
+    matrix."""
+    from pyfe3d_amd.direct import DirectPlan
+    rp, ci, val, _ = _block_system(_graph('13x10'), 6)
+    n = rp.size - 1
+    rows = np.repeat(np.arange(n), np.diff(rp))
+    s = torch.cuda.current_stream().cuda_stream
+    b = T(np.random.default_rng(8).normal(size=6 * n), torch.float64)
+    got = []
+    for on in (rows >= 0, rows >= ci if keep == 'lower' else rows <= ci):
+        orp = np.concatenate([[0], np.cumsum(np.bincount(rows[on], minlength=n))])
+        plan = DirectPlan(orp, ci[on], DEV)
+        new = lambda m: torch.empty(max(1, m), dtype=torch.float64, device=DEV)
+        factor, update, work, x = (new(m) for m in (plan.factor_size, plan.update_size,
+                                                    plan.work_size, 6 * n))
+        bad = torch.zeros(1, dtype=torch.int32, device=DEV)
+        tv = T(val[on].reshape(-1), torch.float64)
+        plan.factor(tv.data_ptr(), factor, update, bad, s)
+        plan.solve(factor, b.data_ptr(), x.data_ptr(), work, s)
+        assert int(bad.item()) == 0
+        got.append(x)
+    assert torch.equal(*got)
+
+
 def test_dissection_of_separate_parts():
     """Plates that are not connected, in one system: level by level beside
     each other, each with the bits of its solution alone."""
