@@ -380,6 +380,8 @@ class SAAMG:
                    c1=1. / theta)
         if self.cheb_degree == 1:
             _axpby(1., cur, 0. if x_zero else 1., x)
+        elif self.cheb_degree < 1 and x_zero:      # (no smoothing)
+            _axpby(0., b, 0., x)
         for k in range(self.cheb_degree - 1):
             rho = 1. / (2. * sigma - rho_old)
             # x += d; r -= A d; d = 2 rho / delta D^-1 r + rho rho_old d

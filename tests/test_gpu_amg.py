@@ -89,6 +89,35 @@ def test_vcycle_is_symmetric_and_positive():
     assert float(Ma @ a) > 0 and float(Mb @ b) > 0
 
 
+@pytest.mark.parametrize('precision', ['fp64', 'fp32'])
+@pytest.mark.parametrize('degree', [0, 1, 2, 3])
+def test_vcycle_overwrites(degree, precision):
+    """The V-cycle depends on its right-hand side only, whatever its output
+    and its buffers held, for every smoother degree (0: the coarse
+    correction alone)."""
+    from pyfe3d_amd.mesh import PlateMesh
+    from pyfe3d_amd.shellprop import isotropic_plate
+    m = PlateMesh(21, 17, 1.0, 0.7)
+    rec = isotropic_plate(thickness=0.004, E=70e9, nu=0.33, calc_scf=True).record()
+    sysm = _system(m, m.quads, 'quad4', rec, m.clamped())
+    sysm.setup_amg(m.ncoords, coarse_nodes=20, precisions=(precision,), graph=False,
+                   cheb_degree=degree)
+    amg = sysm.amg if precision == 'fp64' else sysm.amg32
+    assert len(amg.levels) >= 2
+    g = torch.Generator(device='cpu').manual_seed(1)
+    b = (torch.rand(m.n_dof, generator=g, dtype=torch.float64) - 0.5).to(DEV)
+    first = amg._apply(b, torch.zeros_like(b)).clone()
+    assert torch.isfinite(first).all() and float(first.norm()) > 0
+    assert torch.equal(amg._apply(b, torch.full_like(b, float('nan'))), first)
+    amg._apply(torch.full_like(b, float('nan')), torch.zeros_like(b))
+    assert torch.equal(amg._apply(b, torch.zeros_like(b)), first)
+    # the same operator for several vectors
+    many = amg.apply_block(torch.stack([b, -b]), torch.zeros((2, m.n_dof), dtype=b.dtype,
+                                                             device=DEV))
+    tol = 1e-12 if precision == 'fp64' else 1e-5
+    assert float((many[0] - first).norm()) <= tol * float(first.norm())
+
+
 @pytest.mark.parametrize('method', ['amg', 'amg32'])
 def test_amg_pcg_laminate_64(method):
     """The 64x64 jittered laminate plate of the solve benchmark at 1e-8:
