@@ -603,7 +603,9 @@ struct PcgState {
 };
 
 // a / b, 0 where b is 0: an iteration on a residual that has become exactly
-// zero inside a batch (a single block row, an exact start) changes nothing
+// zero inside a batch (a single block row, an exact start) changes nothing.
+// (Where the residual is not zero, on a singular matrix, the host ends the
+// iteration: alpha is 0.)
 __device__ __forceinline__ double ratio(double a, double b) { return b != 0. ? a / b : 0.; }
 
 // partial[k][blk] for up to 2 dot products, grid-strided over n
@@ -925,6 +927,7 @@ __global__ void __launch_bounds__(UT)
     }
     s = sum256(s, sh);
     const double alpha = ratio(st->rzs[par], s);
+    if (blockIdx.x == 0 && tid == 0) st->alpha = alpha;  // (for the host)
     double s0 = 0., s1 = 0.;  // (threads 0 .. 255: row slot tid)
     for (int64_t base = (int64_t)blockIdx.x * 256; base < nb; base += (int64_t)gridDim.x * 256) {
         if (base != (int64_t)blockIdx.x * 256) load(base);
@@ -1066,7 +1069,7 @@ int pcg_run(const Mat &A, const double *b, double *x, double rtol, int maxiter, 
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) return pf3d_hip_check(e, "pcg iterate");
         rel = sqrt(h.rr / bb);
-        if (!isfinite(rel)) break;
+        if (!isfinite(rel) || h.alpha == 0.) break;  // (no step: it would stand still)
     }
     *iters = it;
     *relres = rel;
@@ -1086,7 +1089,8 @@ int pcg64_restarted(const Mat &A, const double *b, double *x, double rtol, int64
                                          work, s, &it, &rel, 25);
         if (st) return st;
         total += it;
-        if (it == 0 || total >= maxiter) break;  // true residual already below rtol
+        // true residual already below rtol, or no step possible
+        if (it == 0 || total >= maxiter || (rel > rtol && isfinite(rel))) break;
     }
     *iters = total;
     *relres = rel;
@@ -1156,8 +1160,10 @@ int pcg_mixed_run(const Mat &A64, const Mat &A32, const double *b, double *x, do
         e = hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) return pf3d_hip_check(e, "mixed pcg iterate");
+        const double last = rel;
         rel = sqrt(h.rr / bb);
-        if (!isfinite(rel)) break;
+        // (the same residual again and no step in sight: x stood still)
+        if (!isfinite(rel) || (h.pq == 0. && rel == last)) break;
         if (rel <= 0.5 * best) {
             best = rel;
             since = 0;

@@ -351,6 +351,27 @@ def test_pcg_routes(rows, method):
         assert few['iters'] == 3
 
 
+@pytest.mark.parametrize('rows', [2, 1366, 21846])
+@pytest.mark.parametrize('method', ['fp64', 'mixed'])
+def test_pcg_without_a_step(rows, method):
+    """Pairs of block rows (I, -I; -I, I) under equal loads: p.q is exactly 0
+    with a residual of 1 (a singular matrix).  Reported at once, not after
+    maxiter iterations that change nothing."""
+    from types import SimpleNamespace
+    from pyfe3d_amd.solver import StaticSystem
+    pair = np.arange(rows) // 2 * 2
+    plan = SimpleNamespace(row_ptr=T(2 * np.arange(rows + 1), torch.int32),
+                           col_idx=T((pair[:, None] + [0, 1]).ravel(), torch.int32), n_nodes=rows)
+    sign = np.where(np.arange(rows)[:, None] == pair[:, None] + [0, 1], 1., -1.)
+    val = sign.reshape(-1, 1, 1) * np.eye(6)
+    s = StaticSystem(plan, T(val.reshape(-1), torch.float64), np.zeros(6 * rows))
+    f = torch.ones(6 * rows, dtype=torch.float64, device=DEV)
+    u, info = s.solve(f, method=method, maxiter=20000)
+    assert not info['converged'] and info['iters'] <= 1000
+    if method == 'fp64':
+        assert info['iters'] == 25
+
+
 def _bf16(a):
     return torch.as_tensor(a, dtype=torch.float32).to(torch.bfloat16).to(torch.float64)
 
