@@ -537,7 +537,7 @@ int pf3d_pcg(int64_t nb, const int32_t *row_ptr, const int32_t *col_idx, const d
  * counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, serving loops, harnesses that
  * forbid hipMalloc).  The PCG vectors live in a fixed device array of the
- * library (one per GPU, ~30 MiB, held until the process ends), so nb is
+ * library (one per GPU, ~24 MiB, held until the process ends), so nb is
  * limited to PF3D_PCG_STATIC_MAX_ROWS block rows (786,432 DOF); larger
  * systems get PF3D_E_ARG.  Calls that overlap on one GPU share that array
  * and race: serialise them (one stream, or events).  Same kernels, same

@@ -992,11 +992,16 @@ hipError_t spmv(const Mat &A, const VT *x, VT *y, hipStream_t s)
     return hipGetLastError();
 }
 
-// workspace: 5 vectors of T (r, z, p, q, second p), partials of p.q and of
-// (r.z, r.r), state
-size_t pcg_bytes(int64_t n, size_t tsize)
+// workspace: vectors r, z, p, q, partials of (r.z, r.r), state; up to
+// FUSED_MAX entries also the second p and the partials of p.q
+constexpr size_t pcg_vec_bytes(int64_t n, size_t tsize)
 {
-    return ((5 * n * tsize + 255) / 256) * 256 + 4 * RED_BLOCKS * sizeof(double) + 256;
+    return ((n <= FUSED_MAX ? 5 : 4) * n * tsize + 255) / 256 * 256;
+}
+constexpr size_t pcg_partials(int64_t n) { return (n <= FUSED_MAX ? 4 : 2) * RED_BLOCKS; }
+constexpr size_t pcg_bytes(int64_t n, size_t tsize)
+{
+    return pcg_vec_bytes(n, tsize) + pcg_partials(n) * sizeof(double) + 256;
 }
 
 // Solve A x = b to ||r|| <= rtol ||b|| (recursive residual), starting from
@@ -1009,9 +1014,9 @@ int pcg_run(const Mat &A, const double *b, double *x, double rtol, int maxiter, 
     const int64_t n = A.nb * 6;
     char *w = (char *)work;
     double *r = (double *)w, *z = r + n, *p = z + n, *q = p + n, *p2 = q + n;
-    double *partial = (double *)(w + ((5 * n * sizeof(double) + 255) / 256) * 256);
+    double *partial = (double *)(w + pcg_vec_bytes(n, sizeof(double)));
     double *pqpart = partial + 2 * RED_BLOCKS;
-    PcgState *st = (PcgState *)(partial + 4 * RED_BLOCKS);
+    PcgState *st = (PcgState *)(partial + pcg_partials(n));
     const unsigned nv = nblk(n, VB), nr = red_blocks(A.nb), nd = red_blocks(n);
     const double *null = nullptr;
     hipError_t e;
@@ -1112,8 +1117,8 @@ int pcg_mixed_run(const Mat &A64, const Mat &A32, const double *b, double *x, do
     const int64_t n = A64.nb * 6;
     char *w = (char *)work;
     double *r = (double *)w, *z = r + n, *p = z + n, *q = p + n;
-    double *partial = (double *)(w + ((5 * n * 8 + 255) / 256) * 256);
-    PcgState *st = (PcgState *)(partial + 4 * RED_BLOCKS);
+    double *partial = (double *)(w + pcg_vec_bytes(n, sizeof(double)));
+    PcgState *st = (PcgState *)(partial + pcg_partials(n));
     double *y = (double *)(w + pcg_bytes(n, sizeof(double)));
     const unsigned nv = nblk(n, VB), nr = red_blocks(A64.nb), nd = red_blocks(n);
     hipError_t e;
@@ -1373,9 +1378,8 @@ int pf3d_pcg(int64_t nb, const int32_t *row_ptr, const int32_t *col_idx, const d
 }  // extern "C"
 
 namespace {
-constexpr size_t PCG_STATIC_BYTES =
-    ((5 * 6 * (size_t)PF3D_PCG_STATIC_MAX_ROWS * sizeof(double) + 255) / 256) * 256 +
-    4 * RED_BLOCKS * sizeof(double) + 256;
+constexpr size_t PCG_STATIC_BYTES = pcg_bytes(6 * PF3D_PCG_STATIC_MAX_ROWS, sizeof(double));
+static_assert(pcg_bytes(FUSED_MAX, sizeof(double)) <= PCG_STATIC_BYTES, "");
 }  // namespace
 
 static __device__ __align__(256) char scratch[PCG_STATIC_BYTES];

@@ -178,3 +178,15 @@ def test_static_workspace_pcg_limits_need_no_device():
     assert lib.pf3d_pcg_static(131073, *args) == -1
     assert b'static workspace' in lib.pf3d_last_error()
     assert lib.pf3d_pcg_static(10, None, *args[1:]) == -1
+
+
+def test_pcg_workspace_sizes():
+    """Four vectors and some KB of sums above the sizes of the two-launch
+    iteration, which takes a fifth."""
+    lib = _lib.load()
+    size = lambda nb: (lib.pf3d_pcg_bytes(ctypes.c_int64(nb), 0, ctypes.byref(n)), n.value)[1]
+    n = ctypes.c_int64()
+    for nb in (21846, 131072, 1000000):
+        assert 0 <= size(nb) - 4 * 48 * nb <= 40000
+    for nb in (1, 1365, 21845):
+        assert 0 <= size(nb) - 5 * 48 * nb <= 80000
