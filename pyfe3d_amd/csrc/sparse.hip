@@ -499,24 +499,25 @@ __global__ void __launch_bounds__(256)
     blk_apply(int64_t nnzb, const int64_t *__restrict__ src_ptr, const int64_t *__restrict__ src,
               int stride, const double *__restrict__ v, double *__restrict__ out, int accumulate)
 {
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (t >= nnzb * 18) return;
-    const int64_t b = t / 18;
-    const int pr = (int)(t - b * 18), m = pr / 3, n = 2 * (pr - 3 * m);
-    const double *p = v + (int64_t)stride * m + n;
-    dbl2 *o = reinterpret_cast<dbl2 *>(out + 2 * t);
-    dbl2 s = accumulate ? *o : dbl2{0., 0.};
-    const int64_t k1 = src_ptr[b + 1];
-    for (int64_t k = src_ptr[b]; k < k1; k += 4) {
-        dbl2 x[4];
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < nnzb * 18;
+         t += (int64_t)gridDim.x * 256) {
+        const int64_t b = t / 18;
+        const int pr = (int)(t - b * 18), m = pr / 3, n = 2 * (pr - 3 * m);
+        const double *p = v + (int64_t)stride * m + n;
+        dbl2 *o = reinterpret_cast<dbl2 *>(out + 2 * t);
+        dbl2 s = accumulate ? *o : dbl2{0., 0.};
+        const int64_t k1 = src_ptr[b + 1];
+        for (int64_t k = src_ptr[b]; k < k1; k += 4) {
+            dbl2 x[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-            x[j] = *reinterpret_cast<const dbl2 *>(p + src[k + j < k1 ? k + j : k1 - 1]);
+            for (int j = 0; j < 4; j++)
+                x[j] = *reinterpret_cast<const dbl2 *>(p + src[k + j < k1 ? k + j : k1 - 1]);
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-            if (k + j < k1) s += x[j];
+            for (int j = 0; j < 4; j++)
+                if (k + j < k1) s += x[j];
+        }
+        *o = s;
     }
-    *o = s;
 }
 
 }  // namespace
@@ -613,8 +614,10 @@ int pf3d_block_apply(int64_t nnzb, const int64_t *src_ptr, const int64_t *src, i
 {
     if (nnzb <= 0 || !src_ptr || !src || nn < 2 || nn > 4 || !v || !bsr_val)
         return pf3d_fail(PF3D_E_ARG, "pf3d_block_apply: bad arguments");
-    hipLaunchKernelGGL(blk_apply, dim3(nblk(nnzb * 18, 256)), dim3(256), 0, (hipStream_t)stream,
-                       nnzb, src_ptr, src, 6 * nn, v, bsr_val, accumulate);
+    // one pass up to 2^31 threads (a launch has fewer than 2^32)
+    const int64_t blocks = (nnzb * 18 + 255) / 256;
+    hipLaunchKernelGGL(blk_apply, dim3((unsigned)(blocks < 1 << 23 ? blocks : 1 << 23)), dim3(256),
+                       0, (hipStream_t)stream, nnzb, src_ptr, src, 6 * nn, v, bsr_val, accumulate);
     return pf3d_hip_check(hipGetLastError(), "pf3d_block_apply");
 }
 

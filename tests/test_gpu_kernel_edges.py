@@ -85,6 +85,28 @@ def test_static_system_setup(etype, nx, ny):
     assert torch.equal(s.dinv32, s.dinv.to(torch.float32))
 
 
+def test_block_sums_past_32_bits():
+    """More than 2^32 pairs of entries (69 GB of block values): every block
+    is written."""
+    from pyfe3d_amd import _lib
+    if torch.cuda.mem_get_info()[0] < 100e9:
+        pytest.skip('needs 100 GB of free memory')
+    nnzb = 2 ** 32 // 18 + 300
+    v = torch.arange(2 * 144, dtype=torch.float64, device=DEV)  # two elements' blocks
+    src_ptr = torch.arange(nnzb + 1, device=DEV)
+    src = 144 * (src_ptr[:-1] % 2)
+    out = torch.full((nnzb, 36), -1., dtype=torch.float64, device=DEV)
+    _lib.call('pf3d_block_apply', nnzb, src_ptr.data_ptr(), src.data_ptr(), 2, v.data_ptr(),
+              out.data_ptr(), 0, torch.cuda.current_stream().cuda_stream)
+    want = v.view(2, 12, 12)[:, :6, :6].reshape(2, 36)
+    for at in range(0, nnzb, 1 << 24):  # (starts on an even block)
+        part = out[at:at + (1 << 24)]
+        assert torch.equal(part[0::2], want[:1].expand(part[0::2].shape))
+        assert torch.equal(part[1::2], want[1:].expand(part[1::2].shape))
+    del out, src, src_ptr
+    torch.cuda.empty_cache()
+
+
 def _graph(name):
     """Block pattern as a list of neighbour sets."""
     rng = np.random.default_rng(len(name))
