@@ -112,22 +112,24 @@ __global__ void nd_zero(int64_t n, double *__restrict__ p)
 __global__ void nd_scatter(Image g, int64_t nnzb, int64_t n_nodes, const double *__restrict__ val,
                            const double *__restrict__ f, double *__restrict__ L)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t b = t / 36;
-    if (b < nnzb) {
-        const int64_t d = g.dest[b];
-        if (d < 0) return;
-        // consecutive lanes: consecutive rows of a column
-        const int e = (int)(t - b * 36), c = e / 6, r = e - 6 * c;
-        const int ld = g.ld[b];
-        if (ld > 0) L[d + (int64_t)c * ld + r] = val[b * 36 + 6 * r + c];
-        else L[d - (int64_t)c * ld + r] = val[b * 36 + 6 * c + r];
-        return;
+    const int64_t total = nnzb * 36 + (f ? 6 * n_nodes : 0);
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
+         t += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t b = t / 36;
+        if (b < nnzb) {
+            const int64_t d = g.dest[b];
+            if (d < 0) continue;
+            // consecutive lanes: consecutive rows of a column
+            const int e = (int)(t - b * 36), c = e / 6, r = e - 6 * c;
+            const int ld = g.ld[b];
+            if (ld > 0) L[d + (int64_t)c * ld + r] = val[b * 36 + 6 * r + c];
+            else L[d - (int64_t)c * ld + r] = val[b * 36 + 6 * c + r];
+            continue;
+        }
+        const int64_t q = t - nnzb * 36, node = q / 6;
+        const int d = (int)(q - 6 * node);
+        L[g.rdest[node] + (int64_t)d * g.rld[node]] = f[6 * (int64_t)g.pnode[node] + d];
     }
-    const int64_t q = t - nnzb * 36, node = q / 6;
-    if (!f || node >= n_nodes) return;
-    const int d = (int)(q - 6 * node);
-    L[g.rdest[node] + (int64_t)d * g.rld[node]] = f[6 * (int64_t)g.pnode[node] + d];
 }
 
 // the children's update matrices as seen by one front
@@ -511,7 +513,10 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-inline unsigned nb256(int64_t n) { return (unsigned)((n + 255) / 256); }
+inline unsigned blocks(int64_t n, int64_t most)
+{
+    return (unsigned)std::min((n + 255) / 256, most);
+}
 
 }  // namespace
 
@@ -603,10 +608,10 @@ int pf3d_nd_factor(const void *plan, const void *image, const double *val, const
     hipStream_t s = (hipStream_t)stream;
     double *L = factor, *D = factor + p.l_size;
     double *U[2] = {update, update + p.u_size[0]};
-    const unsigned zb = std::min(nb256(p.l_size), 16384u);
-    hipLaunchKernelGGL(nd_zero, dim3(zb), dim3(256), 0, s, p.l_size, L);
-    hipLaunchKernelGGL(nd_scatter, dim3(nb256(p.nnzb * 36 + (f ? 6 * p.n_nodes : 0))), dim3(256),
-                       0, s, g, p.nnzb, p.n_nodes, val, f, L);
+    hipLaunchKernelGGL(nd_zero, dim3(blocks(p.l_size, 1 << 14)), dim3(256), 0, s, p.l_size, L);
+    // (one pass up to 2^31 threads: a launch has fewer than 2^32)
+    hipLaunchKernelGGL(nd_scatter, dim3(blocks(p.nnzb * 36 + (f ? 6 * p.n_nodes : 0), 1 << 23)),
+                       dim3(256), 0, s, g, p.nnzb, p.n_nodes, val, f, L);
     int depth = (int)p.levels.size() - 1;
     for (const Level &lv : p.levels) {
         const double *Uc = U[(depth + 1) & 1];
