@@ -40,6 +40,7 @@ class DirectPlan:
         if ci.size < rp[-1]:
             raise ValueError('col_idx has %d entries, row_ptr says %d' % (ci.size, rp[-1]))
         self.device = torch.device(device)
+        self._made = (rp, ci, self.device, coord, node0, int(leaf))  # (for pickling)
         self._plan = ctypes.c_void_p()
         self._free = _lib.load().pf3d_nd_free
         _lib.call('pf3d_nd_create', self.n_nodes, rp.ctypes.data, ci.ctypes.data,
@@ -58,6 +59,12 @@ class DirectPlan:
         plan, self._plan = getattr(self, '_plan', None), None
         if plan:
             self._free(plan)
+
+    def __deepcopy__(self, memo):
+        return self  # (read-only)
+
+    def __reduce__(self):
+        return DirectPlan, self._made
 
     def factor(self, val, factor, update, bad, stream, f=None):
         """Cholesky factor of the systems with BSR values val (device

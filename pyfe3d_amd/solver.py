@@ -118,7 +118,7 @@ class StaticSystem:
 
     def _direct_plan(self):
         """The pattern's nested-dissection plan, kept with the pattern."""
-        d = getattr(self.plan, '_dissection', None)
+        d = getattr(self.plan, '_dissection', None) or getattr(self, '_dissection', None)
         if d is None:
             from .direct import DirectPlan
             rp = self.plan.row_ptr.cpu().numpy()
@@ -130,7 +130,11 @@ class StaticSystem:
                 if bw > maxb:
                     raise ValueError('bandwidth %d after renumbering exceeds %d: use PCG'
                                      % (bw, maxb))
-            d = self.plan._dissection = DirectPlan(rp, ci, self.val.device)
+            d = DirectPlan(rp, ci, self.val.device)
+            try:
+                self.plan._dissection = d
+            except AttributeError:  # (a tuple, a frozen object: kept with the system)
+                self._dissection = d
         return d
 
     def factor_direct(self, stream=None, b=None):

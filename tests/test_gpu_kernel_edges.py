@@ -235,6 +235,48 @@ def test_dissection_of_one_sided_blocks(keep):
     assert torch.equal(*got)
 
 
+def _duck_plan(nb, seed, make):
+    rp, ci, val, _ = _block_system(nb, seed)
+    return (make(row_ptr=T(rp, torch.int32), col_idx=T(ci, torch.int32), n_nodes=len(nb)),
+            T(val.reshape(-1), torch.float64))
+
+
+def test_direct_plans_copy_and_pickle():
+    """A pattern, a system and a sweep that were solved directly are copied
+    and pickled as before, and go on solving; a pattern object without room
+    for an analysis is accepted."""
+    import copy
+    import pickle
+    from collections import namedtuple
+    from types import SimpleNamespace
+    from pyfe3d_amd.solver import StaticSystem
+    from pyfe3d_amd.sweep import PlateSweep
+    nb = _graph('9x7')
+    f = np.random.default_rng(1).normal(size=6 * len(nb))
+    plan, val = _duck_plan(nb, 3, SimpleNamespace)
+    a = StaticSystem(plan, val, np.zeros(6 * len(nb)))
+    u, _ = a.solve(f, method='direct')
+    again, _ = a.solve(f, method='direct')
+    for b in (copy.deepcopy(a), pickle.loads(pickle.dumps(a))):
+        assert torch.equal(b.solve(f, method='direct')[0], again)
+        assert torch.equal(b.solve(f, method='direct', refactor=True)[0], u)
+        c = StaticSystem(b.plan, val, np.zeros(6 * len(nb)))
+        assert torch.equal(c.solve(f, method='direct')[0], u)
+    fixed_plan, val = _duck_plan(nb, 3, namedtuple('Pattern', 'row_ptr col_idx n_nodes'))
+    d = StaticSystem(fixed_plan, val, np.zeros(6 * len(nb)))
+    assert torch.equal(d.solve(f, method='direct')[0], u)
+    sw = PlateSweep([(5, 4), (7, 9)])
+    h, load = sw.random_designs(2)
+    sw.set_thickness(h)
+    sw.set_loads(load)
+    sw.step(mode='direct')
+    u = sw.u.clone()
+    for other in (copy.deepcopy(sw), pickle.loads(pickle.dumps(sw))):
+        other.u.zero_()
+        other.step(mode='direct')
+        assert torch.equal(other.u, u)
+
+
 def test_dissection_of_separate_parts():
     """Plates that are not connected, in one system: level by level beside
     each other, each with the bits of its solution alone."""
