@@ -20,6 +20,11 @@ def _s(stream):
     return (stream if stream is not None else torch.cuda.current_stream()).cuda_stream
 
 
+def _version(t):
+    """Count of torch's in-place changes of t (inference tensors have none)."""
+    return 0 if t.is_inference() else t._version
+
+
 class StaticSystem:
     def __init__(self, plan, val, fixed, stream=None):
         """plan: BSRPlan; val: its BSR values (copied); fixed: bool per DOF."""
@@ -117,37 +122,45 @@ class StaticSystem:
         return self._band_numbering()[0]
 
     def _direct_plan(self):
-        """The pattern's nested-dissection plan, kept with the pattern."""
-        d = getattr(self.plan, '_dissection', None) or getattr(self, '_dissection', None)
-        if d is None:
-            from .direct import DirectPlan
-            rp = self.plan.row_ptr.cpu().numpy()
-            ci = self.plan.col_idx.cpu().numpy()
-            maxb = _lib.call('pf3d_band_max_width')
-            rows = np.repeat(np.arange(self.nb), np.diff(rp))
-            if 6 * int(np.abs(rows - ci[:rows.size]).max(initial=0)) + 5 > maxb:
-                bw = self._band_numbering()[0]
-                if bw > maxb:
-                    raise ValueError('bandwidth %d after renumbering exceeds %d: use PCG'
-                                     % (bw, maxb))
-            d = DirectPlan(rp, ci, self.val.device)
-            try:
-                self.plan._dissection = d
-            except AttributeError:  # (a tuple, a frozen object: kept with the system)
-                self._dissection = d
+        """The pattern's nested-dissection plan, kept with the pattern as long
+        as its arrays are the ones that were analysed."""
+        of = (self.plan.row_ptr, _version(self.plan.row_ptr),
+              self.plan.col_idx, _version(self.plan.col_idx))
+        for holder in (self.plan, self):
+            d, kept = getattr(holder, '_dissection', (None, None))
+            if d is not None and (kept[0] is of[0] and kept[2] is of[2] and
+                                  kept[1::2] == of[1::2]):
+                return d
+        from .direct import DirectPlan
+        rp = self.plan.row_ptr.cpu().numpy()
+        ci = self.plan.col_idx.cpu().numpy()
+        maxb = _lib.call('pf3d_band_max_width')
+        rows = np.repeat(np.arange(self.nb), np.diff(rp))
+        if 6 * int(np.abs(rows - ci[:rows.size]).max(initial=0)) + 5 > maxb:
+            bw = self._band_numbering()[0]
+            if bw > maxb:
+                raise ValueError('bandwidth %d after renumbering exceeds %d: use PCG'
+                                 % (bw, maxb))
+        d = DirectPlan(rp, ci, self.val.device)
+        try:
+            self.plan._dissection = (d, of)
+        except AttributeError:  # (a tuple, a frozen object: kept with the system)
+            self._dissection = (d, of)
         return d
 
     def factor_direct(self, stream=None, b=None):
         """Cholesky factor of the system on the GPU by nested dissection
         (pyfe3d_amd.direct); b: a right-hand side whose forward substitution
-        is carried along (then direct_solve(None, x) finishes it).  Raises if no numbering of the nodes (given, or
-        reverse Cuthill-McKee) has a band within pf3d_band_max_width."""
+        is carried along (then direct_solve(None, x) finishes it).  Raises if
+        no numbering of the nodes (given, or reverse Cuthill-McKee) has a band
+        within pf3d_band_max_width."""
         d = self._direct_plan()
         dev = self.val.device
-        if not hasattr(self, '_factor'):
+        if getattr(self, '_factor_plan', None) is not d:
             self._factor = torch.empty(d.factor_size, dtype=torch.float64, device=dev)
             self._direct_work = torch.empty(d.work_size, dtype=torch.float64, device=dev)
             self._band_bad = torch.zeros(1, dtype=torch.int32, device=dev)
+            self._factor_plan = d
         with torch.cuda.stream(stream):  # (the scratch belongs to the launch stream)
             update = torch.empty(max(1, d.update_size), dtype=torch.float64, device=dev)
             d.factor(self.val.data_ptr(), self._factor, update, self._band_bad, _s(stream),
@@ -157,8 +170,8 @@ class StaticSystem:
     def direct_solve(self, b, x, stream=None):
         """x = K^-1 b with the factor of :meth:`factor_direct` (b None: the
         right-hand side given there)."""
-        self._direct_plan().solve(self._factor, None if b is None else b.data_ptr(),
-                                  x.data_ptr(), self._direct_work, _s(stream))
+        self._factor_plan.solve(self._factor, None if b is None else b.data_ptr(),
+                                x.data_ptr(), self._direct_work, _s(stream))
         return x
 
     def setup_amg(self, xyz, log=None, precisions=('fp64',), graph=True, **kw):

@@ -277,6 +277,40 @@ def test_direct_plans_copy_and_pickle():
         assert torch.equal(other.u, u)
 
 
+@pytest.mark.parametrize('in_place', [False, True])
+def test_direct_solve_on_a_changed_pattern(in_place):
+    """A pattern object whose arrays are replaced or overwritten is analysed
+    anew for the next system; the system made before keeps its factor."""
+    from types import SimpleNamespace
+    from pyfe3d_amd.solver import StaticSystem
+    chain = lambda p: [{p[j] for j in (i - 1, i, i + 1) if 0 <= j < 40} for i in range(40)]
+    p = np.random.default_rng(2).permutation(40)
+    first = chain(np.arange(40))
+    mixed = [None] * 40
+    for i, nb in enumerate(chain(p)):
+        mixed[p[i]] = nb
+    second = mixed if in_place else _graph('8x6')
+    f = [np.random.default_rng(3).normal(size=6 * len(nb)) for nb in (first, second)]
+    alone = []
+    for nb, b in zip((first, second), f):
+        plan, val = _duck_plan(nb, 5, SimpleNamespace)
+        s = StaticSystem(plan, val, np.zeros(b.size))
+        alone.append([s.solve(b, method='direct')[0] for _ in range(2)])
+    plan, val = _duck_plan(first, 5, SimpleNamespace)
+    a = StaticSystem(plan, val, np.zeros(f[0].size))
+    assert torch.equal(a.solve(f[0], method='direct')[0], alone[0][0])
+    new, val = _duck_plan(second, 5, SimpleNamespace)
+    if in_place:
+        plan.row_ptr.copy_(new.row_ptr)
+        plan.col_idx.copy_(new.col_idx)
+    else:
+        plan.row_ptr, plan.col_idx, plan.n_nodes = new.row_ptr, new.col_idx, new.n_nodes
+    b = StaticSystem(plan, val, np.zeros(f[1].size))
+    assert torch.equal(b.solve(f[1], method='direct')[0], alone[1][0])
+    x = torch.empty_like(alone[0][1])
+    assert torch.equal(a.direct_solve(torch.as_tensor(f[0], device=DEV), x), alone[0][1])
+
+
 def test_dissection_of_separate_parts():
     """Plates that are not connected, in one system: level by level beside
     each other, each with the bits of its solution alone."""
