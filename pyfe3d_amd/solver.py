@@ -44,8 +44,8 @@ class StaticSystem:
         # (values past the plan's blocks are kept as they are)
         whole = src.numel() == 36 * plan.col_idx.numel()
         self.val = torch.empty_like(src) if whole else src.clone()
-        self.val32 = (torch.empty_like(src, dtype=torch.float32) if whole
-                      else src.to(torch.float32))
+        self.val32 = (torch.empty(src.numel(), dtype=torch.float32, device=dev) if whole
+                      else src.to(torch.float32).reshape(-1))
         _lib.call('pf3d_bsr_system', nb, plan.row_ptr.data_ptr(), plan.col_idx.data_ptr(),
                   src.data_ptr(), fixed.data_ptr(), self.val.data_ptr(), self.val32.data_ptr(), s)
         self.dinv = torch.empty(nb * 36, dtype=torch.float64, device=dev)

@@ -85,6 +85,20 @@ def test_static_system_setup(etype, nx, ny):
     assert torch.equal(s.dinv32, s.dinv.to(torch.float32))
 
 
+def test_static_system_copies_are_flat():
+    """Values given as (blocks, 6, 6), with and without some past the pattern:
+    kept in that shape, their FP32 copy flat."""
+    from types import SimpleNamespace
+    from pyfe3d_amd.solver import StaticSystem
+    rp, ci, val, _ = _block_system(_graph('3x3'), 1)
+    plan = SimpleNamespace(row_ptr=T(rp, torch.int32), col_idx=T(ci, torch.int32), n_nodes=9)
+    for more in (0, 2):
+        v = T(np.concatenate([val, np.ones((more, 6, 6))]), torch.float64)
+        s = StaticSystem(plan, v, np.zeros(54))
+        assert s.val.shape == v.shape and torch.equal(s.val, v)
+        assert s.val32.dim() == 1 and torch.equal(s.val32, v.reshape(-1).to(torch.float32))
+
+
 def test_block_sums_past_32_bits():
     """More than 2^32 pairs of entries (69 GB of block values): every block
     is written."""
