@@ -211,7 +211,8 @@ class PlateSweep:
     # ------------------------------------------------------- direct solves
     def _band_setup(self):
         """Node permutations (each plate numbered along its longer side, so
-        the band spans the shorter one), bandwidths and band storage."""
+        the band spans the shorter one), bandwidths and the band storage's
+        offsets (:meth:`factor_direct` allocates it)."""
         var, pinv, bws, sizes = [], [], [], []
         for v, (nxe, nye) in enumerate(self.dims):
             nx, ny = nxe + 1, nye + 1
@@ -239,7 +240,6 @@ class PlateSweep:
         boff = np.concatenate([[0], np.cumsum(sizes)])
         self.band_off = torch.as_tensor(boff[:-1].astype(np.int64), device=dev)
         self.band_size = int(boff[-1])
-        self.band = torch.empty(self.band_size, dtype=torch.float64, device=dev)
         self.band_dof0 = torch.as_tensor(6 * self.node0, device=dev)
         self.band_work = torch.empty(6 * self.n_nodes, dtype=torch.float64, device=dev)
         self.band_bad = torch.zeros(1, dtype=torch.int32, device=dev)
@@ -253,7 +253,7 @@ class PlateSweep:
         variant: column j updates the m_j = min(b, n - 1 - j) entries below
         it with m_j (m_j + 1) / 2 multiply-adds (square roots and divisions
         not counted)."""
-        if not hasattr(self, 'band'):
+        if not hasattr(self, 'band_off'):
             self._band_setup()
         n, b = self.band_n_host, np.minimum(self.band_bw_host, self.band_n_host - 1)
         full = np.maximum(n - b, 0) * b * (b + 1)
@@ -265,7 +265,7 @@ class PlateSweep:
         panel's band entries read and written once and the trailing window's
         lower triangle (T (T + 1) / 2 entries, T = rows below the panel in
         reach) read and written once."""
-        if not hasattr(self, 'band'):
+        if not hasattr(self, 'band_off'):
             self._band_setup()
         total = 0
         for n, b in zip(self.band_n_host.tolist(), self.band_bw_host.tolist()):
@@ -293,8 +293,10 @@ class PlateSweep:
         runs the forward substitution with the current loads (self.f),
         leaving y in self.band_work for :meth:`solve_direct`'s backward
         pass."""
-        if not hasattr(self, 'band'):
+        if not hasattr(self, 'band_off'):
             self._band_setup()
+        if not hasattr(self, 'band'):
+            self.band = torch.empty(self.band_size, dtype=torch.float64, device=self.device)
         ft, mb, _, sft = self._direct_config(config)
         s = _s(stream)
         _lib.call('pf3d_band_load', self.n_nodes, self.band_dof0.data_ptr(),
@@ -328,18 +330,30 @@ class PlateSweep:
             chol(self.n_var - nw, order[nw:].data_ptr(), sft, NARROW_PANEL, side.cuda_stream)
         main.wait_stream(side)
 
+    @property
+    def widest_band(self):
+        """Half-bandwidth (DOF) of the widest plate."""
+        return 6 * (int(np.array(self.dims).min(axis=1).max()) + 2) + 5
+
+    @property
+    def direct_method(self):
+        """What :meth:`solve_direct` runs without a config: 'dissection', or
+        'banded' on a sweep of bands up to BANDED_MAX whose launch shape
+        :meth:`autotune_direct` has chosen."""
+        tuned = self.widest_band <= BANDED_MAX and getattr(self, 'direct_config', None)
+        return 'banded' if tuned else 'dissection'
+
     def _dissection(self):
         """The sweep's nested-dissection plan and buffers, or None where the
         banded kernels are used."""
-        dims = np.array(self.dims)
-        bw = 6 * (dims.min(axis=1) + 2) + 5
-        if bw.max() <= BANDED_MAX and getattr(self, 'direct_config', None):
+        if self.direct_method == 'banded':
             return None
         if not hasattr(self, '_batch'):
-            maxb = _lib.call('pf3d_band_max_width')
-            if bw.max() > maxb:
+            maxb, bw = _lib.call('pf3d_band_max_width'), self.widest_band
+            if bw > maxb:
                 raise ValueError('plate too wide for the direct solver (bandwidth %d > %d)'
-                                 % (bw.max(), maxb))
+                                 % (bw, maxb))
+            dims = np.array(self.dims)
             from .direct import DirectBatch
             ny = np.repeat(dims[:, 1] + 1, np.diff(self.node0))
             local = np.arange(self.n_nodes) - np.repeat(self.node0[:-1], np.diff(self.node0))
@@ -370,7 +384,7 @@ class PlateSweep:
             batch.solve(self.val, self.f, self.u, s)
             self.solve(mode='fp64', rtol=rtol, max_iter=polish_iter, x0=True, stream=stream)
             return
-        if not hasattr(self, 'band'):
+        if not hasattr(self, 'band_off'):
             self._band_setup()
         cfg = self._direct_config(config)
         st = cfg[2]
@@ -388,7 +402,7 @@ class PlateSweep:
         panel class of the widest band, power-of-two buckets of the number
         of variants and of the mean DOF per variant, GPU architecture."""
         from . import autotune as AT
-        if not hasattr(self, 'band'):
+        if not hasattr(self, 'band_off'):
             self._band_setup()
         bmax = int(self.band_bw_host.max())
         panel = min(m for m in (256, 448, 576) if m >= bmax)
@@ -445,15 +459,17 @@ class PlateSweep:
         return table
 
     def autotune_direct(self, log=None, repeats=2, use_table=True):
-        """Launch configuration of the banded solver (factor threads x LDS
-        panel width, solve threads) for solve_direct / step('direct') /
-        capture('direct'): the stored choice for this sweep's key if there is
-        one (use_table), else every configuration that fits the sweep's
-        widest band timed on the current designs, the fastest kept and
-        recorded.  Returns the table of timings (stored or measured)."""
+        """Launch configuration of the banded kernels (factor threads x LDS
+        panel width, solve threads): the stored choice for this sweep's key if
+        there is one (use_table), else every configuration that fits the
+        sweep's widest band timed on the current designs, the fastest kept and
+        recorded.  Returns the table of timings (stored or measured).
+
+        On bands up to BANDED_MAX solve_direct / step('direct') /
+        capture('direct') then run the banded kernels with it.  Wider sweeps
+        are solved by nested dissection all the same: only
+        :meth:`factor_direct` takes the choice, so they need no tuning."""
         from . import autotune as AT
-        if not hasattr(self, 'band'):
-            self._band_setup()
         key = self.autotune_key()
         if use_table:
             entry = AT.lookup(key)
@@ -466,6 +482,7 @@ class PlateSweep:
                     log('autotune %s: stored choice %s' % (key, self.direct_config))
                 return [({k: v for k, v in t.items() if k != 'ms'}, t['ms'])
                         for t in entry.get('timings', [])]
+        held = hasattr(self, 'band')
         bmax = int(self.band_bw.max())
         panels = [m for m in (256, 448, 576) if m >= bmax]
 
@@ -487,6 +504,8 @@ class PlateSweep:
             table += table3
         self.direct_config = (best['ft'], best['mb'], best['st'], best['sft'])
         self.direct_config_source = 'measured'
+        if self.direct_method != 'banded' and not held:
+            del self.band  # (not kept beside the dissection's factor)
         AT.record(key, dict(best), table)
         return table
 

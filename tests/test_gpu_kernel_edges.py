@@ -424,6 +424,41 @@ def test_direct_refuses_wide_bands_and_takes_streams():
         a.solve(f, method='direct', refactor=True)
 
 
+@pytest.mark.parametrize('dims, method', [([(22, 30), (10, 12)], 'banded'),
+                                          ([(40, 41), (10, 12)], 'dissection')])
+def test_tuning_holds_no_unused_band(tmp_path, monkeypatch, dims, method):
+    """Tuning the banded kernels: used by the direct solve up to BANDED_MAX,
+    and no band storage left (or made, from the table) where dissection is
+    run all the same; one that was there before stays."""
+    from pyfe3d_amd.sweep import PlateSweep
+    monkeypatch.setenv('PF3D_AUTOTUNE_CACHE', str(tmp_path / 'tune.json'))
+
+    def sweep():
+        sw = PlateSweep(dims)
+        h, f = sw.random_designs(5)
+        sw.set_thickness(h)
+        sw.set_loads(f)
+        sw.assemble()
+        return sw
+
+    for source in ('measured', 'table'):
+        sw = sweep()
+        assert sw.direct_method == 'dissection'
+        assert sw.autotune_direct(repeats=1) and sw.direct_config_source == source
+        assert sw.direct_method == method
+        if method == 'dissection':
+            assert not hasattr(sw, 'band')
+        sw.solve_direct()
+        sw.check()
+        assert float(sw.relres.max()) <= 1e-8
+        assert hasattr(sw, '_batch') == (method == 'dissection')
+    sw = sweep()
+    sw.solve_direct(config=(512, 448, 512))
+    band = sw.band
+    sw.autotune_direct(repeats=1, use_table=False)
+    assert sw.band is band
+
+
 @pytest.mark.parametrize('rows', [1, 2, 43, 127, 128, 129, 256, 257, 1365, 1366, 2731, 21846])
 @pytest.mark.parametrize('method', ['fp64', 'ir'])
 def test_pcg_routes(rows, method):
