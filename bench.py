@@ -245,7 +245,7 @@ def sweep_rates(n_var, log, steps=2, modes=('direct', 'fp64', 'mixed')):
     captured graph: property records, KC0, BSR, Dirichlet, block Jacobi,
     FP32 copies and the solve."""
     import torch
-    from pyfe3d_amd.sweep import PlateSweep
+    from pyfe3d_amd.sweep import BANDED_MAX, PlateSweep
     t0 = time.perf_counter()
     sw = PlateSweep(sweep_dims(n_var))
     h, f = sw.random_designs(7)
@@ -255,8 +255,9 @@ def sweep_rates(n_var, log, steps=2, modes=('direct', 'fp64', 'mixed')):
         % (n_var, sw.n_elem, 6 * sw.n_nodes, sw.plan.nnzb, time.perf_counter() - t0))
     out = dict(variants=n_var, elements=sw.n_elem, dof=6 * sw.n_nodes)
     tuned = None
-    if 'direct' in modes:
-        # launch configuration of the banded solver chosen by timing
+    if 'direct' in modes and sw.widest_band <= BANDED_MAX:
+        # narrow bands: launch configuration of the banded kernels chosen by
+        # timing (wider sweeps are solved by nested dissection)
         sw.assemble()
         t0 = time.perf_counter()
         table = sw.autotune_direct(log=log, repeats=1)
@@ -299,8 +300,10 @@ def sweep_rates(n_var, log, steps=2, modes=('direct', 'fp64', 'mixed')):
                          max_relres=float(rel.max()), converged=int((rel <= 1e-8).sum()),
                          pcg_iters_total=int(its.sum()), pcg_iters_max=int(its.max()),
                          first_step_s=first)
-        if mode == 'direct' and tuned:
-            out[mode]['autotune'] = tuned
+        if mode == 'direct':
+            out[mode]['method'] = sw.direct_method
+            if tuned:
+                out[mode]['autotune'] = tuned
         if mode in pcg_tuned:
             out[mode]['autotune'] = pcg_tuned[mode]
         log('sweep %s: %.1f ms/sweep, %.1f solves/s, max relres %.2e, iters %d'
@@ -308,8 +311,44 @@ def sweep_rates(n_var, log, steps=2, modes=('direct', 'fp64', 'mixed')):
         del g
         sw.graph = None
     if 'direct' in modes:
-        out['direct']['factor'] = factor_roofline(sw, log)
+        roofline = factor_roofline if sw.direct_method == 'banded' else dissection_roofline
+        out['direct']['factor'] = roofline(sw, log)
     return out
+
+
+def dissection_roofline(sw, log, reps=3):
+    """The multifrontal factorisation of all variants (the loads' forward
+    substitution with it), timed with HIP events, against the FP64
+    matrix-core peak and against the time its factor takes to be written
+    once at 8 TB/s."""
+    import torch
+    st = torch.cuda.current_stream()
+    batch = sw._dissection()
+
+    def factor():
+        for plan, vo, fo in batch.groups:
+            plan.factor(sw.val.data_ptr() + vo, batch.factor, batch.update, batch.bad,
+                        st.cuda_stream, f=sw.f.data_ptr() + fo)
+
+    factor()
+    e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    torch.cuda.synchronize()
+    e0.record(st)
+    for _ in range(reps):
+        factor()
+    e1.record(st)
+    torch.cuda.synchronize()
+    ms = e0.elapsed_time(e1) / reps
+    flop = sum(plan.flops for plan, _, _ in batch.groups)
+    factor_bytes = 8 * sum(plan.factor_size for plan, _, _ in batch.groups)
+    tf = flop / (ms * 1e-3) / 1e12
+    log('sweep factor: %.1f ms, %.3g flop -> %.2f TFLOP/s = %.3f of FP64 peak, factor %.1f GB'
+        % (ms, flop, tf, tf / FP64_PEAK_TFLOPS, factor_bytes * 1e-9))
+    return dict(ms=ms, flop=flop, achieved=tf, peak=FP64_PEAK_TFLOPS, unit='TFLOP/s',
+                frac=tf / FP64_PEAK_TFLOPS, factor_bytes=factor_bytes,
+                min_hbm_ms=factor_bytes / HBM_PEAK_BPS * 1e3, groups=len(batch.groups),
+                fronts=sum(plan.n_fronts for plan, _, _ in batch.groups),
+                note='nested dissection: clearing, scatter, panels and updates of every tree level')
 
 
 def factor_roofline(sw, log, reps=3):
@@ -633,13 +672,13 @@ def profile_kc0(n, launches=3):
           flush=True)
 
 
-def profile_sweep(n_var, steps=3, config=(512, 448, 512, 256)):
+def profile_sweep(n_var, steps=3, config=None):
     """`steps` direct-solve steps of the n_var-plate design sweep (records,
-    KC0, BSR, Dirichlet, sparse Cholesky, triangular solves) with
-    the launch shape given (factor threads, panel bandwidth, solve threads,
-    factor threads of the plates whose band fits the 256-wide panel; default
-    the one the autotuner picks for the 4,096-plate sweep), for kernel
-    traces and counter runs."""
+    KC0, BSR, Dirichlet, sparse Cholesky, triangular solves) for kernel
+    traces and counter runs: nested dissection, or with config the banded
+    kernels with that launch shape (factor threads, panel bandwidth, solve
+    threads, factor threads of the plates whose band fits the 256-wide
+    panel)."""
     import torch
     from pyfe3d_amd.sweep import PlateSweep
     sw = PlateSweep(sweep_dims(n_var))
@@ -713,7 +752,7 @@ def main():
                     help='skip the reference CPU path (tocsc + spsolve) on smaller plates')
     ap.add_argument('--no-solve', action='store_true')
     ap.add_argument('--sweep-variants', type=int, default=4096,
-                    help='plates of the design sweep solved with the banded direct solver')
+                    help='plates of the design sweep solved with the direct solver')
     ap.add_argument('--sweep-pcg-variants', type=int, default=256,
                     help='plates of the same sweep solved with PCG (FP64 and FP32 operator)')
     ap.add_argument('--warm-start-plates', type=int, default=64)
