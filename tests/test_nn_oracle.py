@@ -99,7 +99,12 @@ def _energy_setup(seed=4, B=2, n=8):
         f = np.zeros(m.n_dof)
         f[2::6] = -rng.uniform(0.5, 1.5, m.n_nodes)
         f[fixed] = 0.
-        u = sla.spsolve(K.tocsc(), f)
+        lu, T = sla.splu(K.tocsc()), K.tocoo()
+        u = lu.solve(f)
+        for _ in range(2):  # refined with residuals in extended precision
+            r = f.astype(np.longdouble)
+            np.subtract.at(r, T.row, T.data * u.astype(np.longdouble)[T.col])
+            u = u + lu.solve(r.astype(np.float64))
         Ks.append(K); fs.append(f); ss_.append(float(u @ f)); fx.append(fixed); us.append(u)
     return Ks, fs, np.array(ss_), np.array(fx), us
 
