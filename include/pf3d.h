@@ -605,7 +605,7 @@ int pf3d_batch_solve(int64_t n_var, int64_t nb, const int64_t *row0, const int32
                      double *relres, int n_groups, int threads, void *stream);
 
 /* ------------------------------------------------------------------ */
-/* Batched banded direct solves (the design-sweep counterpart of the     */
+/* Batched direct solves (the design-sweep counterpart of the            */
 /* callers' scipy spsolve, tests/test_quad4_static_point_load.py:84-102) */
 /* ------------------------------------------------------------------ */
 

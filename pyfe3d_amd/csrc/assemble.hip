@@ -934,10 +934,10 @@ shell_kc0_sym(AsmArgs a)
 // the strains B ue, the section forces C B ue and adds B^T of them to the
 // element's forces in registers, about 1,100 FMAs per quad.  (Forming the
 // ten node-pair blocks of K_e on ten lanes that each repeat the geometry
-// was bound by FP64 issue: 484 us for 1e6 quads against 109 us, now bound
-// by the gathers of x and u and the 192 MB of forces.)  230-250 VGPRs, two
-// waves per SIMD.  The forces leave through LDS so that the wave writes its
-// 64 elements' contiguous run with consecutive lanes.
+// was bound by FP64 issue: 484 us for 1e6 quads against 99 us, now bound by
+// the gathers of x and u at two waves per SIMD (230-250 VGPRs) and the 192 MB
+// of forces, 3.3 TB/s and 22 TFLOP/s.)  The forces leave through LDS so that
+// the wave writes its 64 elements' contiguous run with consecutive lanes.
 // ------------------------------------------------------------------------
 
 // forces of one integration point: membrane/bending strains -> C -> B^T

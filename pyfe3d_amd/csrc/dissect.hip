@@ -5,9 +5,11 @@
 //
 // Against the banded factorisation (banded.hip: one workgroup walks a plate
 // 32 columns at a time, n b^2 operations in a chain of n / 32 panels) the
-// separators of a plate need 5-7 times fewer operations and leave a chain of
-// about 35 panels, and every front of a tree level, of every system, is
-// worked on at once by as many workgroups as it has row blocks and tiles.
+// separators of a plate need 2-4 times fewer operations (64 x 48 elements
+// 2.4, 64 x 64 3.6, 512 plates of 8 to 64 a side 2.0) and leave a chain of
+// 39 and 47 panels (64 x 48, 64 x 64), and every front of a tree level, of
+// every system, is worked on at once by as many workgroups as it has row
+// blocks and tiles.
 //
 // Per tree level (deepest first), all launches over all fronts of the level:
 //   * panel p: 32 own columns of each front.  A workgroup takes 128 rows
@@ -23,14 +25,15 @@
 // front (its forward substitution costs no pass of its own); the triangular
 // solves otherwise take one workgroup per front and level.
 //
-// Measured: a 64 x 48 plate (19,110 DOF) 1.04 ms to factorise and 0.28 ms for
+// Measured: a 64 x 48 plate (19,110 DOF) 1.04 ms to factorise and 0.33 ms for
 // the backward pass, against 27.0 and 7.3 ms banded; 512 plates of 8 to 64
-// elements a side (4.2e6 DOF) 17.4 + 2.1 ms against 60.8 + 6.6 ms, 119 GFLOP
-// at 6.8 TFLOP/s.  The single plate is bound by its chain of 39 panel
-// launches of 19-30 us (loads one behind another 6 us, the diagonal block's
-// pivots 6 us, the row solve 3 us, products up to 10 us); the sweep by the
-// row blocks' latency at the lower levels and by memory traffic (each panel
-// and update matrix written and read once or twice, about 4 TB/s).
+// elements a side (4.1e6 DOF) 17.2 + 2.1 ms against 60.8 + 6.6 ms, 118 GFLOP
+// at 6.9 TFLOP/s.  The single plate is bound by its chain of 39 panel
+// launches of 16-30 us (loads one behind another 6 us, the diagonal block's
+// pivots 6 us, the row solve 3 us, products up to 10 us); the sweep by memory
+// latency (waves wait in 65 % of their cycles) and by operands read again:
+// 24 GB in the panels at 2.8 TB/s, 26 GB in the updates at 4.1 TB/s for a
+// factor of 7.8 GB, the matrix cores busy in 9 % and 23 % of the cycles.
 //
 // Every sum has a fixed order: the same bits on every run.
 #include <hip/hip_runtime.h>

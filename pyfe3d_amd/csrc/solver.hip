@@ -195,9 +195,9 @@ int fused_launch(int64_t nb, const int32_t *rp, const int32_t *ci, const MT *val
                  double sa, double sb, double c1, double c2, int xmode, void *stream,
                  const char *name)
 {
-    if (nb < 0 || xmode < 0 || xmode > 3 || (xmode & 2 && !dnew) || (nb && (!r || (xin && (!rp || !ci || !val)) || (dinv && !dnew) ||
-                          (xacc && !dold) || (dold && dold == dnew) ||
-                          (xin && (xin == r || xin == dnew || xin == xacc)))))
+    if (nb < 0 || xmode < 0 || xmode > 3 || (xmode & 2 && !dnew) ||
+        (nb && (!r || (xin && (!rp || !ci || !val)) || (dinv && !dnew) || (xacc && !dold) ||
+                (dold && dold == dnew) || (xin && (xin == r || xin == dnew || xin == xacc)))))
         return pf3d_fail(PF3D_E_ARG, "%s: bad arguments", name);
     if (!nb) return PF3D_OK;
     if (nb < ONE_ROW_MAX)
@@ -1343,8 +1343,8 @@ int pf3d_bjacobi(int64_t nb, const int32_t *row_ptr, const int32_t *col_idx, con
 {
     if (nb <= 0 || !row_ptr || !col_idx || !val || !dinv || !singular)
         return pf3d_fail(PF3D_E_ARG, "pf3d_bjacobi: bad arguments");
-    hipLaunchKernelGGL(bjacobi_setup, dim3(nblk(nb, JB_ROWS)), dim3(JB_ROWS), 0, (hipStream_t)stream, nb,
-                       row_ptr, col_idx, val, dinv, dinv32, singular);
+    hipLaunchKernelGGL(bjacobi_setup, dim3(nblk(nb, JB_ROWS)), dim3(JB_ROWS), 0,
+                       (hipStream_t)stream, nb, row_ptr, col_idx, val, dinv, dinv32, singular);
     return pf3d_hip_check(hipGetLastError(), "pf3d_bjacobi");
 }
 

@@ -4,9 +4,9 @@ preconditioned by the smoothed-aggregation multigrid V-cycle.
 Replaces the reference callers' ``eigsh(A=KC0uu, M=Muu, sigma=-1.,
 which='LM')`` (tests/test_quad4_natural_freq.py:120-123) and
 ``eigsh(A=KGuu, M=KC0uu, which='SM')`` for linear buckling
-(tests/test_quad4_linear_buckling_plate_mat_coord.py:184) where a banded
+(tests/test_quad4_linear_buckling_plate_mat_coord.py:184) where a direct
 factorisation does not fit (the shift-invert Lanczos of
-:mod:`pyfe3d_amd.eigen` factorises K on one workgroup), on the
+:mod:`pyfe3d_amd.eigen` factorises K), on the
 Dirichlet-treated matrices (identity rows of K and zero rows of M or KG on
 fixed DOFs; the basis is zero there):
 

@@ -2,7 +2,7 @@
 
 ``python -m pyfe3d_amd.train_warmstart --samples 20000 --epochs 12 --eval 2000``
 draws seeded 64 x 64 plates (smooth thickness fields, Gaussian pressure
-patches, clamped edges), solves them with the batched banded Cholesky
+patches, clamped edges), solves them with the batched sparse Cholesky
 (every residual checked at 1e-8), trains the network with the library's
 forward/backward/Adam kernels on the energy-norm error of its
 Galerkin-scaled guess, evaluates zero against warm start on held-out seeds

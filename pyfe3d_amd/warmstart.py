@@ -364,7 +364,7 @@ def _dof_loads(f):
 
 def solve_plates(h, f, mode='direct', rtol=1e-8, sweep=None, x0=None, max_iter=200000):
     """Solve every plate (clamped edges) with the batched GPU solvers
-    (banded Cholesky for 'direct', block-Jacobi PCG for 'fp64' / 'mixed').
+    (sparse Cholesky for 'direct', block-Jacobi PCG for 'fp64' / 'mixed').
     Returns (u (V, n+1, n+1, 6) float64 tensor, sweep)."""
     from .sweep import PlateSweep
     V, n = h.shape[0], h.shape[1]
@@ -411,7 +411,7 @@ class EnergyData:
 
 
 def make_energy_dataset(n_samples, seed, n=64, chunk=256, log=None):
-    """Seeded plates solved by the batched banded Cholesky (every residual
+    """Seeded plates solved by the batched sparse Cholesky (every residual
     checked at 1e-8); keeps what the energy loss needs (no nodal targets):
     inputs, thicknesses, loads and u*.f, plus the channel scales."""
     X, H, F, S, U = [], [], [], [], []

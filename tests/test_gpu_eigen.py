@@ -1,5 +1,5 @@
 """Natural frequencies and linear buckling on the GPU (shift-invert Lanczos
-over the banded Cholesky factor) against scipy's eigsh on the
+over the nested-dissection factor) against scipy's eigsh on the
 oracle-assembled matrices, and against the reference tests' closed forms
 (tests/test_quad4_natural_freq.py:131-137 of pyfe3d)."""
 import numpy as np
