@@ -843,9 +843,13 @@ int pf3d_nn_gemm(int M, int N, int K, const float *A, int64_t sam, int64_t sak, 
     if (grid.y > 65535) return pf3d_fail(PF3D_E_ARG, "pf3d_nn_gemm: M too large");
     hipStream_t s = (hipStream_t)stream;
     hipLaunchKernelGGL(gemm_bf16, grid, dim3(256), 0, s, g);
-    if (z > 1)
-        hipLaunchKernelGGL(splitk_reduce<16>, dim3(nb256((int64_t)M * N * 16)), dim3(256), 0, s, g,
-                           z);
+    // 16 threads per entry, one where the entries alone fill the GPU (and 16
+    // would pass a launch's 2^32 threads)
+    const int64_t n = (int64_t)M * N;
+    if (z > 1 && n < 1 << 20)
+        hipLaunchKernelGGL(splitk_reduce<16>, dim3(nb256(n * 16)), dim3(256), 0, s, g, z);
+    else if (z > 1)
+        hipLaunchKernelGGL(splitk_reduce<1>, dim3(nb256(n)), dim3(256), 0, s, g, z);
     return pf3d_hip_check(hipGetLastError(), "pf3d_nn_gemm");
 }
 

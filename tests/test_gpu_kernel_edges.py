@@ -673,6 +673,22 @@ def test_split_products(splits):
     assert (c.cpu().numpy() == a.T @ b + 2.).all()
 
 
+@pytest.mark.parametrize('M, N', [(32, 18), (16384, 64), (16385, 64), (4194240, 65)])
+def test_split_products_of_many_entries(M, N):
+    """Products divided into two slices with few entries, at the line between
+    16 threads and one per entry, and with more than 2^28: every entry."""
+    from pyfe3d_amd import _lib
+    K = 64
+    a = torch.ones((M, K), device=DEV)
+    a *= (torch.arange(M, device=DEV) % 5).to(torch.float32)[:, None]
+    b = (torch.arange(N, device=DEV) % 3).to(torch.float32)[:, None].repeat(1, K)
+    c = torch.full((M, N), -1., device=DEV)
+    part = torch.empty(2 * M * N, device=DEV)
+    _lib.call('pf3d_nn_gemm', M, N, K, a.data_ptr(), K, 1, b.data_ptr(), K, 1, c.data_ptr(), N,
+              0, None, 0, 2, part.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(c, K * a[:, :1] * b[:, 0])
+
+
 @pytest.mark.parametrize('rows', [1, 3, 4, 5, 12287, 12288, 12301])
 def test_product_row_routes(rows):
     """One and four block rows per wave at the line between them and at the
