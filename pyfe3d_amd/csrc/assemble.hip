@@ -1831,7 +1831,8 @@ __global__ void __launch_bounds__(mixed_threads(MAT)) mixed_stream(MixedArgs m)
 {
     constexpr int T = mixed_threads(MAT);
     __shared__ __align__(16) char lds[mixed_stream_lds<MAT>()];
-    const int64_t b = blockIdx.x;
+    const int64_t b = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+    if (b >= m.blk0[4]) return;
     if (b < m.blk0[1]) shell_stream_body<QUAD4, MAT, T>(m.g[0], b, lds);
     else if (b < m.blk0[2]) shell_stream_body<QUAD4R, MAT, T>(m.g[1], b - m.blk0[1], lds);
     else if (b < m.blk0[3]) shell_stream_body<TRIA3R, MAT, T>(m.g[2], b - m.blk0[2], lds);
@@ -2002,10 +2003,14 @@ hipError_t pf3d_launch_mixed(int mat, const AsmArgs *groups, hipStream_t s)
         case 6: hipLaunchKernelGGL(mixed_kc0<6>, grid, blk, 0, s, m); break;
         default: hipLaunchKernelGGL(mixed_kc0<7>, grid, blk, 0, s, m);
         }
-    } else if (mat == KG) {
-        hipLaunchKernelGGL(mixed_stream<KG>, grid, dim3(mixed_threads(KG)), 0, s, m);
     } else {
-        hipLaunchKernelGGL(mixed_stream<MASS>, grid, dim3(mixed_threads(MASS)), 0, s, m);
+        // (rows of 2^23 blocks: a launch has fewer than 2^32 threads along x,
+        // 1.3e8 beams at the mass kernel's 256 threads per 8 of them)
+        const int64_t row = 1 << 23;
+        const dim3 rows((unsigned)(blocks < row ? blocks : row),
+                        (unsigned)((blocks + row - 1) / row));
+        if (mat == KG) hipLaunchKernelGGL(mixed_stream<KG>, rows, dim3(mixed_threads(KG)), 0, s, m);
+        else hipLaunchKernelGGL(mixed_stream<MASS>, rows, dim3(mixed_threads(MASS)), 0, s, m);
     }
     return hipGetLastError();
 }

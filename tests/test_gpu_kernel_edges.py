@@ -99,6 +99,29 @@ def test_static_system_copies_are_flat():
         assert s.val32.dim() == 1 and torch.equal(s.val32, v.reshape(-1).to(torch.float32))
 
 
+def test_mixed_mass_of_many_beams():
+    """Lumped mass of more beams (1.3e8, 39 GB of values) than one row of a
+    launch holds, all between the same two nodes: every one is written."""
+    from pyfe3d_amd import assembly as A
+    if torch.cuda.mem_get_info()[0] < 100e9:
+        pytest.skip('needs 100 GB of free memory')
+    E = (1 << 27) + 4099
+    size = A.slot_count('beamc', 'M', 1)
+    x = T([[0., 0., 0.], [0.3, 0.1, 0.2]], torch.float64)
+    conn = torch.tensor([[0, 6]], device=DEV).repeat(E, 1)
+    evec = torch.tensor([[0., 0., 1.]], dtype=torch.float64, device=DEV).repeat(E, 1)
+    props = T(np.linspace(1., 2., A.BEAM_STRIDE)[None], torch.float64)
+    v = torch.full((E, size), float('nan'), dtype=torch.float64, device=DEV)
+    A.mixed_assemble('M', [A.ElementGroup('beamc', conn, props, evec=evec)], x, None, None,
+                     v.view(-1), mtype=1, values_only=True, overwrite=True, check=False)
+    assert float(v[0].abs().max()) > 0
+    for at in range(0, E, 1 << 24):
+        part = v[at:at + (1 << 24)]
+        assert torch.equal(part, v[:1].expand(part.shape))
+    del v, conn, evec
+    torch.cuda.empty_cache()
+
+
 def test_block_sums_past_32_bits():
     """More than 2^32 pairs of entries (69 GB of block values): every block
     is written."""
