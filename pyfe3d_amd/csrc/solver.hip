@@ -451,7 +451,7 @@ __global__ void __launch_bounds__(256)
     using d2 = double __attribute__((ext_vector_type(2), aligned(8)));
     using f2 = float __attribute__((ext_vector_type(2), aligned(4)));
     const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t row = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (row >= nb) return;
     // pairs of neighbouring entries, 18 per block
     const int b0 = rp[row], n = (rp[row + 1] - b0) * 18;
@@ -1324,8 +1324,13 @@ int pf3d_bsr_system(int64_t nb, const int32_t *row_ptr, const int32_t *col_idx,
 {
     if (nb <= 0 || !row_ptr || !col_idx || !src || !fixed || !val || !val32 || src == val)
         return pf3d_fail(PF3D_E_ARG, "pf3d_bsr_system: bad arguments");
-    hipLaunchKernelGGL(bsr_system, dim3(nblk(nb, 4)), dim3(256), 0, (hipStream_t)stream,
-                       nb, row_ptr, col_idx, src, fixed, val, val32);
+    // (a launch has fewer than 2^32 threads along x: 6.7e7 rows)
+    const int64_t blocks = (nb + 3) / 4, most = 1 << 23;
+    hipLaunchKernelGGL(bsr_system,
+                       dim3((unsigned)(blocks < most ? blocks : most),
+                            (unsigned)((blocks + most - 1) / most)),
+                       dim3(256), 0, (hipStream_t)stream, nb, row_ptr, col_idx, src, fixed, val,
+                       val32);
     return pf3d_hip_check(hipGetLastError(), "pf3d_bsr_system");
 }
 

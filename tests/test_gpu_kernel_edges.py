@@ -99,6 +99,29 @@ def test_static_system_copies_are_flat():
         assert s.val32.dim() == 1 and torch.equal(s.val32, v.reshape(-1).to(torch.float32))
 
 
+def test_static_system_of_many_rows():
+    """Boundary conditions and copies of 6.7e7 block rows with one block each,
+    a wave per row: more than 2^32 threads."""
+    from pyfe3d_amd import _lib
+    if torch.cuda.mem_get_info()[0] < 100e9:
+        pytest.skip('needs 100 GB of free memory')
+    nb = (1 << 26) + 1001
+    rp = torch.arange(nb + 1, dtype=torch.int32, device=DEV)
+    src = (torch.arange(36, dtype=torch.float64, device=DEV) + 1.).repeat(nb, 1)
+    fixed = torch.zeros(6 * nb, dtype=torch.uint8, device=DEV)
+    val = torch.full_like(src, float('nan'))
+    val32 = torch.full((nb, 36), float('nan'), dtype=torch.float32, device=DEV)
+    _lib.call('pf3d_bsr_system', nb, rp.data_ptr(), rp.data_ptr(), src.data_ptr(),
+              fixed.data_ptr(), val.data_ptr(), val32.data_ptr(),
+              torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(val, src)
+    for at in range(0, nb, 1 << 24):
+        part = val32[at:at + (1 << 24)]
+        assert torch.equal(part, src[:1].to(torch.float32).expand(part.shape))
+    del src, val, val32, fixed, rp
+    torch.cuda.empty_cache()
+
+
 def test_mixed_mass_of_many_beams():
     """Lumped mass of more beams (1.3e8, 39 GB of values) than one row of a
     launch holds, all between the same two nodes: every one is written."""
