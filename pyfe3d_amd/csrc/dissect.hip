@@ -521,6 +521,15 @@ inline unsigned blocks(int64_t n, int64_t most)
     return (unsigned)std::min((n + 255) / 256, most);
 }
 
+// fn(first, count) over [first, last) in launches of at most 2^23 blocks (of
+// 256 threads: a launch has fewer than 2^32)
+template <typename F>
+void in_launches(int64_t first, int64_t last, F fn)
+{
+    for (; first < last; first += 1 << 23)
+        fn(first, dim3((unsigned)std::min(last - first, (int64_t)1 << 23)));
+}
+
 }  // namespace
 
 extern "C" {
@@ -619,13 +628,13 @@ int pf3d_nd_factor(const void *plan, const void *image, const double *val, const
     for (const Level &lv : p.levels) {
         const double *Uc = U[(depth + 1) & 1];
         for (size_t q = 0; q < lv.panels.size(); q++) {
-            const auto t = lv.panels[q];
-            hipLaunchKernelGGL(nd_panel, dim3((unsigned)(t.second - t.first)), dim3(256), 0, s, g,
-                               t.first, (int)q, L, D, Uc, bad);
+            in_launches(lv.panels[q].first, lv.panels[q].second, [&](int64_t t, dim3 n) {
+                hipLaunchKernelGGL(nd_panel, n, dim3(256), 0, s, g, t, (int)q, L, D, Uc, bad);
+            });
         }
-        if (lv.upd1 > lv.upd0)
-            hipLaunchKernelGGL(nd_update, dim3((unsigned)(lv.upd1 - lv.upd0)), dim3(256), 0, s, g,
-                               lv.upd0, L, Uc, U[depth & 1]);
+        in_launches(lv.upd0, lv.upd1, [&](int64_t t, dim3 n) {
+            hipLaunchKernelGGL(nd_update, n, dim3(256), 0, s, g, t, L, Uc, U[depth & 1]);
+        });
         depth--;
     }
     return pf3d_hip_check(hipGetLastError(), "pf3d_nd_factor");
@@ -644,11 +653,13 @@ int pf3d_nd_solve(const void *plan, const void *image, const double *factor, con
     const size_t lds = (size_t)p.widest * sizeof(double);
     if (f)
         for (const Level &lv : p.levels)
-            hipLaunchKernelGGL(nd_forward, dim3((unsigned)(lv.front1 - lv.front0)), dim3(256), lds,
-                               s, g, lv.front0, L, D, f, y, w);
+            in_launches(lv.front0, lv.front1, [&](int64_t t, dim3 n) {
+                hipLaunchKernelGGL(nd_forward, n, dim3(256), lds, s, g, t, L, D, f, y, w);
+            });
     for (size_t i = p.levels.size(); i-- > 0;)
-        hipLaunchKernelGGL(nd_backward, dim3((unsigned)(p.levels[i].front1 - p.levels[i].front0)),
-                           dim3(256), lds, s, g, p.levels[i].front0, L, D, y, x, f ? 0 : 1);
+        in_launches(p.levels[i].front0, p.levels[i].front1, [&](int64_t t, dim3 n) {
+            hipLaunchKernelGGL(nd_backward, n, dim3(256), lds, s, g, t, L, D, y, x, f ? 0 : 1);
+        });
     return pf3d_hip_check(hipGetLastError(), "pf3d_nd_solve");
 }
 
