@@ -148,6 +148,14 @@ class StaticSystem:
             self._dissection = (d, of)
         return d
 
+    def _direct_uses(self, stream):
+        """Holds back the reuse of the factor's buffers, and of the index maps
+        that every system on the pattern shares, until the launch stream is
+        past what is enqueued next (they may belong to another stream)."""
+        s = stream if stream is not None else torch.cuda.current_stream()
+        for t in (self._factor_plan.image, self._factor, self._direct_work, self._band_bad):
+            t.record_stream(s)
+
     def factor_direct(self, stream=None, b=None):
         """Cholesky factor of the system on the GPU by nested dissection
         (pyfe3d_amd.direct); b: a right-hand side whose forward substitution
@@ -161,6 +169,7 @@ class StaticSystem:
             self._direct_work = torch.empty(d.work_size, dtype=torch.float64, device=dev)
             self._band_bad = torch.zeros(1, dtype=torch.int32, device=dev)
             self._factor_plan = d
+        self._direct_uses(stream)
         with torch.cuda.stream(stream):  # (the scratch belongs to the launch stream)
             update = torch.empty(max(1, d.update_size), dtype=torch.float64, device=dev)
             d.factor(self.val.data_ptr(), self._factor, update, self._band_bad, _s(stream),
@@ -170,6 +179,7 @@ class StaticSystem:
     def direct_solve(self, b, x, stream=None):
         """x = K^-1 b with the factor of :meth:`factor_direct` (b None: the
         right-hand side given there)."""
+        self._direct_uses(stream)
         self._factor_plan.solve(self._factor, None if b is None else b.data_ptr(),
                                 x.data_ptr(), self._direct_work, _s(stream))
         return x

@@ -371,6 +371,36 @@ def test_direct_solve_on_a_changed_pattern(in_place):
     assert torch.equal(a.direct_solve(torch.as_tensor(f[0], device=DEV), x), alone[0][1])
 
 
+def test_direct_buffers_outlive_a_side_stream():
+    """The index maps that systems on one pattern share, and a factor, are not
+    handed out again while a factorisation on another stream is enqueued."""
+    from types import SimpleNamespace
+    from pyfe3d_amd.solver import StaticSystem
+    nb = _graph('30x29')
+    plan, val = _duck_plan(nb, 5, SimpleNamespace)
+    fixed, f = np.zeros(6 * len(nb)), torch.ones(6 * len(nb), dtype=torch.float64, device=DEV)
+    a, b = (StaticSystem(plan, val, fixed) for _ in range(2))
+    a.factor_direct()
+    b.factor_direct()
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(1 << 30)
+        b.factor_direct(stream=side, b=f)
+        b.direct_solve(None, f, stream=side)
+    held = [t.data_ptr() for t in (a._factor_plan.image, b._factor)]
+    del a, b, plan
+    state = {}
+    for seg in torch.cuda.memory_snapshot():
+        at = seg['address']
+        for block in seg['blocks']:
+            state.update((p, block['state']) for p in held if at <= p < at + block['size'])
+            at += block['size']
+    assert not side.query()
+    assert [state[p] for p in held] == ['active_pending_free'] * 2
+    side.synchronize()
+
+
 def test_dissection_of_separate_parts():
     """Plates that are not connected, in one system: level by level beside
     each other, each with the bits of its solution alone."""
