@@ -394,28 +394,15 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// L y = f, front by front: own part of y (permuted numbering) from f and the
-// children's boundary parts, then the front's own boundary part into w
-__global__ void __launch_bounds__(256)
-    nd_forward(Image g, int64_t front0, const double *__restrict__ L, const double *__restrict__ D,
-               const double *__restrict__ f0, double *__restrict__ y, double *__restrict__ w)
+// one front's part of L y = f in LDS: the own entries of v (k + m of them)
+// against L11, their products subtracted from the boundary entries; T is
+// scratch.  Starts and ends with a barrier.
+__device__ __forceinline__ void forward_front(const Front &f, const double *Lf,
+                                              const double *__restrict__ D, double *v,
+                                              double (*T)[NF + 1])
 {
-    extern __shared__ double v[];  // k + m entries
-    __shared__ double T[NF][NF + 1];
-    const Front f = g.fronts[front0 + blockIdx.x];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = f.k + f.m;
-    const int32_t *map = g.cmap + 2 * f.noff;
-    const double *w0 = f.c0 < 0 ? nullptr : w + g.fronts[f.c0].woff;
-    const double *w1 = f.c1 < 0 ? nullptr : w + g.fronts[f.c1].woff;
-    for (int r = tid; r < n; r += 256) {
-        const int q = r / 6, d = r - 6 * q;
-        double s = r < f.k ? f0[6 * (int64_t)g.pnode[f.own0 + q] + d] : 0.;
-        if (w0 && map[2 * q] >= 0) s += w0[6 * map[2 * q] + d];
-        if (w1 && map[2 * q + 1] >= 0) s += w1[6 * map[2 * q + 1] + d];
-        v[r] = s;
-    }
-    const double *Lf = L + f.loff;
     const int64_t ld = column(n + 1);
     for (int c0 = 0, p = 0; c0 < f.k; c0 += NF, p++) {
         const int jn = min(NF, f.k - c0);
@@ -448,7 +435,81 @@ __global__ void __launch_bounds__(256)
         __syncthreads();
     }
     if (f.k == 0) __syncthreads();
-    for (int r = tid; r < n; r += 256) {
+}
+
+// one front's part of L^T x = y: the own entries of v, its boundary entries
+// known; part is scratch, after_forward: T still holds the last panel's block.
+// Starts and ends with a barrier.
+__device__ __forceinline__ void backward_front(const Front &f, const double *Lf,
+                                               const double *__restrict__ D, double *v,
+                                               double (*T)[NF + 1], double *part,
+                                               bool after_forward)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = f.k + f.m;
+    const int64_t ld = column(n + 1);
+    __syncthreads();
+    for (int p = (f.k + NF - 1) / NF - 1; p >= 0; p--) {
+        const int c0 = p * NF, jn = min(NF, f.k - c0);
+        const double *d = D + f.doff + (int64_t)p * NF * NF;
+        const bool last = c0 + jn == f.k, below = c0 + jn < n;
+        if (!(last && after_forward))
+            for (int t = tid; t < NF * NF; t += 256) T[t >> 5][t & 31] = d[t];
+        if (below) {
+            // wave w: columns 8 w .. 8 w + 7 of the panel against the rows below
+            double s[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) s[j] = 0.;
+            for (int r = c0 + jn + lane; r < n; r += 64) {
+                const double vr = v[r];
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    s[j] = fma(Lf[(int64_t)min(c0 + 8 * wave + j, f.k - 1) * ld + r], vr, s[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) s[j] += __shfl_xor(s[j], o, 64);
+                if (lane == 0) part[8 * wave + j] = s[j];
+            }
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const int rr = lane & 31;
+            double rhs = lane < jn ? v[c0 + lane] - (below ? part[rr] : 0.) : 0.;
+            for (int c = jn - 1; c >= 0; c--) {
+                if (lane == c) rhs *= T[c][c];
+                const double xv = readlane_d(rhs, c);
+                if (lane < c) rhs -= T[c][rr] * xv;
+            }
+            if (lane < jn) v[c0 + lane] = rhs;
+        }
+        __syncthreads();
+    }
+}
+
+// L y = f, front by front: own part of y (permuted numbering) from f and the
+// children's boundary parts, then the front's own boundary part into w
+__global__ void __launch_bounds__(256)
+    nd_forward(Image g, int64_t front0, const double *__restrict__ L, const double *__restrict__ D,
+               const double *__restrict__ f0, double *__restrict__ y, double *__restrict__ w)
+{
+    extern __shared__ double v[];  // k + m entries
+    __shared__ double T[NF][NF + 1];
+    const Front f = g.fronts[front0 + blockIdx.x];
+    const int n = f.k + f.m;
+    const int32_t *map = g.cmap + 2 * f.noff;
+    const double *w0 = f.c0 < 0 ? nullptr : w + g.fronts[f.c0].woff;
+    const double *w1 = f.c1 < 0 ? nullptr : w + g.fronts[f.c1].woff;
+    for (int r = threadIdx.x; r < n; r += 256) {
+        const int q = r / 6, d = r - 6 * q;
+        double s = r < f.k ? f0[6 * (int64_t)g.pnode[f.own0 + q] + d] : 0.;
+        if (w0 && map[2 * q] >= 0) s += w0[6 * map[2 * q] + d];
+        if (w1 && map[2 * q + 1] >= 0) s += w1[6 * map[2 * q + 1] + d];
+        v[r] = s;
+    }
+    forward_front(f, L + f.loff, D, v, T);
+    for (int r = threadIdx.x; r < n; r += 256) {
         if (r < f.k) y[6 * (int64_t)f.own0 + r] = v[r];
         else w[f.woff + r - f.k] = v[r];
     }
@@ -466,54 +527,40 @@ __global__ void __launch_bounds__(256)
     __shared__ double T[NF][NF + 1];
     __shared__ double part[NF];
     const Front f = g.fronts[front0 + blockIdx.x];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = f.k + f.m;
     const int32_t *nodes = g.nodes + f.noff;
     const double *Lf = L + f.loff;
     const int64_t ld = column(n + 1);
-    for (int r = tid; r < n; r += 256) {
+    for (int r = threadIdx.x; r < n; r += 256) {
         const int q = r / 6;
         v[r] = fused && r < f.k ? Lf[r * ld + n] : y[6 * (int64_t)nodes[q] + r - 6 * q];
     }
-    __syncthreads();
-    for (int p = (f.k + NF - 1) / NF - 1; p >= 0; p--) {
-        const int c0 = p * NF, jn = min(NF, f.k - c0);
-        const double *d = D + f.doff + (int64_t)p * NF * NF;
-        for (int t = tid; t < NF * NF; t += 256) T[t >> 5][t & 31] = d[t];
-        // wave w: columns 8 w .. 8 w + 7 of the panel against the rows below
-        double s[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) s[j] = 0.;
-        for (int r = c0 + jn + lane; r < n; r += 64) {
-            const double vr = v[r];
-#pragma unroll
-            for (int j = 0; j < 8; j++)
-                s[j] = fma(Lf[(int64_t)min(c0 + 8 * wave + j, f.k - 1) * ld + r], vr, s[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) s[j] += __shfl_xor(s[j], o, 64);
-            if (lane == 0) part[8 * wave + j] = s[j];
-        }
-        __syncthreads();
-        if (wave == 0) {
-            const int rr = lane & 31;
-            double rhs = lane < jn ? v[c0 + lane] - part[rr] : 0.;
-            for (int c = jn - 1; c >= 0; c--) {
-                if (lane == c) rhs *= T[c][c];
-                const double xv = readlane_d(rhs, c);
-                if (lane < c) rhs -= T[c][rr] * xv;
-            }
-            if (lane < jn) v[c0 + lane] = rhs;
-        }
-        __syncthreads();
-    }
-    for (int r = tid; r < f.k; r += 256) {
+    backward_front(f, Lf, D, v, T, part, false);
+    for (int r = threadIdx.x; r < f.k; r += 256) {
         const int q = r / 6, d = r - 6 * q;
         y[6 * (int64_t)f.own0 + r] = v[r];
         x[6 * (int64_t)g.pnode[f.own0 + q] + d] = v[r];
     }
+}
+
+// both passes of fronts without parents or children (a plan of one level):
+// one launch, the same bits.  Plates of up to 3 x 3 elements are one front:
+// 2 x 2, solved again with its factor, 133 us a call (131 by the banded
+// kernel) against 139 in two launches.
+__global__ void __launch_bounds__(256)
+    nd_solve_alone(Image g, int64_t front0, const double *__restrict__ L,
+                   const double *__restrict__ D, const double *__restrict__ f0,
+                   double *__restrict__ x)
+{
+    extern __shared__ double v[];
+    __shared__ double T[NF][NF + 1];
+    __shared__ double part[NF];
+    const Front f = g.fronts[front0 + blockIdx.x];
+    const int32_t *pnode = g.pnode + f.own0;
+    for (int r = threadIdx.x; r < f.k; r += 256) v[r] = f0[6 * (int64_t)pnode[r / 6] + r % 6];
+    forward_front(f, L + f.loff, D, v, T);
+    backward_front(f, L + f.loff, D, v, T, part, true);
+    for (int r = threadIdx.x; r < f.k; r += 256) x[6 * (int64_t)pnode[r / 6] + r % 6] = v[r];
 }
 
 inline unsigned blocks(int64_t n, int64_t most)
@@ -651,6 +698,12 @@ int pf3d_nd_solve(const void *plan, const void *image, const double *factor, con
     const double *L = factor, *D = factor + p.l_size;
     double *y = work, *w = work + 6 * p.n_nodes;
     const size_t lds = (size_t)p.widest * sizeof(double);
+    if (f && p.levels.size() == 1) {
+        in_launches(p.levels[0].front0, p.levels[0].front1, [&](int64_t t, dim3 n) {
+            hipLaunchKernelGGL(nd_solve_alone, n, dim3(256), lds, s, g, t, L, D, f, x);
+        });
+        return pf3d_hip_check(hipGetLastError(), "pf3d_nd_solve");
+    }
     if (f)
         for (const Level &lv : p.levels)
             in_launches(lv.front0, lv.front1, [&](int64_t t, dim3 n) {

@@ -54,6 +54,7 @@ class DirectPlan:
         image = np.empty(sizes[0], dtype=np.uint8)
         _lib.call('pf3d_nd_image', self._plan, image.ctypes.data)
         self.image = torch.as_tensor(image, device=self.device)
+        self.stream = torch.cuda.current_stream(self.device).cuda_stream  # (the image's)
 
     def __del__(self):
         plan, self._plan = getattr(self, '_plan', None), None

@@ -149,12 +149,15 @@ class StaticSystem:
         return d
 
     def _direct_uses(self, stream):
-        """Holds back the reuse of the factor's buffers, and of the index maps
-        that every system on the pattern shares, until the launch stream is
-        past what is enqueued next (they may belong to another stream)."""
+        """The handle of the launch stream.  Where the factor's buffers, or the
+        index maps that every system on the pattern shares, belong to another
+        stream, their reuse waits for what is enqueued next on this one."""
         s = stream if stream is not None else torch.cuda.current_stream()
-        for t in (self._factor_plan.image, self._factor, self._direct_work, self._band_bad):
-            t.record_stream(s)
+        h = s.cuda_stream
+        if self._factor_plan.stream != h or self._factor_of != (self._factor.data_ptr(), h):
+            for t in (self._factor_plan.image, self._factor, self._direct_work, self._band_bad):
+                t.record_stream(s)
+        return h
 
     def factor_direct(self, stream=None, b=None):
         """Cholesky factor of the system on the GPU by nested dissection
@@ -168,20 +171,20 @@ class StaticSystem:
             self._factor = torch.empty(d.factor_size, dtype=torch.float64, device=dev)
             self._direct_work = torch.empty(d.work_size, dtype=torch.float64, device=dev)
             self._band_bad = torch.zeros(1, dtype=torch.int32, device=dev)
+            self._factor_of = (self._factor.data_ptr(), torch.cuda.current_stream(dev).cuda_stream)
             self._factor_plan = d
-        self._direct_uses(stream)
+        h = self._direct_uses(stream)
         with torch.cuda.stream(stream):  # (the scratch belongs to the launch stream)
             update = torch.empty(max(1, d.update_size), dtype=torch.float64, device=dev)
-            d.factor(self.val.data_ptr(), self._factor, update, self._band_bad, _s(stream),
-                     f=None if b is None else b.data_ptr())
+        d.factor(self.val.data_ptr(), self._factor, update, self._band_bad, h,
+                 f=None if b is None else b.data_ptr())
         self._factored = True
 
     def direct_solve(self, b, x, stream=None):
         """x = K^-1 b with the factor of :meth:`factor_direct` (b None: the
         right-hand side given there)."""
-        self._direct_uses(stream)
         self._factor_plan.solve(self._factor, None if b is None else b.data_ptr(),
-                                x.data_ptr(), self._direct_work, _s(stream))
+                                x.data_ptr(), self._direct_work, self._direct_uses(stream))
         return x
 
     def setup_amg(self, xyz, log=None, precisions=('fp64',), graph=True, **kw):
