@@ -1126,7 +1126,9 @@ int pcg_mixed_run(const Mat &A64, const Mat &A32, const double *b, double *x, do
                        (const double *)nullptr, partial);
     hipLaunchKernelGGL(finish, dim3(1), dim3(VB), 0, s, (int)nd, partial, st, 3);
     if (!x0) hipLaunchKernelGGL(fill0<double>, dim3(nv), dim3(VB), 0, s, n, x);
-    hipLaunchKernelGGL(fill0<double>, dim3(nv), dim3(VB), 0, s, n, p);
+    // (p and q: the first residual goes through the update with alpha = 0,
+    // and 0 times what the workspace held may be NaN)
+    hipLaunchKernelGGL(fill0<double>, dim3(nblk(2 * n, VB)), dim3(VB), 0, s, 2 * n, p);
     // r = b - K64 x ; z = M r ; (r.z, r.r) ; keep p (zero at the start)
     auto true_residual = [&]() -> hipError_t {
         hipError_t e2 = spmv<double, double>(A64, x, y, s);

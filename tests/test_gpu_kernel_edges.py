@@ -595,6 +595,30 @@ def test_pcg_without_a_step(rows, method):
         assert info['iters'] == 25
 
 
+@pytest.mark.parametrize('rows', [40, 2000, 21846])
+@pytest.mark.parametrize('method', ['fp64', 'mixed', 'ir'])
+def test_pcg_ignores_its_workspace(rows, method):
+    """The bits of a solve do not depend on what the workspace held."""
+    from types import SimpleNamespace
+    from pyfe3d_amd.solver import StaticSystem
+    chain = [{j for j in (i - 1, i, i + 1) if 0 <= j < 40} for i in range(40)]
+    rp, ci, val, _ = _block_system(chain, 9)
+    k = -(-rows // 40)
+    plan = SimpleNamespace(
+        row_ptr=T(np.concatenate([[0]] + [rp[1:] + s * ci.size for s in range(k)]), torch.int32),
+        col_idx=T(np.concatenate([ci + 40 * s for s in range(k)]), torch.int32), n_nodes=40 * k)
+    s = StaticSystem(plan, T(np.tile(val.reshape(-1), k), torch.float64), np.zeros(240 * k))
+    rng = np.random.default_rng(rows)
+    f, x0 = rng.normal(size=240 * k), T(rng.normal(size=240 * k), torch.float64)
+    got = []
+    for byte in (0, 255):  # (255: every double a NaN)
+        s._w64.fill_(byte)
+        s._wir.fill_(byte)
+        got.append([s.solve(f, method=method, rtol=1e-6, x0=x) for x in (None, x0)])
+    for (u, a), (v, b) in zip(*got):
+        assert a == b and a['converged'] and torch.equal(u, v)
+
+
 def _bf16(a):
     return torch.as_tensor(a, dtype=torch.float32).to(torch.bfloat16).to(torch.float64)
 
