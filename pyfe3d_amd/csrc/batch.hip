@@ -242,7 +242,8 @@ __global__ void __launch_bounds__(BT) batch_solve(BatchArgs a)
             if (m.slot >= 0)
                 for (int64_t row = r0 + m.slot; row < r1; row += RPG) {
                     const int64_t t = row * 6 + m.comp;
-                    a.p[t] = a.z[t] + beta * a.p[t];
+                    // (0 times what the workspace held may be NaN)
+                    a.p[t] = beta == 0. ? a.z[t] : a.z[t] + beta * a.p[t];
                 }
         };
         double rz = 0., dummy = 0.;

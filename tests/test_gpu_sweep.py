@@ -166,6 +166,21 @@ def test_sweep_rtol_1e8_and_warm_start():
         assert (sw.iters.cpu().numpy() == 0).all(), mode
 
 
+@pytest.mark.parametrize('mode', ['fp64', 'mixed'])
+def test_sweep_ignores_its_workspace(mode):
+    """The bits of a batched solve do not depend on what the workspace held."""
+    sw, h, f = _sweep(seed=6)
+    got = []
+    for byte in (0, 255):  # (255: every double a NaN)
+        sw.work.fill_(byte)
+        sw.assemble()
+        sw.solve(mode=mode, rtol=1e-8)
+        torch.cuda.synchronize()
+        assert (sw.relres.cpu().numpy() <= 1e-8).all()
+        got.append(sw.u.clone())
+    assert torch.equal(*got)
+
+
 def test_sweep_graph_replays_match_eager():
     """The captured step (records, KC0, BSR, Dirichlet, Jacobi, FP32 copies,
     batched solve) replayed for new designs gives the eager results bit
