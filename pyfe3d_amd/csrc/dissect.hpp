@@ -19,6 +19,9 @@ constexpr int NF = 32;    // panel width (DOFs)
 constexpr int RB = 128;   // rows below the diagonal block per workgroup
 constexpr int TS = 64;    // update tile
 constexpr double MAX_SIDE = 0.7;  // largest share of a part on one side of a cut
+// cost of a cut above which the numbering is halved as well: about the nodes in
+// the widest half-bandwidth that the direct solvers take (576 DOF)
+constexpr double NARROW = 96.;
 
 // column length of a panel (n rows and the right-hand side's) and of an
 // update matrix: whole 128-byte lines
@@ -152,16 +155,21 @@ class Dissection {
         return b;
     }
 
-    // cost of the separator q[c.first .. c.second): its size, raised where
-    // one side is much the larger, above that of every other cut where it
-    // holds more than MAX_SIDE of the vertices: a tree of slivers is as deep
+    // cost of a separator of s vertices that leaves at most `side` of n on one
+    // side: its size, raised where that is much the larger, above that of every
+    // other cut where it is more than MAX_SIDE: a tree of slivers is as deep
     // as the part is long (1,000 levels for a comb of 1,000 teeth)
+    static double cut_cost(size_t n, size_t s, size_t side)
+    {
+        const double big = (double)side / (double)n;
+        return (double)s * (1. + 8. * std::max(0., big - 0.55)) + (big > MAX_SIDE ? (double)n : 0.);
+    }
+
+    // the same of the level q[c.first .. c.second), none if it is empty
     static double cut_cost(size_t n, std::pair<size_t, size_t> c)
     {
-        if (c.second <= c.first) return 1e300;
-        const double big = (double)std::max(c.first, n - c.second) / (double)n;
-        return (double)(c.second - c.first) * (1. + 8. * std::max(0., big - 0.55)) +
-               (big > MAX_SIDE ? (double)n : 0.);
+        return c.second <= c.first ? 1e300
+                                   : cut_cost(n, c.second - c.first, std::max(c.first, n - c.second));
     }
 
     // the cheapest inner level of q (in level order): its [begin, end), or
@@ -326,10 +334,40 @@ class Dissection {
                 bc = c;
             }
         }
+        if (best > NARROW && by_index(V, best, S, A, B)) return true;
         if (best >= 1e300) return false;
         A.assign(bq.begin(), bq.begin() + bc.first);
         S.assign(bq.begin() + bc.first, bq.begin() + bc.second);
         B.assign(bq.begin() + bc.second, bq.end());
+        return true;
+    }
+
+    // the given numbering halved, where that costs less: its separator is no
+    // larger than the half-bandwidth, which a level can exceed many times
+    // (branches that end at the same distance)
+    bool by_index(const std::vector<int32_t> &V, double best, std::vector<int32_t> &S,
+                  std::vector<int32_t> &A, std::vector<int32_t> &B)
+    {
+        const size_t n = V.size();
+        std::vector<int32_t> order(V);
+        std::nth_element(order.begin(), order.begin() + n / 2, order.end());
+        const int32_t mid = order[n / 2];
+        const int right = ++stamp_;
+        for (int32_t v : V)
+            if (v >= mid) in(v) = right;
+        std::vector<int32_t> sep, left;
+        for (int32_t v : V) {
+            if (v >= mid) continue;
+            bool touches = false;
+            for (int p = rp_[v]; p < rp_[v + 1] && !touches; p++) touches = in(ci_[p]) == right;
+            (touches ? sep : left).push_back(v);
+        }
+        if (left.empty() || cut_cost(n, sep.size(), std::max(left.size(), n - n / 2)) >= best)
+            return false;
+        for (int32_t v : V)
+            if (v >= mid) B.push_back(v);
+        S = std::move(sep);
+        A = std::move(left);
         return true;
     }
 };

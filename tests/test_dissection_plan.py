@@ -178,6 +178,35 @@ def test_tree_of_a_comb_is_flat(spine, tooth):
     assert Plan(*_pattern(n, edges)).levels <= np.log(n / 16) / np.log(1 / 0.7) + 2
 
 
+def _bush(teeth, twigs, length):
+    """Branches of a spine that end at the same distance from its start, each
+    in a bush."""
+    e, n, spine = [], 0, []
+    for i in range(teeth):
+        tooth = list(range(n, n + teeth - i))
+        n += teeth - i
+        spine.append(tooth[0])
+        e += _chain(tooth)
+        for _ in range(twigs):
+            twig = list(range(n, n + length))
+            n += length
+            e += _chain([tooth[-1]] + twig)
+    return n, e + _chain(spine)
+
+
+@pytest.mark.parametrize('teeth, twigs, length', [(20, 20, 3), (30, 30, 2), (32, 31, 2),
+                                                  (45, 40, 2)])
+def test_wide_levels_are_not_separators(teeth, twigs, length):
+    """Levels of up to 1,800 nodes in patterns with a narrow band: no front
+    much wider than the band."""
+    n, edges = _bush(teeth, twigs, length)
+    rp, ci = _pattern(n, edges)
+    band = np.abs(np.repeat(np.arange(n), np.diff(rp)) - ci).max()
+    plan = Plan(rp, ci)
+    # a separator and what it touches of the ones around
+    assert (plan.fronts['k'] + plan.fronts['m']).max() <= 3 * 6 * band
+
+
 @pytest.mark.parametrize('keep', ['lower', 'upper', 'random'])
 @pytest.mark.parametrize('name', sorted(GRAPHS))
 def test_one_sided_blocks(name, keep):
